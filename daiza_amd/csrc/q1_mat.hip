@@ -2,6 +2,7 @@
 // C ABI (Q1_0Matrix::{from_gguf, row_into_slice, matvec_into_slice, matvec_add_into_slice,
 // matvec_multi_into_slice}, Daiza-engine/src/model/weights.rs:83-972).
 #include "runtime.h"
+#include "q1_digits.h"
 #include "q1_gemm.h"
 
 #include <cstdarg>
@@ -260,35 +261,66 @@ int upload_q1_host(const uint8_t* aos, int64_t rows, int64_t cols, Q1Dev* out, s
 // ------------------------------------------------------------------ N-column products
 
 int packed_x_reserve(Scratch& buf, int n, int64_t K, PackedX* out) {
-  const int Np = (n + kGemmTok - 1) / kGemmTok * kGemmTok;
-  const int64_t Kp = (K + kTileCols - 1) / kTileCols * kTileCols;
-  const size_t part_bytes = (size_t)Np * Kp * 2;
-  const int rc = buf.reserve(kGemmParts * part_bytes + (size_t)Np * 4);
+  const int Np = (n + kWideTok - 1) / kWideTok * kWideTok;
+  const int nt = (int)((K + kTileCols - 1) / kTileCols);
+  const size_t blocks = (size_t)(Np / 16) * nt;
+  const size_t dig = blocks * 2 * kHalfBytes, ex = blocks * 256, ssq = (size_t)nt * Np * 4;
+  const int rc = buf.reserve(dig + ex + ssq);
   if (rc) return rc;
-  char* b = static_cast<char*>(buf.ptr);
-  out->xh = reinterpret_cast<uint16_t*>(b);
-  out->xm = reinterpret_cast<uint16_t*>(b + part_bytes);
-  out->xl = reinterpret_cast<uint16_t*>(b + 2 * part_bytes);
-  out->sig = reinterpret_cast<float*>(b + kGemmParts * part_bytes);
-  out->Kp = Kp;
+  uint8_t* b = static_cast<uint8_t*>(buf.ptr);
+  out->dig = b;
+  out->ex = reinterpret_cast<uint32_t*>(b + dig);
+  out->ssq = reinterpret_cast<float*>(b + dig + ex);
+  out->K = K;
+  out->ntiles = nt;
   out->Np = Np;
   return DZ_OK;
 }
 
-hipError_t launch_x_pack(const float* x, int64_t ldx, int64_t K, int n, const float* w, float eps, const PackedX& p,
+hipError_t launch_x_pack(const float* x, int64_t ldx, int64_t K, int n, const float* w, float eps, PackedX& p,
                          hipStream_t s) {
-  hipLaunchKernelGGL(x_pack_kernel, dim3((unsigned)p.Np), dim3(256), 0, s, x, ldx, K, n, w, eps, p.xh, p.xm, p.xl,
-                     p.sig, p.Kp);
+  p.normed = w != nullptr;
+  p.eps = eps;
+  hipLaunchKernelGGL(digit_pack_kernel, dim3((unsigned)(p.Np / 16), (unsigned)p.ntiles), dim3(256), 0, s, x, ldx, K, n, w,
+                     p.dig, p.ex, p.ssq, p.Np);
   return hipGetLastError();
+}
+
+// CUs of the current device (0 if the query fails).
+static int device_cus() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cus[dev] == 0 && hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus[dev] = 0;
+  return cus[dev];
+}
+
+// Splits of the wide product's K tiles: the workgroups go to the CUs in whole workgroups, and one tile of one
+// workgroup takes about kWideTileUs of a CU's matrix cores; a split adds a pass over its partials (written
+// and read back at about 4 TB/s) and a launch.
+constexpr double kWideTileUs = 3.6;
+static int wide_splits(const Q1Dev& W, int n, int* tps) {
+  const int64_t wgs = ((W.nrb + kWideRb - 1) / kWideRb) * ((n + kWideTok - 1) / kWideTok);
+  const int nt = (int)W.ntiles, cus = std::max(1, device_cus());
+  int best = 1;
+  double bc = 1e30;
+  for (int S = 1; S <= std::min(nt, 32); ++S) {
+    const int t = (nt + S - 1) / S;
+    if ((nt + t - 1) / t != S) continue;
+    double c = (double)((wgs * S + cus - 1) / cus) * t * kWideTileUs;
+    if (S > 1) c += 4.0 + (double)S * n * W.rows * 8 / 4e6;
+    if (c < bc) bc = c, best = S;
+  }
+  *tps = (nt + best - 1) / best;
+  return best;
 }
 
 // Workgroups wanted in flight (two per CU): a product with fewer splits its K tiles over
 // blockIdx.z and sums the partials in a second pass.
 constexpr int kGemmMinWgs = 512;
 
-int gemm_splits(const Q1Dev& W, int n, int* tps) {
-  const int nb = n <= 16 ? 1 : kGemmNB;
-  const int64_t wgs = ((W.nrb + 3) / 4) * ((n + 16 * nb - 1) / (16 * nb));
+static int gemm_splits(const Q1Dev& W, int* tps) {
+  const int64_t wgs = (W.nrb + 3) / 4;
   const int nt = (int)W.ntiles;
   int S = 1;
   if (wgs < kGemmMinWgs && nt > 1) S = (int)std::min<int64_t>(nt, (kGemmMinWgs + wgs - 1) / wgs);
@@ -296,117 +328,90 @@ int gemm_splits(const Q1Dev& W, int n, int* tps) {
   return (nt + *tps - 1) / *tps;
 }
 
-// The wide form takes eight row-blocks per workgroup (each wave a whole row-block: half the
-// activation reads per weight byte and per matrix instruction) when that costs at most a quarter
-// more in whole rounds of workgroups over the CUs (one workgroup per CU either way) than four
-// row-blocks do: measured at the prefill shapes, the eight-block form runs 10-16% faster at equal
-// round cost and about 4% slower at a third more.
-static bool gemm_wide_rb8(const Q1Dev& W, int n, int S) {
-  if (S > 1) return false;
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-  if (cus[dev] == 0 && (hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-                        cus[dev] <= 0)) {
-    cus[dev] = 0;
-    return false;
-  }
-  const int64_t tb = (n + kGemmTok - 1) / kGemmTok, c = cus[dev];
-  const int64_t r4 = (((W.nrb + 3) / 4) * tb + c - 1) / c, r8 = (((W.nrb + 7) / 8) * tb + c - 1) / c;
-  return 8 * r8 <= 5 * r4;
-}
-
-// One product launch: the packed form (p non-null) or the raw form (x f32, row stride ldx).
-static hipError_t launch_q1_gemm_any(const Q1Dev& W, const PackedX* p, const float* xr, int64_t ldx, int n, float* y,
-                                     int64_t ldy, int accumulate, hipStream_t s, Scratch* split,
-                                     GemmDefer* defer = nullptr, const float* norm_w = nullptr, float eps = 0.f) {
+hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int64_t ldy, int accumulate,
+                          hipStream_t s, Scratch* split, GemmDefer* defer) {
   static bool attr = false;
   if (!attr) {
-    const void* ks[5] = {reinterpret_cast<const void*>(q1_gemm_kernel<kGemmNB, false>),
-                         reinterpret_cast<const void*>(q1_gemm_kernel<kGemmNB, false, false, 8>),
-                         reinterpret_cast<const void*>(q1_gemm_kernel<1, false>),
-                         reinterpret_cast<const void*>(q1_gemm_kernel<1, true>),
-                         reinterpret_cast<const void*>(q1_gemm_kernel<1, true, true>)};
-    const size_t sh[5] = {gemm_shmem(kGemmNB), gemm_shmem(kGemmNB), gemm_shmem(1), gemm_shmem(1), gemm_shmem(1, true)};
-    for (int i = 0; i < 5; ++i) {
-      hipError_t e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh[i]);
-      if (e != hipSuccess) return e;
-    }
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_wide_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWideShmem);
+    if (e != hipSuccess) return e;
     attr = true;
   }
-  const bool raw = p == nullptr;
-  if (!raw && (W.ntiles * kTileCols != p->Kp || n > p->Np)) return hipErrorInvalidValue;
-  if (raw && n > 16) return hipErrorInvalidValue;  // the raw form packs one 16-token block per workgroup
-  GemmX gx{};
-  if (raw) {
-    gx.Kp = W.ntiles * kTileCols;
-    gx.xf = xr;
-    gx.ldx = ldx;
-    gx.K = W.cols;
-    gx.nw = norm_w;
-    gx.eps = eps;
-  } else {
-    gx.xh = p->xh;
-    gx.xm = p->xm;
-    gx.xl = p->xl;
-    gx.sig = p->sig;
-    gx.Kp = p->Kp;
-  }
+  if (W.ntiles != p.ntiles || W.cols != p.K || n > p.Np) return hipErrorInvalidValue;
   int tps;
-  int S = gemm_splits(W, n, &tps);
+  int S = wide_splits(W, n, &tps);
   if (S > 1 && !split) S = 1, tps = (int)W.ntiles;
   float* out = y;
   int64_t ld = ldy, zs = 0;
   if (S > 1) {
     zs = (int64_t)n * W.rows;
-    // the partials, then (normed raw form) the per-split sums of squares [S][n]
-    if (split->reserve(((size_t)S * zs + (norm_w ? (size_t)S * n : 0)) * sizeof(float))) return hipErrorOutOfMemory;
+    if (split->reserve((size_t)S * zs * sizeof(float))) return hipErrorOutOfMemory;
     out = static_cast<float*>(split->ptr);
     ld = W.rows;
-    if (raw && norm_w) {
-      gx.ssq = out + (size_t)S * zs;
-      gx.ssq_ld = n;
-    }
   }
-  const unsigned gx_ = (unsigned)((W.nrb + 3) / 4);
-  const dim3 g1(gx_, 1, (unsigned)S), g2(gx_, (unsigned)((n + kGemmTok - 1) / kGemmTok), (unsigned)S);
-  if (n <= 16) {
-    if (raw && n <= 8)  // hi and mid of every token in one operand, lo in a second: two matrix instructions per step
-      hipLaunchKernelGGL((q1_gemm_kernel<1, true, true>), g1, dim3(64 * gemm_waves(1)), gemm_shmem(1, true), s, W.data, W.rows,
-                         W.nrb, (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-    else if (raw)
-      hipLaunchKernelGGL((q1_gemm_kernel<1, true>), g1, dim3(64 * gemm_waves(1)), gemm_shmem(1), s, W.data, W.rows, W.nrb,
-                         (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-    else
-      hipLaunchKernelGGL((q1_gemm_kernel<1, false>), g1, dim3(64 * gemm_waves(1)), gemm_shmem(1), s, W.data, W.rows, W.nrb,
-                         (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-  } else if (gemm_wide_rb8(W, n, S)) {
-    const dim3 g8((unsigned)((W.nrb + 7) / 8), g2.y, 1);
-    hipLaunchKernelGGL((q1_gemm_kernel<kGemmNB, false, false, 8>), g8, dim3(64 * gemm_waves(kGemmNB)), gemm_shmem(kGemmNB), s,
-                       W.data, W.rows, W.nrb, (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-  } else {
-    hipLaunchKernelGGL((q1_gemm_kernel<kGemmNB, false>), g2, dim3(64 * gemm_waves(kGemmNB)), gemm_shmem(kGemmNB), s, W.data, W.rows,
-                       W.nrb, (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-  }
+  const WideGrid g{(int)((W.nrb + kWideRb - 1) / kWideRb), (n + kWideTok - 1) / kWideTok, tps};
+  const DigitX dx{p.dig, p.ex, p.normed ? p.ssq : nullptr, p.Np, p.K, p.eps};
+  hipLaunchKernelGGL(q1_wide_kernel, dim3((unsigned)(g.nrg * g.ntg * S)), dim3(256), kWideShmem, s, W.data, W.rows, W.nrb,
+                     (int)W.ntiles, g, dx, n, out, ld, zs, S > 1 ? 0 : accumulate);
   hipError_t e = hipGetLastError();
-  const float* ssq = S > 1 && raw && norm_w ? gx.ssq : nullptr;
-  if (defer) *defer = GemmDefer{out, S, zs, ssq, n, W.cols, eps};
+  if (defer) *defer = GemmDefer{out, S, zs, nullptr, 0, W.cols, 0.f};
   if (e != hipSuccess || S == 1 || defer) return e;
   hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((W.rows + 255) / 256), (unsigned)n), dim3(256), 0, s,
-                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, ssq, n, W.cols, eps);
+                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, (const float*)nullptr, 0, W.cols, 0.f);
   return hipGetLastError();
-}
-
-hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int64_t ldy, int accumulate,
-                          hipStream_t s, Scratch* split, GemmDefer* defer) {
-  return launch_q1_gemm_any(W, &p, nullptr, 0, n, y, ldy, accumulate, s, split, defer);
 }
 
 hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n, float* y, int64_t ldy,
                               int accumulate, hipStream_t s, Scratch* split, const float* norm_w, float eps,
                               GemmDefer* defer) {
   if ((W.cols & 3) || (ldx & 3)) return hipErrorInvalidValue;  // 16-byte loads of x rows
-  return launch_q1_gemm_any(W, nullptr, x, ldx, n, y, ldy, accumulate, s, split, defer, norm_w, eps);
+  if (n > 16) return hipErrorInvalidValue;  // one 16-token block per workgroup
+  static bool attr = false;
+  if (!attr) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_gemm_kernel<false>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_shmem(false));
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_gemm_kernel<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_shmem(true));
+    if (e != hipSuccess) return e;
+    attr = true;
+  }
+  GemmX gx{};
+  gx.xf = x;
+  gx.ldx = ldx;
+  gx.K = W.cols;
+  gx.nw = norm_w;
+  gx.eps = eps;
+  int tps;
+  int S = gemm_splits(W, &tps);
+  if (S > 1 && !split) S = 1, tps = (int)W.ntiles;
+  float* out = y;
+  int64_t ld = ldy, zs = 0;
+  if (S > 1) {
+    zs = (int64_t)n * W.rows;
+    // the partials, then (normed) the per-split sums of squares [S][n]
+    if (split->reserve(((size_t)S * zs + (norm_w ? (size_t)S * n : 0)) * sizeof(float))) return hipErrorOutOfMemory;
+    out = static_cast<float*>(split->ptr);
+    ld = W.rows;
+    if (norm_w) {
+      gx.ssq = out + (size_t)S * zs;
+      gx.ssq_ld = n;
+    }
+  }
+  const dim3 g((unsigned)((W.nrb + 3) / 4), 1, (unsigned)S);
+  if (n <= 8)  // hi and mid of every token in one operand, lo in a second: two matrix instructions per step
+    hipLaunchKernelGGL(q1_gemm_kernel<true>, g, dim3(64 * kGemmWaves), gemm_shmem(true), s, W.data, W.rows, W.nrb,
+                       (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
+  else
+    hipLaunchKernelGGL(q1_gemm_kernel<false>, g, dim3(64 * kGemmWaves), gemm_shmem(false), s, W.data, W.rows, W.nrb,
+                       (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
+  hipError_t e = hipGetLastError();
+  const float* ssq = S > 1 && norm_w ? gx.ssq : nullptr;
+  if (defer) *defer = GemmDefer{out, S, zs, ssq, n, W.cols, eps};
+  if (e != hipSuccess || S == 1 || defer) return e;
+  hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((W.rows + 255) / 256), (unsigned)n), dim3(256), 0, s,
+                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, ssq, n, W.cols, eps);
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ matrix API state

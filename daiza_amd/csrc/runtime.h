@@ -62,17 +62,20 @@ hipError_t launch_partial_reduce(const float* part, int64_t ld, int n_tg, const 
 // N-column products on the matrix cores (q1_gemm.h): activations packed once per input, then
 // one launch per matrix.
 struct PackedX {
-  uint16_t* xh = nullptr;
-  uint16_t* xm = nullptr;
-  uint16_t* xl = nullptr;
-  float* sig = nullptr;
-  int64_t Kp = 0;  // padded columns
-  int Np = 0;      // padded tokens (multiple of kGemmTok)
+  uint8_t* dig = nullptr;   // digit operands (q1_digits.h)
+  uint32_t* ex = nullptr;   // block scales
+  float* ssq = nullptr;     // sums of squares per tile and token
+  bool normed = false;      // packed with an RMSNorm weight: 1/rms is applied to the product
+  float eps = 0.f;
+  int64_t K = 0;
+  int ntiles = 0;
+  int Np = 0;               // padded tokens (multiple of kWideTok)
 };
 // Carves a PackedX for n tokens of K columns out of `buf` (grown on demand).
 int packed_x_reserve(Scratch& buf, int n, int64_t K, PackedX* out);
-// x[n][K] (row stride ldx) -> p; RMS-normalised with weight w first when w is non-null.
-hipError_t launch_x_pack(const float* x, int64_t ldx, int64_t K, int n, const float* w, float eps, const PackedX& p,
+// x[n][K] (row stride ldx) -> p; RMS-normalised with weight w when w is non-null (p is then of x ⊙ w
+// with the sums of squares beside it).
+hipError_t launch_x_pack(const float* x, int64_t ldx, int64_t K, int n, const float* w, float eps, PackedX& p,
                          hipStream_t s);
 // y[n][rows] (row stride ldy) =|+= p · Wᵀ; W.cols must match the packed K.  A product with too
 // few workgroups to fill the device splits its K tiles into partials held in `split` (grown on

@@ -1,0 +1,76 @@
+"""The many-token Q1_0 product (more than 16 columns) at the edges of its tiles: 512-row and 32-token
+workgroup tiles, 16-row and 16-token operand blocks, half and whole K tiles, split and unsplit K.
+
+Bound: with u = 2^-24, a group of 128 columns takes six f32 additions and one fma into the row's sum, and
+the activations' digits keep 2^-29 of their 32-column block's largest value, so a row's error is at most
+(ngroups + 8) u Σ|w x| + 2^-29 Σ|w| max|x|, which the comparison below uses as it stands (the accumulate
+form and the split sums add one rounding each).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(rng, rows, cols):
+    blk = np.empty((rows, cols // 128, 18), np.uint8)
+    blk[:, :, 2:] = rng.integers(0, 256, (rows, cols // 128, 16), dtype=np.uint8)
+    sc = (np.abs(rng.standard_normal((rows, cols // 128))) * 0.02).astype(np.float16)
+    blk[:, :, :2] = sc[..., None].view(np.uint8)
+    sign = np.unpackbits(blk[:, :, 2:], axis=-1, bitorder="little").astype(np.float64) * 2 - 1
+    return blk.reshape(-1), (sign * sc[..., None].astype(np.float64)).reshape(rows, cols)
+
+
+def _check(y, w, x, extra=0.0):
+    ref = x.astype(np.float64) @ w.T
+    u = 2.0 ** -24
+    mass = np.abs(x.astype(np.float64)) @ np.abs(w).T
+    bound = (w.shape[1] // 128 + 8 + 8) * u * mass + 2.0 ** -29 * np.abs(x).max(1)[:, None] * np.abs(w).sum(1)[None]
+    err = np.abs(y - ref)
+    assert np.all(err <= bound + extra), float((err / (bound + extra)).max())
+
+
+@pytest.mark.parametrize("rows,cols,n", [
+    (1, 128, 17),          # one row, one group of the first half tile
+    (16, 256, 32),         # one operand block, a whole half tile
+    (511, 384, 33),        # a row short of a tile, three groups, one token into the second token group
+    (513, 640, 31),        # one row into the second row group, one group into the second tile
+    (1088, 1152, 48),      # three row groups, half a token group
+    (8 * 64 * 9 + 5, 512, 64),  # more than one band of row groups
+    (5120, 17408, 40),     # few workgroups: K is split
+])
+def test_tile_edges(dz, rows, cols, n):
+    rng = np.random.default_rng(rows + cols + n)
+    aos, w = _matrix(rng, rows, cols)
+    m = dz.Q1_0Matrix(aos, rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    _check(m.matvec_batch(x), w, x)
+    y0 = rng.standard_normal((n, rows)).astype(np.float32)
+    y = y0.copy()
+    m.matvec_add_batch_into_slice(x, n, y)
+    _check(y - y0.astype(np.float64), w, x, extra=2.0 ** -23 * (np.abs(y0) + np.abs(y)))
+
+
+def test_block_ranges_and_non_finite(dz):
+    """Blocks of 32 columns of very different size, tiny and huge values; a token with an infinity or a
+    NaN gives NaN in its own results and leaves the others as they are."""
+    rows, cols, n = 200, 1024, 20
+    rng = np.random.default_rng(3)
+    aos, w = _matrix(rng, rows, cols)
+    m = dz.Q1_0Matrix(aos, rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[0, 32:64] *= np.float32(2.0 ** 30)
+    x[1, ::32] *= np.float32(2.0 ** -20)
+    x[2] *= np.float32(2.0 ** -90)
+    x[3] *= np.float32(2.0 ** 100)
+    x[4] = 0
+    x[5, 64:] = 0
+    y = m.matvec_batch(x)
+    _check(y, w, x)
+    assert np.all(y[4] == 0)
+    bad = x.copy()
+    bad[7, 500], bad[9, 0] = np.inf, np.nan
+    yb = m.matvec_batch(bad)
+    assert np.all(np.isnan(yb[7])) and np.all(np.isnan(yb[9]))
+    keep = [i for i in range(n) if i not in (7, 9)]
+    assert np.array_equal(yb[keep], y[keep])
