@@ -325,173 +325,13 @@ __global__ __launch_bounds__(256) void bt_attn_prep_kernel(const float* __restri
   }
 }
 
-// Causal GQA attention of tokens t0 .. t0+TPW-1 (positions pos0 + t) over cache positions
-// [0, pos0 + t] for the GRP q-heads of kv-head kvh (online softmax, attention.rs:149-199), then
-// o·sigmoid(gate) (attention.rs:202-203) -> ao[t][h·256 ..].  The TPW tokens of a workgroup share
-// every cache row it reads (R = TPW·GRP query rows).  The 4 waves take blocks of 64 positions in turn
-// with their own running (m, l, o) per row and are merged at the end.  Grid (ceil(n/TPW), nkv, nch),
-// 256 threads: with nch > 1 workgroup z takes positions [z·csz, (z+1)·csz) and writes its record
-// (m, l, o[256]) per (token, q-head) to rec[t][h][z] for bt_attn_merge_kernel instead.
-template <int GRP, int TPW>
-__global__ __launch_bounds__(256) void bt_attn_kernel(const float* __restrict__ qb, const float* __restrict__ gate,
-                                                      const float* __restrict__ kcache,
-                                                      const float* __restrict__ vcache, int max_ctx, int nq,
-                                                      int pos0, int n, float* __restrict__ ao, int csz,
-                                                      float* __restrict__ rec, int n_xcd, int nkv_x, int nch_x) {
-  constexpr int HD = 256, BP = 64, R = TPW * GRP;
-  // the query rows and block probabilities during the walk; the waves' (o) for the final merge after
-  // it, in the same memory
-  constexpr int kWalk = (R * HD + 4 * R * BP) * 4, kMerge = 4 * R * HD * 4;
-  __shared__ __align__(16) unsigned char buf[kWalk > kMerge ? kWalk : kMerge];
-  __shared__ float wm[4][R], wl[4][R];
-  float(*qs)[HD] = reinterpret_cast<float(*)[HD]>(buf);
-  float(*ps)[R][BP] = reinterpret_cast<float(*)[R][BP]>(buf + R * HD * 4);
-  float(*wo)[R][HD] = reinterpret_cast<float(*)[R][HD]>(buf);
-  int tg, kvh, z, nch;
-  if (n_xcd > 0) {
-    // 1-D grid: workgroup L runs on XCD L % 8 (round-robin dispatch); the token groups of one
-    // (kv-head, chunk) pair get indices with the same residue, so the chunk's cache rows are fetched
-    // into one XCD's L2 and read there once per group, instead of once per XCD
-    const int L = (int)blockIdx.x, u = L >> 3, pair = (u / n_xcd) * 8 + (L & 7);
-    if (pair >= nkv_x * nch_x) return;
-    tg = u % n_xcd;
-    kvh = pair % nkv_x;
-    z = pair / nkv_x;
-    nch = nch_x;
-  } else {
-    tg = (int)blockIdx.x;
-    kvh = (int)blockIdx.y;
-    z = (int)blockIdx.z;
-    nch = (int)gridDim.z;
-  }
-  const int t0 = tg * TPW, nt = min(TPW, n - t0);
-  const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const int pbeg = nch > 1 ? z * csz : 0;
-  const int pend = nch > 1 ? (z + 1) * csz : 0x7FFFFFFF;
-  int ctxt[TPW];  // positions visible to each token within this chunk: [pbeg, ctxt)
-#pragma unroll
-  for (int tt = 0; tt < TPW; ++tt) ctxt[tt] = tt < nt ? min(pos0 + t0 + tt + 1, pend) : pbeg;
-  const int ctx = ctxt[nt - 1];  // the group's last token sees the most
-  for (int i = (int)tid; i < R * HD; i += 256) {
-    const int r = i / HD, tt = r / GRP, gi = r % GRP;
-    qs[r][i % HD] = tt < nt ? qb[((size_t)(t0 + tt) * nq + kvh * GRP + gi) * HD + i % HD] : 0.f;
-  }
-  __syncthreads();
-  const float* kb = kcache + (size_t)kvh * max_ctx * HD;
-  const float* vb = vcache + (size_t)kvh * max_ctx * HD;
-  float m[R], l[R];
-  float4 o[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    m[r] = -INFINITY;
-    l[r] = 0.f;
-    o[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  // Blocks of 64 positions, wave w taking blocks w, w+4, ...  Scores: lane = position, each lane
-  // walks its key row against the query rows in LDS (a broadcast read), so a score costs 256 FMAs in
-  // one lane instead of a 64-lane reduction per (position, row).  (Four lanes per position, each
-  // reading a quarter of the row so that a load touches 16 rows instead of 64, measured slower here:
-  // 119 against 83 us per layer at context 8192.)  Values: lane = 4 dims, walking the block's
-  // positions with their probabilities from LDS.
-  for (int b0 = pbeg + (int)wave * BP; b0 < ctx; b0 += 4 * BP) {
-    const int pp = b0 + (int)lane;
-    const float* kr = kb + (size_t)(pp < ctx ? pp : b0) * HD;
-    float sc[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) sc[r] = 0.f;
-#pragma unroll 4
-    for (int j = 0; j < HD / 4; ++j) {
-      const float4 k4 = *reinterpret_cast<const float4*>(kr + 4 * j);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float4 q4 = *reinterpret_cast<const float4*>(&qs[r][4 * j]);
-        float d = sc[r];
-        d = __builtin_fmaf(q4.x, k4.x, d);
-        d = __builtin_fmaf(q4.y, k4.y, d);
-        d = __builtin_fmaf(q4.z, k4.z, d);
-        sc[r] = __builtin_fmaf(q4.w, k4.w, d);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const bool valid = pp < ctxt[r / GRP];
-      const float x = valid ? sc[r] : -INFINITY;
-      const float mn = fmaxf(m[r], wave_max(x));
-      // a row with no visible position yet keeps m = -inf: its factors are 0 and 1 by definition
-      const float al = mn == -INFINITY ? 1.0f : expf(m[r] - mn);
-      const float pr = valid ? expf(x - mn) : 0.f;
-      l[r] = l[r] * al + wave_sum(pr);
-      o[r].x *= al;
-      o[r].y *= al;
-      o[r].z *= al;
-      o[r].w *= al;
-      m[r] = mn;
-      ps[wave][r][lane] = pr;
-    }
-    // the other lanes' probabilities of this wave (LDS accesses of one wave complete in order)
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();
-    const int np = min(BP, ctx - b0);
-#pragma unroll 4
-    for (int pi = 0; pi < np; ++pi) {
-      const float4 v4 = *reinterpret_cast<const float4*>(vb + (size_t)(b0 + pi) * HD + 4 * lane);
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float pr = ps[wave][r][pi];
-        o[r].x = __builtin_fmaf(pr, v4.x, o[r].x);
-        o[r].y = __builtin_fmaf(pr, v4.y, o[r].y);
-        o[r].z = __builtin_fmaf(pr, v4.z, o[r].z);
-        o[r].w = __builtin_fmaf(pr, v4.w, o[r].w);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_wave_barrier();  // this block's reads of ps before the next block's writes
-  }
-  __syncthreads();  // every wave is done with qs and ps: the merge buffer reuses them
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (lane == 0) {
-      wm[wave][r] = m[r];
-      wl[wave][r] = l[r];
-    }
-    *reinterpret_cast<float4*>(&wo[wave][r][4 * lane]) = o[r];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int tt = r / GRP, gi = r % GRP;
-    if (tt >= nt) continue;
-    const int t = t0 + tt;
-    float M = -INFINITY;
-    for (int w = 0; w < 4; ++w)
-      if (wl[w][r] > 0.f) M = fmaxf(M, wm[w][r]);
-    float L = 0.f, O = 0.f;
-    for (int w = 0; w < 4; ++w) {
-      const float e = wl[w][r] > 0.f ? expf(wm[w][r] - M) : 0.f;
-      L = __builtin_fmaf(wl[w][r], e, L);
-      O = __builtin_fmaf(wo[w][r][tid], e, O);
-    }
-    const int h = kvh * GRP + gi;
-    if (nch > 1) {
-      float* rr = rec + (((size_t)t * nq + h) * nch + z) * (2 + HD);
-      if (tid == 0) {
-        rr[0] = M;
-        rr[1] = L;
-      }
-      rr[2 + tid] = O;
-    } else {
-      const float gt = gate[((size_t)t * nq + h) * HD + tid];
-      ao[((size_t)t * nq + h) * HD + tid] = (O * (1.0f / L)) * sigmoidf_(gt);
-    }
-  }
-}
-
-// Causal GQA attention of few tokens on the matrix cores, f32 operands (v_mfma_f32_16x16x4_f32: the
+// Causal GQA attention of a chunk's tokens on the matrix cores, f32 operands (v_mfma_f32_16x16x4_f32: the
 // products and sums are f32, in another order than the reference's loop, attention.rs:149-203).
-// The n·GRP (token, q-head) rows of kv-head kvh, row ρ = t·GRP + g, are one matrix: wave w holds
-// rows 16w .. 16w+15 (n·GRP <= 64), so each cache row is read by one workgroup for every token.
-// Workgroup (z, kvh) takes positions [z·csz, (z+1)·csz) in blocks of 16 and writes the record
-// (m, l, o[256]) of each row to rec[t][h][z] for bt_attn_merge_kernel.  Per block:
+// The n·GRP (token, q-head) rows of kv-head kvh, row ρ = t·GRP + g, are one matrix; a workgroup takes 64
+// of them (wave w rows 16w .. 16w+15), so each cache row it reads serves about 64/GRP tokens.
+// Workgroup (row tile, kvh, z) takes the positions [z·csz, (z+1)·csz) that its rows see, in blocks of 16,
+// and writes the record (m, l, o[256]) of each row to rec[t][h][z] for bt_attn_merge_kernel, or with one
+// chunk (nch == 1) the gated output itself.  Per block:
 //   S^T = K_blk · Q^T: A = K rows (lane = position p0 + (lane & 15), dims 16j + 4(lane >> 4) + c
 //   in step 4j + c), B = the same dims of the wave's Q rows (registers); the result leaves lane
 //   (r, k) the scores of row 16w + r at positions p0 + 4k + i, so the online softmax of a row runs
@@ -499,19 +339,33 @@ __global__ __launch_bounds__(256) void bt_attn_kernel(const float* __restrict__ 
 //   O += P · V_blk in position order 4k + s (step s): no transpose through LDS.
 //   B of step s, tile (th, c): V[p0 + 4k + s][64th + 4r + c]; O tile (th, c) leaves lane (r, k)
 //   rows 16w + 4k + i at dim 64th + 4r + c.
-// Grid (nch, nkv), 256 threads, no LDS.
-template <int GRP>
+// Bound by the f32 matrix instructions (128 of 32 cycles per wave and block) once a workgroup walks many
+// blocks.  Against the vector kernel that prefill used (one lane per position, a token per workgroup),
+// whose cache rows were read once per token: 1024 tokens into an empty context 414 -> 194 us per layer,
+// 333 tokens behind 7000 1821 -> 679 (and 27 for the merge).
+// 1-D grid row tiles x (kv-head, chunk) pairs, 256 threads, no LDS: workgroup L runs on XCD L % 8
+// (round-robin dispatch), so where the pairs are a multiple (or a divisor) of eight a pair's row tiles meet
+// in one L2 (or a few); the last row tiles, which see the most positions, come first.
+// AHEAD: the next block's scores are formed while this block's softmax runs (one wave per SIMD: nothing else
+// would fill the matrix cores then), at the price of one block's scores for nothing per chunk; without
+// it a chunk's last block is the only one.  The launch takes it for chunks of at least 32 blocks: at 112
+// blocks 679 against 710 us, at nine 39.5 against 37.4.
+template <int GRP, bool AHEAD>
 __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restrict__ qb, const float* __restrict__ kcache,
                                                            const float* __restrict__ vcache, int max_ctx, int nq,
-                                                           int pos0, int n, int csz, int nch, float* __restrict__ rec) {
+                                                           int pos0, int n, int csz, int nch, int nkv, float* __restrict__ rec,
+                                                           const float* __restrict__ gate, float* __restrict__ ao) {
   constexpr int HD = 256;
-  const int z = (int)blockIdx.x, kvh = (int)blockIdx.y;
+  const int ntile = (n * GRP + 63) / 64;
+  const int pairs = nkv * nch, pair = (int)blockIdx.x % pairs;
+  const int tile = ntile - 1 - (int)blockIdx.x / pairs, kvh = pair % nkv, z = pair / nkv;
   const unsigned tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
   const int ln = (int)(lane & 15u), lk = (int)(lane >> 4);
   const int rows = n * GRP;
-  const int pbeg = z * csz, pend = min((z + 1) * csz, pos0 + n);  // the chunk's positions seen by anyone
-  // the softmax row of this lane: ρ = 16w + ln, visible positions [pbeg, ctx_r)
-  const int rho = 16 * (int)w + ln;
+  // the chunk's positions seen by any row of the tile
+  const int pbeg = z * csz, pend = min((z + 1) * csz, pos0 + (min(64 * tile + 64, rows) - 1) / GRP + 1);
+  // the softmax row of this lane, visible positions [pbeg, ctx_r)
+  const int rho = 64 * tile + 16 * (int)w + ln;
   const bool rv = rho < rows;
   const int ctx_r = rv ? min(pos0 + rho / GRP + 1, pend) : pbeg;
   float4 q[16];  // Q[ρ][16j + 4lk .. +3]
@@ -526,8 +380,8 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
   float m = -INFINITY, l = 0.f;
   const float* kb = kcache + (size_t)kvh * max_ctx * HD;
   const float* vb = vcache + (size_t)kvh * max_ctx * HD;
-  // A block's key and value rows are requested one block ahead (keys while the previous block's
-  // values are multiplied, values while its scores are formed), so that no matrix instruction waits
+  // A block's key and value rows are requested ahead (keys while the values of the block before the
+  // previous one are multiplied, values while its scores are formed), so that no matrix instruction waits
   // for a load issued just before it.  Positions past the chunk are clamped to its last one
   // (written, finite) and masked.
   float4 kk[16], vv[16];  // kk[j]: K[p][16j + 4lk ..]; vv[4s + th]: V[p0 + 4lk + s][64th + 4ln ..]
@@ -544,13 +398,11 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
       for (int th = 0; th < 4; ++th) vv[4 * s + th] = *reinterpret_cast<const float4*>(vr + 64 * th);
     }
   };
-  if (pbeg < pend) {
-    load_k(pbeg);
-    load_v(pbeg);
-  }
-  for (int p0 = pbeg; p0 < pend; p0 += 16) {
-    const int pn = p0 + 16 < pend ? p0 + 16 : p0;  // the next block (the last one reloads itself)
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+  // scores of the block whose keys are in kk
+  f32x4 s0, s1;
+  auto scores = [&]() {
+    s0 = f32x4{0.f, 0.f, 0.f, 0.f};
+    s1 = s0;
 #pragma unroll
     for (int j = 0; j < 16; j += 2) {
       s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j].x, q[j].x, s0, 0, 0, 0);
@@ -562,11 +414,29 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
       s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j].w, q[j].w, s0, 0, 0, 0);
       s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j + 1].w, q[j + 1].w, s1, 0, 0, 0);
     }
-    load_k(pn);
+  };
+  if (pbeg < pend) {
+    load_k(pbeg);
+    load_v(pbeg);
+    if constexpr (AHEAD) {
+      scores();
+      load_k(min(pbeg + 16, pend - 1));
+    }
+  }
+  for (int p0 = pbeg; p0 < pend; p0 += 16) {
+    f32x4 cur;
+    if constexpr (AHEAD) {
+      cur = s0 + s1;
+      scores();  // of the next block (of nothing at the last one)
+    } else {
+      scores();
+      load_k(min(p0 + 16, pend - 1));
+      cur = s0 + s1;
+    }
     float sc[4], bm = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      sc[i] = p0 + 4 * lk + i < ctx_r ? s0[i] + s1[i] : -INFINITY;
+      sc[i] = p0 + 4 * lk + i < ctx_r ? cur[i] : -INFINITY;
       bm = fmaxf(bm, sc[i]);
     }
     bm = fmaxf(bm, __shfl_xor(bm, 16));
@@ -584,6 +454,14 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
     ps += __shfl_xor(ps, 32);
     l = l * al + ps;
     m = mn;
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) {  // the softmax among the next block's matrix instructions
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x006, 6, 0);
+      }
+      load_k(min(p0 + 32, pend - 1));
+    }
     // the O rows of this lane are 16w + 4lk + i: their factors live in lanes 4lk + i (skipped when
     // no row of the wave has a new maximum: every factor is then exactly 1)
     if (__builtin_amdgcn_ballot_w64(al != 1.0f)) {
@@ -604,9 +482,27 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
         o[4 * th + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], v4.z, o[4 * th + 2], 0, 0, 0);
         o[4 * th + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[s], v4.w, o[4 * th + 3], 0, 0, 0);
       }
-    load_v(pn);
+    load_v(min(p0 + 16, pend - 1));
   }
-  // records: (m, l) of row ρ from lanes lk = 0; o rows 16w + 4lk + i, dims 64th + 4ln .. +3
+  const int ro0 = 64 * tile + 16 * (int)w + 4 * lk;  // the lane's first o row
+  if (nch == 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float inv = 1.0f / __shfl(l, 4 * lk + i);
+      const int ro = ro0 + i;
+      if (ro >= rows) continue;
+      const size_t off = ((size_t)(ro / GRP) * nq + kvh * GRP + ro % GRP) * HD + 4 * ln;
+#pragma unroll
+      for (int th = 0; th < 4; ++th) {
+        const float4 gt = *reinterpret_cast<const float4*>(gate + off + 64 * th);
+        *reinterpret_cast<float4*>(ao + off + 64 * th) =
+            make_float4((o[4 * th][i] * inv) * sigmoidf_(gt.x), (o[4 * th + 1][i] * inv) * sigmoidf_(gt.y),
+                        (o[4 * th + 2][i] * inv) * sigmoidf_(gt.z), (o[4 * th + 3][i] * inv) * sigmoidf_(gt.w));
+      }
+    }
+    return;
+  }
+  // records: (m, l) of row ρ from lanes lk = 0; o rows ro0 + i, dims 64th + 4ln .. +3
   if (lk == 0 && rv) {
     float* rr = rec + (((size_t)(rho / GRP) * nq + kvh * GRP + rho % GRP) * nch + z) * (2 + HD);
     rr[0] = m;
@@ -614,16 +510,18 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int ro = 16 * (int)w + 4 * lk + i;
+    const int ro = ro0 + i;
     if (ro >= rows) continue;
     float* rr = rec + (((size_t)(ro / GRP) * nq + kvh * GRP + ro % GRP) * nch + z) * (2 + HD) + 2 + 4 * ln;
 #pragma unroll
-    for (int th = 0; th < 4; ++th)
-      *reinterpret_cast<float4*>(rr + 64 * th) = make_float4(o[4 * th][i], o[4 * th + 1][i], o[4 * th + 2][i], o[4 * th + 3][i]);
+    for (int th = 0; th < 4; ++th)  // rr is 8-byte aligned
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        *reinterpret_cast<float2*>(rr + 64 * th + 2 * c) = make_float2(o[4 * th + 2 * c][i], o[4 * th + 2 * c + 1][i]);
   }
 }
 
-// Merge of the position chunks of bt_attn_kernel (records with l = 0 held no position), then
+// Merge of the position chunks of bt_attn_mfma_kernel (records with l = 0 held no position), then
 // o·sigmoid(gate).  Grid (n, nq), 256 threads (one output dim each); nch <= 256.  Thread z < nch
 // brings chunk z's (m, l) to LDS, so that every chunk's weight exp(m_z - M) is formed once, and the
 // dims are summed over the chunks in order, the first 64 requested with the statistics and the

@@ -1328,42 +1328,18 @@ static hipError_t launch(K kfn, dim3 g, dim3 b, hipStream_t s, Args... args) {
   return hipGetLastError();
 }
 
-// Grid (token groups, nkv, nch); with at least 8 (kv-head, chunk) pairs, a 1-D grid that keeps each
-// pair's token groups on one XCD (bt_attn_kernel).  A few tokens (speculative verify) go two to a
-// workgroup, so that each cache row is read half as often; a long prefill keeps one token per
-// workgroup (more workgroups, fewer registers each).
-static hipError_t launch_bt_attn(int grp, int n, int nkv, int nch, hipStream_t s, const float* qb, const float* gate,
-                                 const float* kc, const float* vc, int max_ctx, int nq, int pos0, float* ao, int csz,
-                                 float* rec) {
-  const int tpw = n <= 16 ? 2 : 1;
-  const int ng = (n + tpw - 1) / tpw;
-  const int pairs = nkv * nch;
-  const bool xcd = nch > 1 && pairs >= 8;
-  const dim3 g = xcd ? dim3((unsigned)(8 * ((pairs + 7) / 8) * ng)) : dim3((unsigned)ng, (unsigned)nkv, (unsigned)nch);
-  const int nx = xcd ? ng : 0;
-#define DZ_ATTN(G_, T_) \
-  launch(bt_attn_kernel<G_, T_>, g, dim3(256), s, qb, gate, kc, vc, max_ctx, nq, pos0, n, ao, csz, rec, nx, nkv, nch)
-#define DZ_ATTN_G(G_) return tpw == 2 ? DZ_ATTN(G_, 2) : DZ_ATTN(G_, 1)
-  switch (grp) {
-    case 1: DZ_ATTN_G(1);
-    case 2: DZ_ATTN_G(2);
-    case 3: DZ_ATTN_G(3);
-    case 4: DZ_ATTN_G(4);
-    case 6: DZ_ATTN_G(6);
-    case 8: DZ_ATTN_G(8);
-    default: return hipErrorInvalidValue;
-  }
-#undef DZ_ATTN_G
-#undef DZ_ATTN
-}
-
-// The few-token attention on the matrix cores (every token of a kv-head in one workgroup), grid
-// (nch, nkv), with about one workgroup per CU (one wave per SIMD: the kernel holds its block's
-// keys and values a block ahead in registers).
+// The chunk's attention on the matrix cores: row tiles of 64 (token, q-head) rows x kv-heads x position
+// chunks, about one workgroup per CU at a time (one wave per SIMD: the kernel holds its block's keys and
+// values a block ahead in registers).
 static hipError_t launch_bt_attn_mfma(int grp, int nkv, int nch, hipStream_t s, const float* qb, const float* kc,
-                                      const float* vc, int max_ctx, int nq, int pos0, int n, int csz, float* rec) {
-  const dim3 g((unsigned)nch, (unsigned)nkv);
-#define DZ_ATTN_M(G_) return launch(bt_attn_mfma_kernel<G_>, g, dim3(256), s, qb, kc, vc, max_ctx, nq, pos0, n, csz, nch, rec)
+                                      const float* vc, int max_ctx, int nq, int pos0, int n, int csz, float* rec,
+                                      const float* gate, float* ao) {
+  const int ntile = (n * grp + 63) / 64;
+  const dim3 g((unsigned)(nkv * nch * ntile));
+  const bool ahead = csz >= 32 * 16;
+#define DZ_ATTN_MA(G_, A_) \
+  launch(bt_attn_mfma_kernel<G_, A_>, g, dim3(256), s, qb, kc, vc, max_ctx, nq, pos0, n, csz, nch, nkv, rec, gate, ao)
+#define DZ_ATTN_M(G_) return ahead ? DZ_ATTN_MA(G_, true) : DZ_ATTN_MA(G_, false)
   switch (grp) {
     case 1: DZ_ATTN_M(1);
     case 2: DZ_ATTN_M(2);
@@ -1374,23 +1350,18 @@ static hipError_t launch_bt_attn_mfma(int grp, int nkv, int nch, hipStream_t s, 
     default: return hipErrorInvalidValue;
   }
 #undef DZ_ATTN_M
+#undef DZ_ATTN_MA
 }
 
-static int bt_attn_mfma_chunks(int nkv, int ctx_max, int* csz) {
-  int nch = std::max(1, std::min(256, (256 + nkv - 1) / nkv));
-  *csz = ((ctx_max + nch - 1) / nch + 15) / 16 * 16;  // whole blocks of 16 positions
-  return (ctx_max + *csz - 1) / *csz;
-}
-
-// Position chunks of the chunk's attention: enough workgroups to fill the device when the chunk
-// has few tokens (speculative verify at long context), one chunk for a long prefill.
-// A chunk of several positions is a whole number of 256-position rounds (the kernel's 4 waves take
-// 64 each) where that keeps about the wanted number of chunks.
-static int bt_attn_chunks(int n, int nkv, int ctx_max, int* csz) {
-  int nch = (1024 + n * nkv - 1) / (n * nkv);
-  nch = std::max(1, std::min({nch, std::max(1, ctx_max / 64), 256}));  // the merge takes up to 256
-  *csz = (ctx_max + nch - 1) / nch;
-  if (nch > 1 && *csz > 256) *csz = (*csz + 128) / 256 * 256;
+// Position chunks of the chunk's attention: whole blocks of 16 positions, enough of them that the row
+// tiles of all kv-heads make about kAttnWgs workgroups (one round of the CUs for few tokens, where
+// every workgroup is as long; two where later row tiles see more than earlier ones), at most 256 (the
+// merge's bound).  A chunk's records cost a pass of their own, so a prefill whose row tiles fill the
+// device keeps one chunk, which needs none.
+static int bt_attn_mfma_chunks(int n, int grp, int nkv, int ctx_max, int* csz) {
+  const int wgs = (n * grp + 63) / 64 * nkv, want = n * grp <= 64 ? 256 : 512;
+  const int nch = wgs >= 256 ? 1 : std::max(1, std::min(256, (want + wgs - 1) / wgs));
+  *csz = ((ctx_max + nch - 1) / nch + 15) / 16 * 16;
   return (ctx_max + *csz - 1) / *csz;
 }
 
@@ -1473,25 +1444,17 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
                           (const float*)x->bt.yin, ld_in, (int)c.n_head, (int)c.n_head_kv, (const float*)l.q_norm,
                           (const float*)l.k_norm, c.rms_eps, (const float*)x->rope, (int)c.rope_dim, p0, x->bt.qb,
                           x->bt.gate, kc, vc, (int)c.max_ctx));
-      // few tokens (verify): all of a kv-head's query rows in one matrix-core workgroup, chunk records
-      // always merged; otherwise token groups per workgroup
       const int grp = (int)(c.n_head / c.n_head_kv);
-      const bool mf = n * grp <= 64;
       int csz;
-      const int nch = mf ? bt_attn_mfma_chunks((int)c.n_head_kv, p0 + n, &csz)
-                         : bt_attn_chunks(n, (int)c.n_head_kv, p0 + n, &csz);
+      const int nch = bt_attn_mfma_chunks(n, grp, (int)c.n_head_kv, p0 + n, &csz);
       float* rec = nullptr;
-      if (nch > 1 || mf) {
+      if (nch > 1) {
         if ((rc = x->bt.arec.reserve((size_t)n * c.n_head * nch * (2 + c.head_dim) * sizeof(float)))) return rc;
         rec = static_cast<float*>(x->bt.arec.ptr);
       }
-      if (mf)
-        DZ_HIP_CHECK(launch_bt_attn_mfma(grp, (int)c.n_head_kv, nch, s, x->bt.qb, kc, vc, (int)c.max_ctx, (int)c.n_head,
-                                         p0, n, csz, rec));
-      else
-        DZ_HIP_CHECK(launch_bt_attn(grp, n, (int)c.n_head_kv, nch, s, x->bt.qb, x->bt.gate, kc, vc, (int)c.max_ctx,
-                                    (int)c.n_head, p0, x->bt.gy, csz, rec));
-      if (nch > 1 || mf)
+      DZ_HIP_CHECK(launch_bt_attn_mfma(grp, (int)c.n_head_kv, nch, s, x->bt.qb, kc, vc, (int)c.max_ctx, (int)c.n_head, p0, n,
+                                       csz, rec, x->bt.gate, x->bt.gy));
+      if (nch > 1)
         DZ_HIP_CHECK(launch(bt_attn_merge_kernel, dim3(nb, (unsigned)c.n_head), dim3(256), s, (const float*)rec, nch,
                             (const float*)x->bt.gate, (int)c.n_head, x->bt.gy));
       if ((rc = bt_gemm(x, l.out_proj, x->bt.gy, qd, n, nullptr, x->bt.h, H, 1))) return rc;
