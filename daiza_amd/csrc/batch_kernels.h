@@ -231,6 +231,342 @@ __global__ __launch_bounds__(256) void bt_scan_kernel(const float* __restrict__ 
   if (!rec.d) state_row_store(S, s);
 }
 
+// ---- the delta rule over many tokens, 32 at a time on the matrix cores ----
+//
+// With a_t the decay, β_t the gate, L_t = Σ_{s<=t} ln a_s within a chunk of 32 tokens and S the state before
+// it, the recurrence of bt_scan_kernel is, for the chunk's tokens together:
+//   N[t][s] = β_t e^(L_t - L_s) k_t·k_s (s < t),  T = (I + N)^-1
+//   U = T diag(β) V,  W = T diag(β e^L) K          [32][128] each
+//   D = U - W S^T                                    the tokens' deltas d_t
+//   Y = diag(e^L) Q S^T + A D,  A[t][s] = e^(L_t - L_s) q_t·k_s (s <= t)
+//   S <- e^(L_31) S + Σ_t e^(L_31 - L_t) d_t k_t^T
+// bt_chunk_prep_kernel forms what does not depend on the state (-W, U, A, K^T and the decays) for every
+// chunk at once; bt_chunk_scan_kernel walks the chunks.  All products are f32 matrix instructions; L is
+// summed and subtracted in f64 (ln a is known directly, so e^(L_t - L_s) keeps an f32's precision), and
+// every factor is at most 1.  The token-by-token kernel is one chain of about 1100 cycles per token (489 us
+// for 1024 tokens of 48 heads, 161 for 333); the chunks take 37 + 145 us (prep + walk), 18 + 56 for 333.
+constexpr int kScanC = 32;
+
+// What bt_chunk_prep_kernel leaves for the walk, per chunk c and v-head (k-head for kt).
+struct ChunkPrep {
+  float* w;   // [c][nvh][32][128]  -W
+  float* u;   // [c][nvh][32][128]
+  float* a;   // [c][nvh][32][32]
+  float* kt;  // [c][nkh][128][32]  K^T
+  float* g;   // [c][nvh][2][32]    e^(L_t), e^(L_31 - L_t)
+};
+__host__ __device__ inline size_t chunk_prep_floats(int n, int nkh, int nvh) {
+  const size_t c = (size_t)(n + kScanC - 1) / kScanC;
+  return c * ((size_t)nvh * (2 * kScanC * 128 + kScanC * kScanC + 2 * kScanC) + (size_t)nkh * 128 * kScanC);
+}
+__host__ __device__ inline ChunkPrep chunk_prep_carve(float* p, int n, int nkh, int nvh) {
+  const size_t c = (size_t)(n + kScanC - 1) / kScanC, hv = c * nvh;
+  ChunkPrep r;
+  r.w = p;
+  r.u = r.w + hv * kScanC * 128;
+  r.a = r.u + hv * kScanC * 128;
+  r.kt = r.a + hv * kScanC * kScanC;
+  r.g = r.kt + c * nkh * 128 * kScanC;
+  return r;
+}
+
+// Grid (nvh, chunks), 256 threads.  Tokens past n count as k = q = v = 0, β = 0, a = 1.
+// 16x16x4 f32 products: A lane (row = lane & 15, slot = lane >> 4), B lane (column, slot), D lane column
+// lane & 15, rows 4(lane >> 4) + i; step r of a 16-wide K block takes K index 4·slot + r, so that a lane's
+// four A values are one float4 of a row and a D tile's registers are the B operand of the next product.
+__global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __restrict__ yin, int64_t ldin,
+                                                            const float* __restrict__ cout, int64_t qkvd,
+                                                            const float* __restrict__ qk, int n, int nkh, int nvh,
+                                                            int64_t off_a, int64_t off_b, const float* __restrict__ ssm_a,
+                                                            const float* __restrict__ dt_bias, ChunkPrep o) {
+  constexpr int HD = 128, C = kScanC, LDT = 36;
+  __shared__ double Ls[C];
+  __shared__ float la[C], bet[C], be[C];  // ln a, β, β e^L
+  __shared__ __align__(16) float N[C][LDT], T[C][LDT];
+  const int vh = blockIdx.x, c = blockIdx.y, kh = vh % nkh, t0 = c * C;
+  const unsigned tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
+  const int ln = (int)(lane & 15u), lk = (int)(lane >> 4);
+  const int64_t kdim = (int64_t)nkh * HD;
+  if (tid < C) {
+    const int t = t0 + (int)tid, tc = min(t, n - 1);
+    const float x = yin[(size_t)tc * ldin + off_a + vh] + dt_bias[vh], b = yin[(size_t)tc * ldin + off_b + vh];
+    const float spl = x > 20.0f ? x : logf(1.0f + expf(x));
+    la[tid] = t < n ? ssm_a[vh] * spl : 0.f;
+    bet[tid] = t < n ? sigmoidf_(b) : 0.f;
+  }
+  __syncthreads();
+  if (tid < C) {
+    double L = 0.0, last = 0.0;
+    for (int s = 0; s < C; ++s) {
+      last += (double)la[s];
+      if (s <= (int)tid) L += (double)la[s];
+    }
+    Ls[tid] = L;
+    const float eL = expf((float)L);
+    be[tid] = bet[tid] * eL;
+    float* g = o.g + ((size_t)c * nvh + vh) * 2 * C;
+    g[tid] = eL;
+    g[C + tid] = expf((float)(last - L));
+  }
+  __syncthreads();
+  const size_t hv = (size_t)c * nvh + vh;
+  // K·K^T and Q·K^T: wave w < 3 takes tile (t, s) = (0, 0), (1, 0), (1, 1); tile (0, 1) lies above the diagonal
+  auto krow = [&](int t) { return qk + (size_t)min(t0 + t, n - 1) * 2 * kdim + kdim + (size_t)kh * HD; };
+  if (w < 3) {
+    const int tt = w > 0, ts = w > 1;
+    const float* kr = krow(16 * tt + ln) + 4 * lk;
+    const float* qr = qk + (size_t)min(t0 + 16 * tt + ln, n - 1) * 2 * kdim + (size_t)kh * HD + 4 * lk;
+    const float* sr = krow(16 * ts + ln) + 4 * lk;
+    f32x4 dk = {0.f, 0.f, 0.f, 0.f}, dq = dk;
+#pragma unroll
+    for (int J = 0; J < HD / 16; ++J) {
+      const float4 ka = *reinterpret_cast<const float4*>(kr + 16 * J), qa = *reinterpret_cast<const float4*>(qr + 16 * J),
+                   sb = *reinterpret_cast<const float4*>(sr + 16 * J);
+      dk = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, sb.x, dk, 0, 0, 0);
+      dq = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.x, sb.x, dq, 0, 0, 0);
+      dk = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, sb.y, dk, 0, 0, 0);
+      dq = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.y, sb.y, dq, 0, 0, 0);
+      dk = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, sb.z, dk, 0, 0, 0);
+      dq = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.z, sb.z, dq, 0, 0, 0);
+      dk = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.w, sb.w, dk, 0, 0, 0);
+      dq = __builtin_amdgcn_mfma_f32_16x16x4f32(qa.w, sb.w, dq, 0, 0, 0);
+    }
+    const int s = 16 * ts + ln;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * tt + 4 * lk + i;
+      const bool in = t0 + t < n;  // (a token past n has read the last one's rows)
+      const float e = s <= t && in ? expf((float)(Ls[t] - Ls[s])) : 0.f;
+      N[t][s] = s < t ? bet[t] * e * dk[i] : 0.f;
+      o.a[(hv * C + t) * C + s] = e * dq[i];
+    }
+  } else {  // the tile above the diagonal, and (once per k-head) K^T
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.a[(hv * C + 4 * lk + i) * C + 16 + ln] = 0.f;
+    if (vh < nkh) {
+      float* kt = o.kt + ((size_t)c * nkh + kh) * HD * C;
+      // lane: token lane & 31, dims 64(lane >> 5) .. +63
+      const int t = (int)(lane & 31u), j0 = 64 * (int)(lane >> 5);
+      const float4* kr = reinterpret_cast<const float4*>(krow(t) + j0);
+      const bool in = t0 + t < n;
+      float4 f[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) f[j] = kr[j];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        float* d = kt + (size_t)(j0 + 4 * j) * C + t;
+        d[0] = in ? f[j].x : 0.f;
+        d[C] = in ? f[j].y : 0.f;
+        d[2 * C] = in ? f[j].z : 0.f;
+        d[3 * C] = in ? f[j].w : 0.f;
+      }
+    }
+  }
+  __syncthreads();
+  // T = [[T0, 0], [-T1 N10 T0, T1]]: the 16x16 inverses T0 and T1 by forward substitution, a column per
+  // lane (four partial sums break the chain), then the block below by two products
+  if (w == 0) {
+    if (lane < 32u) {
+      const int b0 = 16 * lk;  // lanes 0..15: T0, 16..31: T1
+      float col[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        float p[4] = {t == ln ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < t; ++s) p[s & 3] = __builtin_fmaf(-N[b0 + t][b0 + s], col[s], p[s & 3]);
+        col[t] = (p[0] + p[1]) + (p[2] + p[3]);
+        T[b0 + t][b0 + ln] = col[t];
+      }
+    }
+    __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
+    f32x4 m = {0.f, 0.f, 0.f, 0.f}, tl = m;
+    const float4 na = *reinterpret_cast<const float4*>(&N[16 + ln][4 * lk]);
+    const float4 t1 = *reinterpret_cast<const float4*>(&T[16 + ln][16 + 4 * lk]);
+    const float nr[4] = {na.x, na.y, na.z, na.w}, tr[4] = {t1.x, t1.y, t1.z, t1.w};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) m = __builtin_amdgcn_mfma_f32_16x16x4f32(nr[r], T[4 * lk + r][ln], m, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tl = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[r], m[r], tl, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T[16 + 4 * lk + i][ln] = -tl[i];
+  }
+  __syncthreads();
+  // -W and U: wave w takes columns 32w .. 32w + 31 of both
+#pragma unroll
+  for (int jt = 0; jt < 2; ++jt) {
+    const int col = 32 * (int)w + 16 * jt + ln;
+    float kx[2][4], vx[2][4];
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int s = 16 * st + 4 * lk + r;
+        const float* vr = cout + (size_t)min(t0 + s, n - 1) * qkvd + 2 * kdim + (size_t)vh * HD;
+        kx[st][r] = krow(s)[col];
+        vx[st][r] = vr[col];
+      }
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int s = 16 * st + 4 * lk + r;
+        kx[st][r] *= -be[s];
+        vx[st][r] *= bet[s];
+      }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      f32x4 dw = {0.f, 0.f, 0.f, 0.f}, du = dw;
+#pragma unroll
+      for (int st = 0; st <= tt; ++st) {
+        const float4 ta = *reinterpret_cast<const float4*>(&T[16 * tt + ln][16 * st + 4 * lk]);
+        const float tr[4] = {ta.x, ta.y, ta.z, ta.w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          dw = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[r], kx[st][r], dw, 0, 0, 0);
+          du = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[r], vx[st][r], du, 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const size_t off = (hv * C + 16 * tt + 4 * lk + i) * HD + col;
+        o.w[off] = dw[i];
+        o.u[off] = du[i];
+      }
+    }
+  }
+}
+
+// The walk over the chunks: one wave per (v-head, 16 rows i of its state), no exchange between waves.  The
+// state's S^T tiles (rows j, columns i) stay in the wave's accumulators and are the B operands of W S^T and
+// Q S^T; D's tiles are the B operands of A D and K^T D.  W, U and Q are requested two chunks ahead, the
+// rest when this chunk is done with it.  Bound by the f32 matrix instructions (208 of 32 cycles per chunk, one wave per
+// SIMD on 384 of the 1024 SIMDs).  Workgroup b runs on XCD b % 8, which takes heads b % 8 + 8k: the eight
+// waves of a head read the same operands in one L2.  Grid 8·8·ceil(nvh / 8), 64 threads.
+__global__ __launch_bounds__(64) void bt_chunk_scan_kernel(const float* __restrict__ qk, int n, int nkh, int nvh,
+                                                           const ChunkPrep o, float* __restrict__ state,
+                                                           float* __restrict__ y) {
+  constexpr int HD = 128, C = kScanC;
+  const int b = (int)blockIdx.x, vh = (b >> 6) * 8 + (b & 7), ib = (b >> 3) & 7;
+  if (vh >= nvh) return;
+  const int lane = (int)threadIdx.x, ln = lane & 15, lk = lane >> 4, kh = vh % nkh;
+  const int i = 16 * ib + ln;
+  const int64_t kdim = (int64_t)nkh * HD;
+  float* Sp = state + (size_t)vh * HD * HD + (size_t)i * HD + 4 * lk;
+  f32x4 S[8];  // S^T tile J: rows j = 16J + 4lk + r, column i
+#pragma unroll
+  for (int J = 0; J < 8; ++J) S[J] = *reinterpret_cast<const f32x4*>(Sp + 16 * J);
+  const int nc = (n + C - 1) / C;
+  // W, Q rows t (of two chunks); K^T rows j; A tiles (0,0), (1,0), (1,1)
+  struct WQ {
+    f32x4 w[2][8], q[2][8];
+    float u[2][4];
+  } even, odd;
+  f32x4 kv[8][2], av[3];
+  f32x4 ge[2], gd[2];
+  auto load_w = [&](int c, WQ& o_) {
+    const float* p = o.w + (((size_t)c * nvh + vh) * C + ln) * HD + 4 * lk;
+    const float* u = o.u + (((size_t)c * nvh + vh) * C + 4 * lk) * HD + i;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+#pragma unroll
+      for (int J = 0; J < 8; ++J) o_.w[tt][J] = *reinterpret_cast<const f32x4*>(p + 16 * tt * HD + 16 * J);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o_.u[tt][r] = u[(16 * tt + r) * HD];
+    }
+  };
+  auto load_q = [&](int c, WQ& o_) {
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      const float* p = qk + (size_t)min(c * C + 16 * tt + ln, n - 1) * 2 * kdim + (size_t)kh * HD + 4 * lk;
+#pragma unroll
+      for (int J = 0; J < 8; ++J) o_.q[tt][J] = *reinterpret_cast<const f32x4*>(p + 16 * J);
+    }
+  };
+  auto load_k = [&](int c) {
+    const size_t hv = (size_t)c * nvh + vh;
+    const float* p = o.kt + (((size_t)c * nkh + kh) * HD + ln) * C + 4 * lk;
+#pragma unroll
+    for (int J = 0; J < 8; ++J)
+#pragma unroll
+      for (int st = 0; st < 2; ++st) kv[J][st] = *reinterpret_cast<const f32x4*>(p + (size_t)16 * J * C + 16 * st);
+    const float* a = o.a + (hv * C + ln) * C + 4 * lk;
+    av[0] = *reinterpret_cast<const f32x4*>(a);
+    av[1] = *reinterpret_cast<const f32x4*>(a + 16 * C);
+    av[2] = *reinterpret_cast<const f32x4*>(a + 16 * C + 16);
+    const float* g = o.g + hv * 2 * C + 4 * lk;
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      ge[tt] = *reinterpret_cast<const f32x4*>(g + 16 * tt);
+      gd[tt] = *reinterpret_cast<const f32x4*>(g + C + 16 * tt);
+    }
+  };
+  load_w(0, even);
+  load_q(0, even);
+  load_k(0);
+  load_w(min(1, nc - 1), odd);
+  load_q(min(1, nc - 1), odd);
+  auto chunk = [&](int c, WQ& x) {
+    f32x4 d[2], yy[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      d[tt] = f32x4{x.u[tt][0], x.u[tt][1], x.u[tt][2], x.u[tt][3]};
+      yy[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int J = 0; J < 8; ++J)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        d[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[0][J][r], S[J][r], d[0], 0, 0, 0);
+        d[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[1][J][r], S[J][r], d[1], 0, 0, 0);
+        yy[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[0][J][r], S[J][r], yy[0], 0, 0, 0);
+        yy[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[1][J][r], S[J][r], yy[1], 0, 0, 0);
+      }
+    load_w(min(c + 2, nc - 1), x);
+    load_q(min(c + 2, nc - 1), x);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) yy[tt][r] *= ge[tt][r];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      yy[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[0][r], d[0][r], yy[0], 0, 0, 0);
+      yy[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[1][r], d[0][r], yy[1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) yy[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[2][r], d[1][r], yy[1], 0, 0, 0);
+    // e^(L_31): the last token's e^(L_t), in lane group 3's fourth slot of the second tile
+    const float gc = __shfl(ge[1][3], 48);
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[tt][r] *= gd[tt][r];
+#pragma unroll
+    for (int J = 0; J < 8; ++J)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[J][r] *= gc;
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int J = 0; J < 8; ++J) S[J] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[J][st][r], d[st][r], S[J], 0, 0, 0);
+    load_k(min(c + 1, nc - 1));
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = c * C + 16 * tt + 4 * lk + r;
+        if (t < n) y[(size_t)t * nvh * HD + (size_t)vh * HD + i] = yy[tt][r];
+      }
+  };
+  for (int c = 0; c < nc; c += 2) {
+    chunk(c, even);
+    if (c + 1 < nc) chunk(c + 1, odd);
+  }
+#pragma unroll
+  for (int J = 0; J < 8; ++J) *reinterpret_cast<f32x4*>(Sp + 16 * J) = S[J];
+}
+
 // Applies the first a recorded tokens of a verify chunk to the state: s = decay·s, s = fma(d, k, s)
 // per token, the same operations in the same order as the scan, so the result equals a scan over
 // those a tokens.  Grid 4·nvh, 256 threads (the scan's row mapping).

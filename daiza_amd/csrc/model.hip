@@ -101,7 +101,7 @@ struct dz_ctx {
     float *ygu = nullptr, *sw = nullptr, *qb = nullptr, *gate = nullptr;
     float* logits = nullptr;  // [logits_rows][vocab]
     int logits_rows = 0;
-    dz::Scratch pack, split, arec, spec;
+    dz::Scratch pack, split, arec, spec, chunk;
     // verify records per DeltaNet layer: conv inputs [kv][qkvd] and the scan's rollback record
     int kv_cap = 0;
     std::vector<float*> rx;
@@ -1256,10 +1256,12 @@ static void bt_release(dz_ctx* x) {
   if (x->bt.split.ptr) (void)hipFree(x->bt.split.ptr);
   if (x->bt.arec.ptr) (void)hipFree(x->bt.arec.ptr);
   if (x->bt.spec.ptr) (void)hipFree(x->bt.spec.ptr);
+  if (x->bt.chunk.ptr) (void)hipFree(x->bt.chunk.ptr);
   x->bt.pack = Scratch{};
   x->bt.split = Scratch{};
   x->bt.arec = Scratch{};
   x->bt.spec = Scratch{};
+  x->bt.chunk = Scratch{};
 }
 
 // Activation buffers for chunks of up to cap tokens.
@@ -1384,6 +1386,11 @@ static int bt_gemm(dz_ctx* x, const Q1Dev& W, const float* xin, int64_t ldx, int
   return DZ_OK;
 }
 
+// From this many tokens the delta rule goes by chunks of 32 (bt_chunk_prep_kernel, bt_chunk_scan_kernel)
+// instead of token by token: a chunk costs about 5 us and the prep 13, a token of the other kernel 0.48,
+// so the line lies at about one chunk; a verify chunk keeps the token kernel, whose records the commit replays.
+constexpr int kScanMinTokens = 33;
+
 // The forward of tokens ids[0..n) (host) at positions pos_host .. pos_host+n-1 (forward_batch,
 // forward.rs:394-1407, with the per-token block order of forward.rs:204-375).  Writes the logits
 // of the last out_rows tokens to bt.logits.  With verify set, the DeltaNet states and conv rings
@@ -1429,10 +1436,20 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
                             n, ring, head0, qkvd));
       }
       float* state = x->ssm_state + (size_t)si * c.ssm_v_heads * hd * hd;
-      DZ_HIP_CHECK(launch(bt_scan_kernel, dim3((unsigned)(4 * c.ssm_v_heads)), dim3(256), s, (const float*)x->bt.yin,
-                          ld_in, (const float*)x->bt.cout, qkvd, (const float*)x->bt.qk, n, (int)c.ssm_k_heads,
-                          (int)c.ssm_v_heads, qkvd + inner, qkvd + inner + c.ssm_v_heads, (const float*)l.ssm_a,
-                          (const float*)l.dt_bias, state, x->bt.ys, rec));
+      const int nkh = (int)c.ssm_k_heads, nvh = (int)c.ssm_v_heads;
+      if (!verify && n >= kScanMinTokens) {
+        if ((rc = x->bt.chunk.reserve(chunk_prep_floats(n, nkh, nvh) * sizeof(float)))) return rc;
+        const ChunkPrep cp = chunk_prep_carve(static_cast<float*>(x->bt.chunk.ptr), n, nkh, nvh);
+        DZ_HIP_CHECK(launch(bt_chunk_prep_kernel, dim3((unsigned)nvh, (unsigned)((n + kScanC - 1) / kScanC)), dim3(256), s,
+                            (const float*)x->bt.yin, ld_in, (const float*)x->bt.cout, qkvd, (const float*)x->bt.qk, n, nkh,
+                            nvh, qkvd + inner, qkvd + inner + nvh, (const float*)l.ssm_a, (const float*)l.dt_bias, cp));
+        DZ_HIP_CHECK(launch(bt_chunk_scan_kernel, dim3((unsigned)(64 * ((nvh + 7) / 8))), dim3(64), s,
+                            (const float*)x->bt.qk, n, nkh, nvh, cp, state, x->bt.ys));
+      } else {
+        DZ_HIP_CHECK(launch(bt_scan_kernel, dim3((unsigned)(4 * nvh)), dim3(256), s, (const float*)x->bt.yin, ld_in,
+                            (const float*)x->bt.cout, qkvd, (const float*)x->bt.qk, n, nkh, nvh, qkvd + inner,
+                            qkvd + inner + nvh, (const float*)l.ssm_a, (const float*)l.dt_bias, state, x->bt.ys, rec));
+      }
       DZ_HIP_CHECK(launch(bt_gate_y_kernel, dim3(nb, (unsigned)c.ssm_v_heads), dim3(128), s, (const float*)x->bt.ys,
                           (const float*)x->bt.yin, ld_in, qkvd, (const float*)l.ssm_norm, c.rms_eps,
                           (int)c.ssm_v_heads, x->bt.gy));
