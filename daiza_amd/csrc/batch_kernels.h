@@ -4,6 +4,7 @@
 // DeltaNet scan records what a rollback needs instead of writing the state back.
 #pragma once
 #include "model_kernels.h"
+#include "q1_digits.h"
 
 namespace dz {
 
@@ -18,30 +19,36 @@ __device__ __forceinline__ float lane8_sum(float v) {
 
 // h[t] = embedding row of ids[t] (forward.rs:212): the f16 table through the reference's
 // f16_to_f32 (tensor/tensor.rs:62-76), or a Q1_0 table through dequantize_q1_0_row_into
-// (quant.rs:161-194).  Grid n, 256 threads.
+// (quant.rs:161-194).  Grid (n, ceil(H / 1024)), 256 threads of four columns each: with one workgroup per token
+// the row's twenty dependent rounds took 13 us for eight tokens.
 __global__ __launch_bounds__(256) void bt_embed_kernel(const int* __restrict__ ids, int64_t H,
                                                        const uint16_t* __restrict__ emb_f16,
                                                        const uint8_t* __restrict__ emb_q1, int emb_ntiles,
                                                        float* __restrict__ h) {
   const int t = blockIdx.x;
   const int tok = ids[t];
-  float* out = h + (size_t)t * H;
+  const int64_t k0 = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 4;  // H is a multiple of 128
+  if (k0 >= H) return;
+  float o[4];
   if (emb_f16) {
-    const uint16_t* row = emb_f16 + (size_t)tok * H;
-    for (int64_t c = threadIdx.x; c < H; c += 256) out[c] = ref_f16_to_f32_dev(row[c]);
-    return;
-  }
-  const int64_t rb = tok / kRowBlock;
-  const unsigned L = (unsigned)(tok % kRowBlock);
-  for (int64_t k = threadIdx.x; k < H; k += 256) {
-    const int tt = (int)(k / kTileCols);
-    const unsigned p = (unsigned)((k % kTileCols) / 8), j = (unsigned)(k % 8), s = L ^ p;
+    const ushort4 v = *reinterpret_cast<const ushort4*>(emb_f16 + (size_t)tok * H + k0);
+    o[0] = ref_f16_to_f32_dev(v.x);
+    o[1] = ref_f16_to_f32_dev(v.y);
+    o[2] = ref_f16_to_f32_dev(v.z);
+    o[3] = ref_f16_to_f32_dev(v.w);
+  } else {
+    const int64_t rb = tok / kRowBlock;
+    const unsigned L = (unsigned)(tok % kRowBlock);
+    const int tt = (int)(k0 / kTileCols);
+    const unsigned p = (unsigned)((k0 % kTileCols) / 8), s = L ^ p;
     const uint8_t* u = emb_q1 + ((size_t)rb * emb_ntiles + tt) * kUnitBytes;
     const unsigned byte = u[((s >> 4) * 64 + L) * 16 + (s & 15)];
     const uint16_t* scp = reinterpret_cast<const uint16_t*>(u + kUnitSignBytes);
     const float scale = ref_f16_to_f32_dev(scp[L * 4 + ((p >> 4) ^ (L >> 4))]);
-    out[k] = ((float)((byte >> j) & 1u) * 2.0f - 1.0f) * scale;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = ((float)((byte >> ((k0 & 7) + i)) & 1u) * 2.0f - 1.0f) * scale;
   }
+  *reinterpret_cast<float4*>(h + (size_t)t * H + k0) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
 // Causal conv over the chunk + SiLU (ssm.rs:467-518): out[t][ch] = silu(Σ_tap x[t-3+tap][ch]·w[tap][ch]),
@@ -915,6 +922,139 @@ __global__ __launch_bounds__(256) void bt_attn_merge_kernel(const float* __restr
   ao[((size_t)t * nq + h) * HD + tid] = (O * (1.0f / L)) * sigmoidf_(gt);
 }
 
+// ---- few tokens (n <= 16): the kernels that form a product's activations hand them over as digits ----
+//
+// One wave per (token, K tile of the next product), lane columns 4·lane .. +3 and 256 + 4·lane .. +3 of the tile; the
+// digits go to dig[tile] (FewForm<T>), for a normed product with the next norm's weight nw multiplied in and the
+// tile's sum of squares beside them (ssq[tile][n]).  Grid (tiles, n), 64 threads.
+template <int T>
+struct FewOut {
+  uint8_t* dig;
+  const float* nw;  // null: no norm follows
+  float* ssq;
+  int64_t K;
+};
+template <int T>
+__device__ __forceinline__ void few_out(const FewOut<T>& o, float4 x0, float4 x1) {
+  __shared__ __align__(16) unsigned char rec[few_rec<T>()];
+  __shared__ __align__(16) float st[kFewStage / 4];
+  const unsigned lane = threadIdx.x;
+  const int t = blockIdx.x, tok = blockIdx.y;
+  if (o.nw) {
+    const float s = wave_sum(((x0.x * x0.x + x0.y * x0.y) + (x0.z * x0.z + x0.w * x0.w)) +
+                             ((x1.x * x1.x + x1.y * x1.y) + (x1.z * x1.z + x1.w * x1.w)));
+    if (lane == 0) o.ssq[(size_t)t * gridDim.y + tok] = s;
+    const int64_t c0 = (int64_t)t * kTileCols + 4 * lane;  // columns past K hold zeros
+    const float4 w0 = *reinterpret_cast<const float4*>(o.nw + (c0 < o.K ? c0 : 0));
+    const float4 w1 = *reinterpret_cast<const float4*>(o.nw + (c0 + 256 < o.K ? c0 + 256 : 0));
+    x0 = make_float4(x0.x * w0.x, x0.y * w0.y, x0.z * w0.z, x0.w * w0.w);
+    x1 = make_float4(x1.x * w1.x, x1.y * w1.y, x1.z * w1.z, x1.w * w1.w);
+  }
+  few_pack_out<T>(o.dig + (size_t)t * FewForm<T>::kTile, rec, st, lane, tok, x0, x1);
+}
+
+// out[m] = Σ_z p[m][z·stride] for z < n in split order (four consecutive columns each), N splits of all M sums in
+// flight at a time (a split past n reloads the last one; its value is not added): one memory round trip per N.
+template <int M, int N>
+__device__ __forceinline__ void ordered_sums4(const float* const (&p)[M], int64_t stride, int n, float4 (&out)[M]) {
+  for (int b = 0; b < n; b += N) {
+    float4 v[N][M];
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int m = 0; m < M; ++m) v[k][m] = *reinterpret_cast<const float4*>(p[m] + (size_t)min(b + k, n - 1) * stride);
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first sum waits for one
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const float4 f = v[k][m];
+        if (b + k == 0) out[m] = f;
+        else if (b + k < n) out[m] = make_float4(out[m].x + f.x, out[m].y + f.y, out[m].z + f.z, out[m].w + f.w);
+      }
+  }
+}
+
+// h += Σ_z part[z] (a split product into the residual; part null: h as it is), and h's digits.
+template <int T>
+__global__ __launch_bounds__(64) void few_resid_kernel(float* __restrict__ h, int64_t H, const float* __restrict__ part,
+                                                       int splits, int64_t zstride, FewOut<T> o) {
+  const int64_t c0 = (int64_t)blockIdx.x * kTileCols + 4 * threadIdx.x, c1 = c0 + 256;
+  const size_t row = (size_t)blockIdx.y * H;
+  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int64_t cc[2] = {c0 < H ? c0 : 0, c1 < H ? c1 : 0};
+  float4 x[2] = {*reinterpret_cast<const float4*>(h + row + cc[0]), *reinterpret_cast<const float4*>(h + row + cc[1])};
+  if (part) {
+    const float* const p[2] = {part + row + cc[0], part + row + cc[1]};
+    float4 d[2];
+    ordered_sums4<2, 18>(p, zstride, splits, d);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x[i] = make_float4(x[i].x + d[i].x, x[i].y + d[i].y, x[i].z + d[i].z, x[i].w + d[i].w);
+    if (c0 < H) *reinterpret_cast<float4*>(h + row + c0) = x[0];
+    if (c1 < H) *reinterpret_cast<float4*>(h + row + c1) = x[1];
+  }
+  if (c0 >= H) x[0] = z;
+  if (c1 >= H) x[1] = z;
+  few_out<T>(o, x[0], x[1]);
+}
+
+// silu(gate) · up from a split gate/up product's partials part[z][t][2F] (with its tokens' 1/rms), as digits.
+template <int T>
+__global__ __launch_bounds__(64) void few_swiglu_kernel(const float* __restrict__ part, int splits, int64_t zstride, int64_t F,
+                                                        const float* __restrict__ ssq, int ssq_n, int ssq_ld, int64_t K,
+                                                        float eps, FewOut<T> o) {
+  const int64_t c0 = (int64_t)blockIdx.x * kTileCols + 4 * threadIdx.x;
+  const size_t row = (size_t)blockIdx.y * 2 * F;
+  const int64_t d0 = c0 < F ? c0 : 0, d1 = c0 + 256 < F ? c0 + 256 : 0;
+  const float* const p[4] = {part + row + d0, part + row + d1, part + row + F + d0, part + row + F + d1};
+  float4 gu[4], x[2];
+  const float* sp = ssq + blockIdx.y;
+  const float sq = threadIdx.x < (unsigned)ssq_n ? sp[(size_t)threadIdx.x * ssq_ld] : 0.f;  // ssq_n <= 16 tiles of H
+  ordered_sums4<4, 5>(p, zstride, splits, gu);
+  const float inv = 1.0f / sqrtf(wave_sum(sq) / (float)K + eps);
+  const float4 g[2] = {gu[0], gu[1]}, u[2] = {gu[2], gu[3]};
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    x[i] = c0 + 256 * i < F ? make_float4(siluf_(g[i].x * inv) * (u[i].x * inv), siluf_(g[i].y * inv) * (u[i].y * inv),
+                                          siluf_(g[i].z * inv) * (u[i].z * inv), siluf_(g[i].w * inv) * (u[i].w * inv))
+                            : make_float4(0.f, 0.f, 0.f, 0.f);
+  few_out<T>(o, x[0], x[1]);
+}
+
+// bt_gate_y_kernel's result as digits: a tile holds four v-heads, each 32 lanes' columns of one half.
+template <int T>
+__global__ __launch_bounds__(64) void few_gate_kernel(const float* __restrict__ y, const float* __restrict__ yin, int64_t ldin,
+                                                      int64_t off_z, const float* __restrict__ nw, float eps, int nvh,
+                                                      FewOut<T> o) {
+  const unsigned lane = threadIdx.x;
+  const int64_t inner = (int64_t)nvh * 128, c0 = (int64_t)blockIdx.x * kTileCols + 4 * lane;
+  const int t = blockIdx.y;
+  float4 v[2], zz[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int64_t c = c0 + 256 * i, cc = c < inner ? c : 0;
+    v[i] = *reinterpret_cast<const float4*>(y + (size_t)t * inner + cc);
+    const float* zp = yin + (size_t)t * ldin + off_z + cc;  // rows of yin are not 16-byte aligned for every shape
+    zz[i] = make_float4(zp[0], zp[1], zp[2], zp[3]);
+  }
+  const float4 w = *reinterpret_cast<const float4*>(nw + 4 * (lane & 31u));
+  float4 x[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float s = (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    s = dpp_add<0xB1>(s);  // the 16 lanes of a DPP row, then the head's two rows
+    s = dpp_add<0x4E>(s);
+    s = dpp_add<0x141>(s);
+    s = dpp_add<0x140>(s);
+    s += __shfl_xor(s, 16);
+    const float inv = 1.0f / sqrtf(s * (1.0f / 128.0f) + eps);
+    x[i] = c0 + 256 * i < inner ? make_float4(((v[i].x * inv) * w.x) * siluf_(zz[i].x), ((v[i].y * inv) * w.y) * siluf_(zz[i].y),
+                                              ((v[i].z * inv) * w.z) * siluf_(zz[i].z), ((v[i].w * inv) * w.w) * siluf_(zz[i].w))
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  few_out<T>(o, x[0], x[1]);
+}
+
 // SwiGLU (mlp.rs:28-47, swiglu_inplace_simd): s[t][i] = silu(gate[t][i]) · up[t][i], gate rows
 // [0, F) and up rows [F, 2F) of the gate/up product.
 __global__ __launch_bounds__(256) void bt_swiglu_kernel(const float* __restrict__ gu, int64_t F, int n,
@@ -932,14 +1072,14 @@ __global__ __launch_bounds__(256) void bt_swiglu_kernel(const float* __restrict_
 __global__ __launch_bounds__(256) void bt_split_swiglu_kernel(const float* __restrict__ part, int splits,
                                                               int64_t zstride, int64_t F, int n,
                                                               float* __restrict__ s, const float* __restrict__ ssq,
-                                                              int ssq_ld, int64_t K, float eps) {
+                                                              int ssq_n, int ssq_ld, int64_t K, float eps) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int t = blockIdx.y;
   if (i >= F || t >= n) return;
   const size_t off = (size_t)t * 2 * F + i;
   float g = ordered_sum(part + off, zstride, splits), u = ordered_sum(part + off + F, zstride, splits);
   if (ssq) {  // a normed raw product: 1/rms applied to the sums
-    const float inv = split_inv_rms(ssq, ssq_ld, splits, t, K, eps);
+    const float inv = split_inv_rms(ssq, ssq_ld, ssq_n, t, K, eps);
     g *= inv;
     u *= inv;
   }

@@ -59,6 +59,26 @@ struct Q1Dev {
   int64_t ntiles = 0;          // K tiles (cols padded to 512)
 };
 
+// Sum over a full wave (all 64 lanes active).  DPP inside each row of 16 lanes (xor 1, xor 2,
+// half-row mirror, row mirror: every lane then holds its row's sum), then the four row sums
+// read with v_readlane; the result is wave-uniform and independent of lane order.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v = dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
+  v = dpp_add<0x141>(v);  // row_half_mirror
+  v = dpp_add<0x140>(v);  // row_mirror
+  const int b = __builtin_bit_cast(int, v);
+  const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0));
+  const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16));
+  const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32));
+  const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
+  return (r0 + r1) + (r2 + r3);
+}
+
 // p[0] + p[s] + p[2s] + ... + p[(n-1)s] (n >= 1), added in index order, with the loads issued 16 at a
 // time: a loop of dependent adds with a run-time count otherwise waits one memory round trip per term.
 // Every load of a round is issued (a term past n reloads term n-1, whose value is not added), so

@@ -101,7 +101,7 @@ struct dz_ctx {
     float *ygu = nullptr, *sw = nullptr, *qb = nullptr, *gate = nullptr;
     float* logits = nullptr;  // [logits_rows][vocab]
     int logits_rows = 0;
-    dz::Scratch pack, split, arec, spec, chunk;
+    dz::Scratch pack, split, arec, spec, chunk, dig;
     // verify records per DeltaNet layer: conv inputs [kv][qkvd] and the scan's rollback record
     int kv_cap = 0;
     std::vector<float*> rx;
@@ -1257,11 +1257,13 @@ static void bt_release(dz_ctx* x) {
   if (x->bt.arec.ptr) (void)hipFree(x->bt.arec.ptr);
   if (x->bt.spec.ptr) (void)hipFree(x->bt.spec.ptr);
   if (x->bt.chunk.ptr) (void)hipFree(x->bt.chunk.ptr);
+  if (x->bt.dig.ptr) (void)hipFree(x->bt.dig.ptr);
   x->bt.pack = Scratch{};
   x->bt.split = Scratch{};
   x->bt.arec = Scratch{};
   x->bt.spec = Scratch{};
   x->bt.chunk = Scratch{};
+  x->bt.dig = Scratch{};
 }
 
 // Activation buffers for chunks of up to cap tokens.
@@ -1371,9 +1373,9 @@ static int bt_attn_mfma_chunks(int n, int grp, int nkv, int ctx_max, int* csz) {
 static int bt_gemm(dz_ctx* x, const Q1Dev& W, const float* xin, int64_t ldx, int n, const float* norm_w, float* y,
                    int64_t ldy, int accumulate, GemmDefer* defer = nullptr) {
   if (n <= 16) {
-    // few tokens (verify): the product packs its tiles itself (folding in the RMSNorm, whose 1/rms is
-    // applied to the sums), which saves the packing launch; with many tokens every row-block group
-    // would repeat the packing of the same tiles
+    // few tokens whose activations no kernel has packed: the product packs its tiles itself (folding in the
+    // RMSNorm, whose 1/rms is applied to the sums), which saves a packing launch; with many tokens every
+    // row chunk would repeat the packing of the same tiles
     DZ_HIP_CHECK(launch_q1_gemm_raw(W, xin, ldx, n, y, ldy, accumulate, x->s, &x->bt.split, norm_w,
                                     x->m->cfg.rms_eps, defer));
     return DZ_OK;
@@ -1384,6 +1386,32 @@ static int bt_gemm(dz_ctx* x, const Q1Dev& W, const float* xin, int64_t ldx, int
   DZ_HIP_CHECK(launch_x_pack(xin, ldx, W.cols, n, norm_w, x->m->cfg.rms_eps, p, x->s));
   DZ_HIP_CHECK(launch_q1_gemm(W, p, n, y, ldy, accumulate, x->s, &x->bt.split, defer));
   return DZ_OK;
+}
+
+// Few tokens: where the activations of the next product go as digits (one buffer: each product has read it before
+// the next kernel writes it), and the sums of squares beside them.
+struct FewBuf {
+  uint8_t* dig;
+  float* ssq;
+};
+template <class F>
+static hipError_t with_few_form(int n, F&& f) {
+  if (n <= 2) f(std::integral_constant<int, 2>{});
+  else if (n <= 4) f(std::integral_constant<int, 4>{});
+  else if (n <= 8) f(std::integral_constant<int, 8>{});
+  else f(std::integral_constant<int, 16>{});
+  return hipGetLastError();
+}
+static hipError_t few_resid(dz_ctx* x, const FewBuf& fb, int n, const GemmDefer* gd, const float* norm_w) {
+  const int64_t H = x->m->cfg.hidden;
+  // a product with one split has added itself to h already
+  const bool add = gd && gd->part != x->bt.h;
+  return with_few_form(n, [&](auto B) {
+    constexpr int T = decltype(B)::value;
+    const FewOut<T> o{fb.dig, norm_w, fb.ssq, H};
+    hipLaunchKernelGGL(few_resid_kernel<T>, dim3((unsigned)((H + kTileCols - 1) / kTileCols), (unsigned)n), dim3(64), 0, x->s,
+                       x->bt.h, H, add ? gd->part : (const float*)nullptr, add ? gd->splits : 0, add ? gd->zstride : (int64_t)0, o);
+  });
 }
 
 // From this many tokens the delta rule goes by chunks of 32 (bt_chunk_prep_kernel, bt_chunk_scan_kernel)
@@ -1412,12 +1440,26 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
   const int64_t qd = (int64_t)c.n_head * c.head_dim;
   const size_t kvsz = (size_t)c.n_head_kv * c.max_ctx * c.head_dim;
   const unsigned nb = (unsigned)n;
-  DZ_HIP_CHECK(launch(bt_embed_kernel, dim3(nb), dim3(256), s, (const int*)x->bt.ids, H, (const uint16_t*)m->emb_f16,
+  DZ_HIP_CHECK(launch(bt_embed_kernel, dim3(nb, (unsigned)((H + 1023) / 1024)), dim3(256), s, (const int*)x->bt.ids, H, (const uint16_t*)m->emb_f16,
                       (const uint8_t*)m->emb_q1.data, (int)m->emb_q1.ntiles, x->bt.h));
+  // few tokens (verify, short batches): every kernel that forms a product's activations packs them
+  const bool few = n <= 16;
+  FewBuf fb{nullptr, nullptr};
+  GemmDefer gd;
+  if (few) {
+    const size_t tiles = (size_t)((std::max({H, F, inner, qd}) + kTileCols - 1) / kTileCols), db = tiles * few_tile_bytes(n);
+    if ((rc = x->bt.dig.reserve(db + tiles * n * sizeof(float)))) return rc;
+    fb.dig = static_cast<uint8_t*>(x->bt.dig.ptr);
+    fb.ssq = reinterpret_cast<float*>(fb.dig + db);
+    DZ_HIP_CHECK(few_resid(x, fb, n, nullptr, m->L[0].attn_norm));
+  }
   for (size_t li = 0; li < m->L.size(); ++li) {
     const LayerDev& l = m->L[li];
     const int64_t ld_in = l.in_proj.rows;
-    if ((rc = bt_gemm(x, l.in_proj, x->bt.h, H, n, l.attn_norm, x->bt.yin, ld_in, 0))) return rc;
+    if (few)
+      DZ_HIP_CHECK(launch_q1_few_packed(l.in_proj, fb.dig, fb.ssq, c.rms_eps, n, x->bt.yin, ld_in, 0, s, &x->bt.split));
+    else if ((rc = bt_gemm(x, l.in_proj, x->bt.h, H, n, l.attn_norm, x->bt.yin, ld_in, 0)))
+      return rc;
     if (!l.attn) {
       const int si = l.kind_idx;
       float* ring = x->conv + (size_t)si * 4 * qkvd;
@@ -1450,10 +1492,21 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
                             (const float*)x->bt.cout, qkvd, (const float*)x->bt.qk, n, nkh, nvh, qkvd + inner,
                             qkvd + inner + nvh, (const float*)l.ssm_a, (const float*)l.dt_bias, state, x->bt.ys, rec));
       }
-      DZ_HIP_CHECK(launch(bt_gate_y_kernel, dim3(nb, (unsigned)c.ssm_v_heads), dim3(128), s, (const float*)x->bt.ys,
-                          (const float*)x->bt.yin, ld_in, qkvd, (const float*)l.ssm_norm, c.rms_eps,
-                          (int)c.ssm_v_heads, x->bt.gy));
-      if ((rc = bt_gemm(x, l.out_proj, x->bt.gy, inner, n, nullptr, x->bt.h, H, 1))) return rc;
+      if (few) {
+        DZ_HIP_CHECK(with_few_form(n, [&](auto B) {
+          constexpr int T = decltype(B)::value;
+          const FewOut<T> o{fb.dig, nullptr, nullptr, inner};
+          hipLaunchKernelGGL(few_gate_kernel<T>, dim3((unsigned)((inner + kTileCols - 1) / kTileCols), nb), dim3(64), 0, s,
+                             (const float*)x->bt.ys, (const float*)x->bt.yin, ld_in, qkvd, (const float*)l.ssm_norm, c.rms_eps,
+                             (int)c.ssm_v_heads, o);
+        }));
+        DZ_HIP_CHECK(launch_q1_few_packed(l.out_proj, fb.dig, nullptr, 0.f, n, x->bt.h, H, 1, s, &x->bt.split, &gd));
+      } else {
+        DZ_HIP_CHECK(launch(bt_gate_y_kernel, dim3(nb, (unsigned)c.ssm_v_heads), dim3(128), s, (const float*)x->bt.ys,
+                            (const float*)x->bt.yin, ld_in, qkvd, (const float*)l.ssm_norm, c.rms_eps,
+                            (int)c.ssm_v_heads, x->bt.gy));
+        if ((rc = bt_gemm(x, l.out_proj, x->bt.gy, inner, n, nullptr, x->bt.h, H, 1))) return rc;
+      }
     } else {
       float* kc = x->kv + (size_t)l.kind_idx * 2 * kvsz;
       float* vc = kc + kvsz;
@@ -1474,21 +1527,37 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
       if (nch > 1)
         DZ_HIP_CHECK(launch(bt_attn_merge_kernel, dim3(nb, (unsigned)c.n_head), dim3(256), s, (const float*)rec, nch,
                             (const float*)x->bt.gate, (int)c.n_head, x->bt.gy));
-      if ((rc = bt_gemm(x, l.out_proj, x->bt.gy, qd, n, nullptr, x->bt.h, H, 1))) return rc;
+      if ((rc = bt_gemm(x, l.out_proj, x->bt.gy, qd, n, nullptr, x->bt.h, H, 1, few ? &gd : nullptr))) return rc;
     }
     // MLP (mlp.rs:28-47): h += W_down (silu(W_gate n) * W_up n), n = rmsnorm(h, post_attention_norm)
-    // a split gate/up product (few tokens) goes from its partials straight to the SwiGLU
-    GemmDefer gd;
+    if (few) {
+      DZ_HIP_CHECK(few_resid(x, fb, n, &gd, l.post_norm));
+      DZ_HIP_CHECK(launch_q1_few_packed(l.gate_up, fb.dig, fb.ssq, c.rms_eps, n, x->bt.ygu, 2 * F, 0, s, &x->bt.split, &gd));
+      DZ_HIP_CHECK(with_few_form(n, [&](auto B) {
+        constexpr int T = decltype(B)::value;
+        const FewOut<T> o{fb.dig, nullptr, nullptr, F};
+        hipLaunchKernelGGL(few_swiglu_kernel<T>, dim3((unsigned)((F + kTileCols - 1) / kTileCols), nb), dim3(64), 0, s, gd.part,
+                           gd.splits, gd.zstride, F, gd.ssq, gd.ssq_n, gd.ssq_ld, gd.K, gd.eps, o);
+      }));
+      DZ_HIP_CHECK(launch_q1_few_packed(l.down, fb.dig, nullptr, 0.f, n, x->bt.h, H, 1, s, &x->bt.split, &gd));
+      DZ_HIP_CHECK(few_resid(x, fb, n, &gd, li + 1 < m->L.size() ? m->L[li + 1].attn_norm : m->output_norm));
+      continue;
+    }
+    // a split gate/up product goes from its partials straight to the SwiGLU
     if ((rc = bt_gemm(x, l.gate_up, x->bt.h, H, n, l.post_norm, x->bt.ygu, 2 * F, 0, &gd))) return rc;
     if (gd.splits > 1)
       DZ_HIP_CHECK(launch(bt_split_swiglu_kernel, dim3((unsigned)((F + 255) / 256), nb), dim3(256), s, gd.part,
-                          gd.splits, gd.zstride, F, n, x->bt.sw, gd.ssq, gd.ssq_ld, gd.K, gd.eps));
+                          gd.splits, gd.zstride, F, n, x->bt.sw, gd.ssq, gd.ssq_n, gd.ssq_ld, gd.K, gd.eps));
     else
       DZ_HIP_CHECK(launch(bt_swiglu_kernel, dim3((unsigned)((F + 255) / 256), nb), dim3(256), s,
                           (const float*)x->bt.ygu, F, n, x->bt.sw));
     if ((rc = bt_gemm(x, l.down, x->bt.sw, F, n, nullptr, x->bt.h, H, 1))) return rc;
   }
   // output norm + lm_head for the last out_rows tokens
+  if (few && out_rows == n) {
+    DZ_HIP_CHECK(launch_q1_few_packed(m->lm_head, fb.dig, fb.ssq, c.rms_eps, n, x->bt.logits, c.vocab, 0, s, &x->bt.split));
+    return DZ_OK;
+  }
   const float* hl = x->bt.h + (size_t)(n - out_rows) * H;
   if ((rc = bt_gemm(x, m->lm_head, hl, H, out_rows, m->output_norm, x->bt.logits, c.vocab, 0))) return rc;
   return DZ_OK;

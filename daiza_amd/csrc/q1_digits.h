@@ -1,4 +1,4 @@
-// q1_digits.h — the N-column Q1_0 product for many tokens (prefill) on gfx950's scaled 4/6-bit
+// q1_digits.h — the N-column Q1_0 products (prefill, speculative verify) on gfx950's scaled 4/6-bit
 // matrix instruction: matvec_batch_into_slice / matvec_add_batch_into_slice
 // (Daiza-engine/src/model/weights.rs:475-682, 976-980).
 //
@@ -24,7 +24,7 @@
 // replaced: 34816 x 5120 865 -> 447 us, 16480 x 5120 457 -> 248, 5120 x 17408 565 -> 267 (with the
 // split sum), 5120 x 6144 204 -> 135; error against 64 bits of a four-layer block 4.3e-6 -> 0.9e-6.
 #pragma once
-#include "common.h"
+#include "q1_gemv.h"
 
 namespace dz {
 
@@ -33,33 +33,22 @@ typedef unsigned u32x6 __attribute__((ext_vector_type(6)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 6;
-constexpr int kFragBytes = 1536;                       // one digit operand: 64 lanes x 24 B (16 B plane, 8 B plane)
-constexpr int kHalfBytes = 2 * kDigits * kFragBytes;   // two groups (256 columns) of 16 tokens
-constexpr int kWideTokBlocks = 2;                      // 16-token blocks per workgroup
-constexpr int kWideTok = 16 * kWideTokBlocks;
-constexpr int kWideRb = 8;                             // row-blocks per workgroup (two per wave)
-constexpr int kWideStage = kWideTokBlocks * kHalfBytes;  // bytes of one staged half tile
-constexpr size_t kWideShmem = 2 * (size_t)kWideStage;
-
-// Digit operands of a batch of activations.
-//   dig: [16-token block][half tile h][group 2][digit 6][plane 0: 64 lanes x 16 B | plane 1: 64 x 8 B],
-//        lane (r = lane & 15, q = lane >> 4) holding token r's block q of the group; element 8k + j of
-//        a lane's 32 is column 4j + k of the block (expand_f4's order).
-//   ex:  [16-token block][tile][lane]: byte g = digit 0's block scale of group g.
-//   ssq: [tile][Np] sums of squares of the unweighted x (with an RMSNorm only).
-struct DigitX {
-  const uint8_t* dig;
-  const uint32_t* ex;
-  const float* ssq;
-  int Np;
-  int64_t K;
-  float eps;
-};
 
 // 32 signs (bit 4j + k of w = element 8k + j) as f4 values: bit set -> +1 (0x2), clear -> -1 (0xA).
 __device__ __forceinline__ void expand_f4(unsigned w, i32x8& a) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) a[k] = (int)(((w << (3 - k)) & 0x88888888u) ^ 0xAAAAAAAAu);
+}
+
+// Digit 0's block scale of a block whose largest |value| has the bits mb, and the exponent e its values are
+// taken by (v = x · 2^(4-e)).  Scales go down to 35 below digit 0's (an operand's zero slots included) and
+// have to stay block scales: a block whose largest value is below 2^-90 is held to 2^-115 absolute.
+__device__ __forceinline__ unsigned digit_scale(unsigned mb, int& e) {
+  e = 0;
+  if (mb >= 0x7F800000u) return 0xFFu;  // an infinity or a NaN in the block
+  (void)frexpf(__builtin_bit_cast(float, mb), &e);
+  e = mb == 0 ? 0 : (e < -90 ? -90 : e);
+  return (unsigned)(126 + e);
 }
 
 // The six digit operands and digit 0's block scale of 32 values (column order).
@@ -70,12 +59,9 @@ __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)
     const unsigned b = __builtin_bit_cast(unsigned, x[i]) & 0x7FFFFFFFu;
     mb = b > mb ? b : mb;
   }
-  const bool finite = mb < 0x7F800000u;
-  int e = 0;
-  (void)frexpf(__builtin_bit_cast(float, mb), &e);
-  // the smallest digit's scale 2^(e - 1 - 25) has to be a block scale too: a block whose largest value
-  // is below 2^-101 is held to 2^-126 absolute
-  e = !finite || mb == 0 ? 0 : (e < -101 ? -101 : e);
+  int e;
+  const unsigned b0 = digit_scale(mb, e);
+  const bool finite = b0 != 0xFFu;
   f32x16 a, b;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -96,270 +82,365 @@ __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)
     // element 2i = ra[i], 2i + 1 = rb[i], each over 8: code n for a whole n
     d[k] = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
   }
-  return finite ? (unsigned)(126 + e) : 0xFFu;
+  return b0;
 }
 
-// Grid (Np / 16, ntiles), 256 threads: wave g packs group g of the tile for 16 tokens, one block of 32
-// columns per lane; tokens past n_tok and columns past K are zero.  With w, the digits are those of
-// x ⊙ w and ssq gets the tile's sums of squares of x (rmsnorm_into, rmsnorm.rs:17-200, with 1/rms
-// applied to the product).  Bound by HBM: 4 B in and 4.5 B out per value.
-__global__ __launch_bounds__(256) void digit_pack_kernel(const float* __restrict__ x, int64_t ldx, int64_t K, int n_tok,
-                                                         const float* __restrict__ w, uint8_t* __restrict__ dig,
-                                                         uint32_t* __restrict__ ex, float* __restrict__ ssq, int Np) {
-  __shared__ unsigned sb[4][64];
-  __shared__ float ss[4][16];
-  const unsigned tid = threadIdx.x, lane = tid & 63u, g = tid >> 6, r = lane & 15u, q = lane >> 4;
-  const int tb = blockIdx.x, t = blockIdx.y;
-  const int tok = 16 * tb + (int)r;
-  const int64_t col = (int64_t)t * kTileCols + kGroup * g + 32 * q;
-  const bool live = tok < n_tok && col < K;
-  const float4* xp = reinterpret_cast<const float4*>(x + (live ? (size_t)tok * ldx + col : 0));
-  const float4* wp = reinterpret_cast<const float4*>(w + (live ? col : 0));
-  float v[32];
+// ---- few columns (n <= 16): every workgroup packs the tiles it needs itself ----
+//
+// The 16 rows of the token operand hold T tokens x P = 16/T digits (row ρ = p·T + token, digit f·P + p of
+// operand f), so a group of 128 columns takes F operands and F matrix instructions per 16 weight rows:
+//   n <= 2: T = 2, P = 8, F = 1;  n <= 4: T = 4, P = 4, F = 2;  n <= 8: T = 8, P = 2, F = 3;  else T = 16, F = 6
+// (slots past the six digits hold zeros).  A weight row's sums of the slots are kept apart until the end and
+// then added.
+template <int T>
+struct FewForm {
+  static constexpr int P = 16 / T;
+  static constexpr int F = (kDigits + P - 1) / P;
+  // LDS of a tile: [group][operand][block q: 416 B][row ρ: 24 B], the block and group strides chosen so that the
+  // 2-byte writes of the packing (16 blocks x 4 quarters at once) meet few banks twice
+  static constexpr int kBlk = 16 * 24 + 32;
+  static constexpr int kOp = 4 * kBlk;
+  static constexpr int kGrp = F * kOp + 32;
+  static constexpr int kEx = 4 * kGrp;                            // the block scales: [lane] a byte per group
+  static constexpr int kTile = kEx + 256;
+};
+constexpr int kFewStage = 16 * 36 * 4;  // a wave's 512 staged columns, blocks of 32 padded to 36
+
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_umax(unsigned v) {
+  const unsigned o = (unsigned)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, false);
+  return o > v ? o : v;
+}
+
+// One wave's 512 columns of a token (lane: columns 4·lane and 256 + 4·lane as x0, x1; st the wave's staging
+// area) split into digits: lane (block blk = lane >> 2, quarter kq) takes columns 4j + kq of its block, elements
+// 8kq .. 8kq + 7 of a digit operand: 48 bits, handed to put(digit, lo, hi) for every slot of form T (zero past
+// the six digits).  Returns digit 0's block scale.
+template <int T, class Put>
+__device__ __forceinline__ unsigned few_digits(float* st, unsigned lane, float4 x0, float4 x1, Put&& put) {
+  using FF = FewForm<T>;
+  *reinterpret_cast<float4*>(st + 36 * (lane >> 3) + 4 * (lane & 7u)) = x0;
+  *reinterpret_cast<float4*>(st + 36 * (8 + (lane >> 3)) + 4 * (lane & 7u)) = x1;
+  __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
+  const unsigned blk = lane >> 2, kq = lane & 3u;
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = st[36 * blk + 4 * j + kq];
+  __builtin_amdgcn_wave_barrier();
+  unsigned mb = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float4 f = xp[j];
-    v[4 * j] = live ? f.x : 0.f;
-    v[4 * j + 1] = live ? f.y : 0.f;
-    v[4 * j + 2] = live ? f.z : 0.f;
-    v[4 * j + 3] = live ? f.w : 0.f;
+    const unsigned b = __builtin_bit_cast(unsigned, v[j]) & 0x7FFFFFFFu;
+    mb = b > mb ? b : mb;
   }
-  if (w) {
-    float s = 0.f;
+  mb = dpp_umax<0xB1>(mb);  // the block's four quarters: quad xor 1, xor 2
+  mb = dpp_umax<0x4E>(mb);
+  int e;
+  const unsigned b0 = digit_scale(mb, e);
+  const int sh = 4 - e;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) s = __builtin_fmaf(v[i], v[i], s);
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    if (q == 0) ss[g][r] = s;
+  for (int j = 0; j < 8; ++j) v[j] = b0 != 0xFFu ? ldexpf(v[j], sh) : 0.f;
+  f32x16 ra = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, rb = ra;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float4 f = wp[j];
-      v[4 * j] *= f.x;
-      v[4 * j + 1] *= f.y;
-      v[4 * j + 2] *= f.z;
-      v[4 * j + 3] *= f.w;
-    }
-  }
-  u32x6 d[kDigits];
-  sb[g][lane] = pack_digits(v, d);
-  uint8_t* o = dig + (((size_t)tb * gridDim.y + t) * 2 + (g >> 1)) * kHalfBytes + (size_t)(g & 1u) * kDigits * kFragBytes;
+  for (int k = 0; k < FF::F * FF::P; ++k) {
+    unsigned lo = 0, hi = 0;
+    if (k < kDigits) {
 #pragma unroll
-  for (int k = 0; k < kDigits; ++k) {
-    *reinterpret_cast<u32x4*>(o + k * kFragBytes + 16 * lane) = u32x4{d[k][0], d[k][1], d[k][2], d[k][3]};
-    *reinterpret_cast<u32x2*>(o + k * kFragBytes + 1024 + 8 * lane) = u32x2{d[k][4], d[k][5]};
-  }
-  __syncthreads();
-  if (tid < 64) ex[((size_t)tb * gridDim.y + t) * 64 + tid] = sb[0][tid] | sb[1][tid] << 8 | sb[2][tid] << 16 | sb[3][tid] << 24;
-  if (w && tid < 16) ssq[(size_t)t * Np + 16 * tb + tid] = (ss[0][tid] + ss[1][tid]) + (ss[2][tid] + ss[3][tid]);
-}
-
-// N KiB (N <= 4) from g + voff (g wave-uniform, voff = 16·lane and whole KiB) to LDS lds_base + 16·lane:
-// 16 bytes per lane and KiB, without passing through registers.  The compiler does not count these
-// loads: the reader waits with lds_dma_wait before the barrier that publishes them.  (m0 holds the LDS
-// base; nothing else in these kernels uses it.)
-template <int N>
-__device__ __forceinline__ void lds_dma(const void* g, unsigned voff, unsigned lds_base) {
-  static_assert(N >= 1 && N <= 4, "the instruction offset holds three KiB");
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(g), "s"(lds_base) : "memory");
-  if constexpr (N > 1) asm volatile("global_load_lds_dwordx4 %0, %1 offset:1024" ::"v"(voff), "s"(g) : "memory");
-  if constexpr (N > 2) asm volatile("global_load_lds_dwordx4 %0, %1 offset:2048" ::"v"(voff), "s"(g) : "memory");
-  if constexpr (N > 3) asm volatile("global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(voff), "s"(g) : "memory");
-}
-__device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-// Ends one step of the product: the sums are formed before it and the next step's loads stay after it.
-// Without it the compiler reads all of a half tile's digit operands first, which takes more registers
-// than there are.
-__device__ __forceinline__ void step_fence(f32x4 (&d)[8]) {
-  asm volatile("" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]), "+v"(d[4]), "+v"(d[5]), "+v"(d[6]), "+v"(d[7])::"memory");
-}
-
-// A digit operand from LDS: the 16-byte plane, then the 8-byte plane.
-__device__ __forceinline__ i32x8 read_frag(const unsigned char* f, unsigned lane) {
-  const u32x4 lo = *reinterpret_cast<const u32x4*>(f + 16 * lane);
-  const u32x2 hi = *reinterpret_cast<const u32x2*>(f + 1024 + 8 * lane);
-  return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], 0, 0};
-}
-
-// Workgroup tile of the wide product: 512 rows x 32 tokens; the K loop goes by half tiles (two groups,
-// 256 columns).  Four waves, each holding 128 rows (eight 16-row blocks) x 32 tokens of f32 sums.
-//   A operand (lane & 15 = token): digit k of the token block, read from LDS and used for eight
-//     matrix instructions (one per 16-row block).
-//   B operand (lane & 15 = weight row): 32 signs of one group as f4.
-//   D: lane holds tokens 4q .. 4q+3 of weight row lane & 15, so a group's scale is one value per lane.
-// The digits of the next half tile travel to the other LDS buffer (lds_dma16) while this one is
-// multiplied; its signs go into the registers that the expansion has just read.  Two workgroups share a CU
-// (2 x 72 KiB of LDS), so one's barrier and scale fmas hide behind the other's matrix instructions.
-// Bound by the matrix instructions: per group and wave 96 of them (about 20 cycles each) against
-// 18 KiB of LDS reads (48 B per cycle and CU) and ~130 VALU operations.
-// Grid: 1-D, row groups x token groups x splits (wide_tile); y and splits as q1_gemm_kernel's.
-struct WideGrid {
-  int nrg;  // row groups: ceil(nrb / kWideRb)
-  int ntg;  // token groups: Np / kWideTok
-  int tps;  // K tiles per split
-};
-
-// Workgroup index -> (row group, token group, split).  The hardware deals workgroups to the eight XCDs in turn, so
-// XCD x takes a contiguous run of the tile order, and that order walks bands of eight row groups token group by token
-// group: the workgroups an XCD runs together share eight row groups' weights and a few token groups' digits in its L2.
-__device__ __forceinline__ void wide_tile(const WideGrid& g, int total, int& rg, int& tg, int& z) {
-  const int b = (int)blockIdx.x, per = g.nrg * g.ntg;
-  const int full = total / 8, rem = total % 8, x = b % 8;
-  int T = x * full + min(x, rem) + b / 8;
-  z = T / per;
-  T %= per;
-  const int band = T / (8 * g.ntg), r0 = 8 * band, w = min(8, g.nrg - r0), in = T - band * 8 * g.ntg;
-  tg = in / w;
-  rg = r0 + in % w;
-}
-
-__global__ __launch_bounds__(256, 2) void q1_wide_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb, int ntiles,
-                                                         const WideGrid wg, const DigitX x, int n_tok, float* __restrict__ y,
-                                                         int64_t ldy, int64_t zstride, int accumulate) {
-  constexpr int SB = 8, NB = kWideTokBlocks;
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ float tok_inv[kWideTok];
-  int rg, tg, z;
-  wide_tile(wg, (int)gridDim.x, rg, tg, z);
-  const unsigned tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
-  const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int t0 = z * wg.tps, t1 = min(ntiles, t0 + wg.tps);
-  const int s_end = 2 * t1;
-  y += (size_t)z * zstride;
-  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
-  // stage s's digits of the workgroup's token blocks: 36 KiB, nine consecutive ones per wave (two waves
-  // per token block)
-  static_assert(kHalfBytes == 2 * 9216 && NB == 2, "nine KiB per wave");
-  const uint8_t* dsrc = x.dig + ((size_t)(tg * NB + (int)(wave >> 1)) * ntiles * 2) * kHalfBytes + 9216 * (wave & 1u);
-  auto stage = [&](int s, int b) {
-    const uint8_t* src = dsrc + (size_t)s * kHalfBytes;
-    const unsigned dst = lds0 + (unsigned)b * kWideStage + 9216u * wave;
-    lds_dma<4>(src, 16 * lane, dst);
-    lds_dma<4>(src, 16 * lane + 4096, dst + 4096);
-    lds_dma<1>(src, 16 * lane + 8192, dst + 8192);
-  };
-  // the weights of the workgroup's row-blocks; reads past the matrix return 0 (those rows are not stored)
-  const int64_t rb0 = (int64_t)rg * kWideRb + 2 * wave;
-  const size_t wbytes = (size_t)(nrb - (int64_t)rg * kWideRb) * ntiles * kUnitBytes;
-  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(W) + (size_t)rg * kWideRb * ntiles * kUnitBytes, 0, (int)(wbytes < 0x7FFFFFFFu ? wbytes : 0x7FFFFFFFu), 0x00027000);
-  const int u0 = (int)(2 * wave) * ntiles * kUnitBytes, u1 = u0 + ntiles * kUnitBytes;
-  const int woff = (int)(16u * r + 4u * (q ^ (r >> 2)));   // the lane's dword of a 16-row block's chunk
-  const int soff = kUnitSignBytes + 8 * (int)r;
-  const unsigned psel = 0x03020100u ^ (0x01010101u * (r & 3u));  // its bytes back to column order
-  unsigned sg[2][SB];
-  u32x2 sc[SB];
-  auto load_signs = [&](int t, int h, int g) {
-    const int uo = t * kUnitBytes;
-#pragma unroll
-    for (int sb = 0; sb < SB; ++sb)
-      sg[g][sb] = __builtin_amdgcn_raw_buffer_load_b32(
-          wr, woff, (sb < 4 ? u0 : u1) + uo + (int)(1024u * ((2u * h + g) ^ (sb & 3u)) + 256u * (sb & 3)), 0);
-  };
-  auto load_scales = [&](int t) {
-#pragma unroll
-    for (int sb = 0; sb < SB; ++sb)
-      sc[sb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, soff, (sb < 4 ? u0 : u1) + t * kUnitBytes + 128 * (sb & 3), 0));
-  };
-  unsigned exv[NB], exn[NB];
-  auto load_ex = [&](int t, unsigned (&o)[NB]) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) o[nb] = x.ex[((size_t)(tg * NB + nb) * ntiles + t) * 64 + lane];
-  };
-  f32x4 acc[NB][SB];
-#pragma unroll
-  for (int sb = 0; sb < SB; ++sb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc[nb][sb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  stage(2 * t0, 0);
-  load_signs(t0, 0, 0);
-  load_signs(t0, 0, 1);
-  load_ex(t0, exv);
-  if (tid < kWideTok) {  // 1/rms of the tokens, from the tiles' sums of squares
-    float inv = 1.0f;
-    if (x.ssq) inv = 1.0f / sqrtf(ordered_sum(x.ssq + tg * kWideTok + tid, x.Np, ntiles) / (float)x.K + x.eps);
-    tok_inv[tid] = inv;
-  }
-  lds_dma_wait();
-  __syncthreads();
-  for (int t = t0; t < t1; ++t) {
-    const int tn = min(t + 1, t1 - 1);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int s = 2 * t + h;
-      if (s + 1 < s_end) stage(s + 1, h ^ 1);  // the buffer's last reads ended before the previous barrier
-      // the tile's scales, first used after the first group's matrix instructions
-      if (h == 0) load_scales(t);
-      if (h == 1) load_ex(tn, exn);
-      // the 24 digit operands of the half tile in order (group, token block, digit 5 .. 0), each read one
-      // ahead of the eight matrix instructions that use it
-      const unsigned char* buf = smem + h * kWideStage;
-      i32x8 a = read_frag(buf + (kDigits - 1) * kFragBytes, lane);
-#pragma unroll
-      for (int g = 0; g < 2; ++g) {
-        i32x8 b[SB];
-        asm volatile("" : "+v"(sg[g][0]), "+v"(sg[g][1]), "+v"(sg[g][2]), "+v"(sg[g][3]), "+v"(sg[g][4]), "+v"(sg[g][5]),
-                     "+v"(sg[g][6]), "+v"(sg[g][7]));  // this group's signs are expanded here, not earlier
-#pragma unroll
-        for (int sb = 0; sb < SB; ++sb) expand_f4(__builtin_amdgcn_perm(sg[g][sb], sg[g][sb], psel), b[sb]);
-        load_signs(h == 0 ? t : tn, h ^ 1, g);  // half a tile ahead, into the registers just read
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          f32x4 d[SB];
-          // digit k's block scales: 5k below digit 0's in every byte (no borrow: digit 0's are >= 25)
-          unsigned sx = exv[nb] - 0x19191919u;
-#pragma unroll
-          for (int k = kDigits - 1; k >= 0; --k) {
-            const int nx = k > 0 ? (nb * 2 + g) * kDigits + k - 1
-                                 : nb + 1 < NB ? ((nb + 1) * 2 + g) * kDigits + kDigits - 1 : (g + 1) * kDigits + kDigits - 1;
-            const i32x8 an = k > 0 || nb + 1 < NB || g == 0 ? read_frag(buf + nx * kFragBytes, lane) : a;
-#pragma unroll
-            for (int sb = 0; sb < SB; ++sb) {
-              const f32x4 c = k == kDigits - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
-              if (h == 0 && g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, (int)sx, 0, 0x7F);
-              else if (h == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, (int)sx, 0, 0x7F);
-              else if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, (int)sx, 0, 0x7F);
-              else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, (int)sx, 0, 0x7F);
-            }
-            a = an;
-            asm("v_add_u32 %0, 0x5050505, %0" : "+v"(sx));  // (opaque: the six values would each take a register)
-            step_fence(d);
-          }
-#pragma unroll
-          for (int sb = 0; sb < SB; ++sb) {
-            const unsigned slot = (2u * h + g) ^ (sb & 3u);  // the scale slot of this group
-            const unsigned two = sc[sb][slot >> 1];
-            const float sf = (float)__builtin_bit_cast(_Float16, (unsigned short)(slot & 1 ? two >> 16 : two & 0xFFFFu));
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[nb][sb][v] = __builtin_fmaf(sf, d[sb][v], acc[nb][sb][v]);
-          }
-          step_fence(acc[nb]);
-        }
+      for (int j = 0; j < 8; ++j) {
+        const float r = __builtin_rintf(v[j]);
+        v[j] = (v[j] - r) * 32.0f;
+        if (j & 1) rb[j >> 1] = r;
+        else ra[j >> 1] = r;
       }
-      lds_dma_wait();
-      __syncthreads();
+      const u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
+      lo = d[0];
+      hi = d[1];
+    }
+    put(k, lo, hi);
+  }
+  return b0;
+}
+
+// Packs the wave's 512 columns of token tok into the LDS tile.
+template <int T>
+__device__ __forceinline__ void few_pack(unsigned char* tile, float* st, unsigned lane, int tok, float4 x0, float4 x1) {
+  using FF = FewForm<T>;
+  const unsigned g = lane >> 4, q = (lane >> 2) & 3u, kq = lane & 3u;
+  unsigned char* o = tile + g * FF::kGrp + q * FF::kBlk + 6 * kq;
+  const unsigned b0 = few_digits<T>(st, lane, x0, x1, [&](int k, unsigned lo, unsigned hi) {
+    unsigned short* w = reinterpret_cast<unsigned short*>(o + (k / FF::P) * FF::kOp + 24 * ((k % FF::P) * T + tok));
+    w[0] = (unsigned short)lo;
+    w[1] = (unsigned short)(lo >> 16);
+    w[2] = (unsigned short)hi;
+  });
+  if (kq == 0) {
+#pragma unroll
+    for (int p = 0; p < FF::P; ++p) tile[FF::kEx + 4 * (16 * q + p * T + tok) + g] = (unsigned char)(b0 - 5 * p);
+  }
+}
+
+// The same into a tile in global memory (layout FewForm<T>), for kernels that hand their results to a product:
+// rec is FF::F·FF::P·384 bytes of the wave's LDS, from which the 24-byte pieces go out as 8-byte words.
+template <int T>
+__host__ __device__ constexpr int few_rec() { return FewForm<T>::F * FewForm<T>::P * 384; }
+template <int T>
+__device__ __forceinline__ void few_pack_out(uint8_t* __restrict__ tile, unsigned char* rec, float* st, unsigned lane, int tok,
+                                             float4 x0, float4 x1) {
+  using FF = FewForm<T>;
+  constexpr int W = FF::F * FF::P * 48;  // 8-byte words
+  const unsigned b0 = few_digits<T>(st, lane, x0, x1, [&](int k, unsigned lo, unsigned hi) {
+    unsigned short* w = reinterpret_cast<unsigned short*>(rec + 384 * k + 6 * lane);  // [digit][block][24 B]
+    w[0] = (unsigned short)lo;
+    w[1] = (unsigned short)(lo >> 16);
+    w[2] = (unsigned short)hi;
+  });
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < (W + 63) / 64; ++i) {
+    const int w = 64 * i + (int)lane;
+    if (W % 64 == 0 || w < W) {
+      const int k = w / 48, blk = (w % 48) / 3, part = w % 3;
+      *reinterpret_cast<u32x2*>(tile + (blk >> 2) * FF::kGrp + (k / FF::P) * FF::kOp + (blk & 3) * FF::kBlk +
+                                24 * ((k % FF::P) * T + tok) + 8 * part) = *reinterpret_cast<const u32x2*>(rec + 8 * w);
+    }
+  }
+  if ((lane & 3u) == 0) {
+#pragma unroll
+    for (int p = 0; p < FF::P; ++p)
+      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - 5 * p);
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
+// A unit's weights in a wave: the signs of (16-row block sb, group g) and the rows' four scales.
+struct FewUnit {
+  unsigned s[4][4];  // [g][sb]
+  u32x2 sc[4];
+};
+__device__ __forceinline__ void few_load(const __amdgpu_buffer_rsrc_t& wr, int woff, int soff, int unit, FewUnit& u) {
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+      u.s[g][sb] = __builtin_amdgcn_raw_buffer_load_b32(wr, woff, unit + 1024 * (g ^ sb) + 256 * sb, 0);
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb)
+    u.sc[sb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, soff, unit + 128 * sb, 0));
+}
+
+// acc[sb] += the unit's products with the tile's digits: slot rows 4q + i of weight row 16·sb + r.
+template <int T>
+__device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lane, unsigned psel, const FewUnit& u, f32x4 (&acc)[4]) {
+  using FF = FewForm<T>;
+  const unsigned ex = *reinterpret_cast<const unsigned*>(tile + FF::kEx + 4 * lane);
+  const unsigned char* fl = tile + (lane >> 4) * FF::kBlk + 24 * (lane & 15u);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    i32x8 b[4];
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) expand_f4(__builtin_amdgcn_perm(u.s[g][sb], u.s[g][sb], psel), b[sb]);
+    f32x4 d[4];
+#pragma unroll
+    for (int f = FF::F - 1; f >= 0; --f) {
+      const u32x2* p = reinterpret_cast<const u32x2*>(fl + g * FF::kGrp + f * FF::kOp);
+      const u32x2 p0 = p[0], p1 = p[1], p2 = p[2];
+      const i32x8 a = {(int)p0.x, (int)p0.y, (int)p1.x, (int)p1.y, (int)p2.x, (int)p2.y, 0, 0};
+      const int sx = (int)(ex - 0x05050505u * (unsigned)(f * FF::P));
+#pragma unroll
+      for (int sb = 0; sb < 4; ++sb) {
+        const f32x4 c = f == FF::F - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
+        if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, 0x7F);
+        else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, 0x7F);
+        else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, 0x7F);
+        else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, 0x7F);
+      }
     }
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) exv[nb] = exn[nb];
-  }
-  // lane (r, q): weight row 16·sb + r, tokens 16·nb + 4q .. +3
+    for (int sb = 0; sb < 4; ++sb) {
+      const unsigned slot = (unsigned)(g ^ sb), two = u.sc[sb][slot >> 1];
+      const float sf = (float)__builtin_bit_cast(_Float16, (unsigned short)(slot & 1 ? two >> 16 : two & 0xFFFFu));
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+      for (int v = 0; v < 4; ++v) acc[sb][v] = __builtin_fmaf(sf, d[sb][v], acc[sb][v]);
+    }
+  }
+}
+
+// Adds a weight row's slots: afterwards lane (r, q), register i holds token (4q + i) mod T of row r (T < 4:
+// registers 0 and 1 of every lane the two tokens).
+template <int T>
+__device__ __forceinline__ void few_slots(f32x4& a) {
+  if constexpr (T == 2) {
+    a[0] += a[2];
+    a[1] += a[3];
+    a[0] += __shfl_xor(a[0], 16);
+    a[1] += __shfl_xor(a[1], 16);
+    a[0] += __shfl_xor(a[0], 32);
+    a[1] += __shfl_xor(a[1], 32);
+  } else if constexpr (T == 4) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int tl = 16 * nb + 4 * (int)q + v, n = tg * kWideTok + tl;
-      if (n >= n_tok) continue;
-      const float inv = tok_inv[tl];
-      float* yr = y + (size_t)n * ldy;
-#pragma unroll
-      for (int sb = 0; sb < SB; ++sb) {
-        const int64_t row = (rb0 + (sb >> 2)) * kRowBlock + 16 * (sb & 3) + r;
-        if (row < rows) {
-          const float val = acc[nb][sb][v] * inv;
-          yr[row] = accumulate ? yr[row] + val : val;
-        }
-      }
+      a[v] += __shfl_xor(a[v], 16);
+      a[v] += __shfl_xor(a[v], 32);
     }
+  } else if constexpr (T == 8) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) a[v] += __shfl_xor(a[v], 32);
+  }
+}
+
+// Activations of the few-column product: x[n][K] f32 with row stride ldx.
+struct FewX {
+  const float* xf;
+  int64_t ldx, K;
+  const uint8_t* dig;  // PRE: packed tiles [ntiles][FewForm<T>::kTile] instead (x, nw and ssq unused)
+  // with RMSNorm (rmsnorm_into, rmsnorm.rs:17-200): the digits are those of x·nw, and y = inv · W (x·nw) with
+  // inv = 1/sqrt(Σx²/K + eps): applied by the kernel when its workgroups see every tile, else by the consumer
+  // of the split partials, from the per-split sums of squares ssq[z][ssq_ld] that the first row chunk's
+  // workgroups write
+  const float* nw;
+  float* ssq;
+  int ssq_ld;
+  float eps;
+};
+template <int T>
+__host__ __device__ constexpr size_t few_shmem(int nw, int tps) {
+  return (size_t)tps * FewForm<T>::kTile + (size_t)nw * kFewStage;
+}
+// K tiles of a workgroup (its LDS)
+constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
+
+// Grid (ceil(nrb / NW), splits), 64·NW threads: workgroup (chunk, z) takes K tiles [z·tps, min(ntiles, (z+1)·tps))
+// of NW row-blocks, one per wave.  The inputs are requested first, the first unit's weights behind them, and the
+// packing runs while the weights arrive; one barrier, then every wave goes its own way.  With more than one
+// split, workgroup z writes its partial to y + z·zstride.
+// At eight tokens a product is bound by latencies: of 34816 x 5120's 15.2 us (packed tiles) about 7 are launch, digits
+// and the stores of the partials, 5 the weights (25 MB) and 3 the signs' expansion and the matrix instructions.  The
+// f16 form it replaced (three parts, K tiles packed one by one with a barrier each) against this one with packed
+// tiles, us per launch in the verify forward: 34816 x 5120 22.7 -> 15.9, 16480 x 5120 15.7 -> 11.7, 5120 x 17408
+// 14.2 -> 11.3, 5120 x 6144 7.5 -> 6.6.
+//
+// PRE: the digits come packed by the kernel that formed the activations: at eight tokens the packing costs 2 to
+// 4 us of each product.
+template <int T, int NW, bool PRE>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
+                                                                     int ntiles, int tps, const FewX x, int n_tok,
+                                                                     float* __restrict__ y, int64_t ldy, int64_t zstride,
+                                                                     int accumulate) {
+  using FF = FewForm<T>;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ float ssqs[few_max_tiles(T)][T];
+  const unsigned tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
+  const int wave = (int)__builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t0 = (int)blockIdx.y * tps, nt = min(ntiles - t0, tps);
+  const int64_t rb = (int64_t)blockIdx.x * NW + wave;
+  float* st = reinterpret_cast<float*>(smem + (size_t)tps * FF::kTile) + wave * (kFewStage / 4);
+  // packing task i of the wave: (token, tile) number wave + NW·i, tokens first.  The first MT tasks' inputs are
+  // requested before any weights: the CU returns loads in issue order
+  constexpr int MT = 2;
+  const int tasks = n_tok * nt;
+  struct In {
+    float4 x0, x1, w0, w1;
+  };
+  auto load_x = [&](int k) {  // (a task past the last reloads it)
+    const int kc = min(k, tasks - 1), tok = kc % n_tok;
+    const int64_t c0 = (int64_t)(t0 + kc / n_tok) * kTileCols + 4 * lane, c1 = c0 + 256;
+    // K is a multiple of 128, so a float4 is wholly in or out; past it, column 0 is read and dropped
+    const bool i0 = c0 < x.K, i1 = c1 < x.K;
+    const float* p = x.xf + (size_t)tok * x.ldx;
+    In v;
+    v.x0 = *reinterpret_cast<const float4*>(p + (i0 ? c0 : 0));
+    v.x1 = *reinterpret_cast<const float4*>(p + (i1 ? c1 : 0));
+    if (x.nw) {
+      v.w0 = *reinterpret_cast<const float4*>(x.nw + (i0 ? c0 : 0));
+      v.w1 = *reinterpret_cast<const float4*>(x.nw + (i1 ? c1 : 0));
+    }
+    return v;
+  };
+  In in[MT];
+  // PRE: the tiles as 16-byte pieces, the first MP per thread requested before the weights
+  constexpr int MP = PRE ? (NW == 8 ? 8 : 10) : 1;
+  u32x4 pc[MP];
+  const int pieces = nt * (FF::kTile / 16);
+  const u32x4* psrc = reinterpret_cast<const u32x4*>(PRE ? x.dig + (size_t)t0 * FF::kTile : nullptr);
+  if constexpr (PRE) {
+#pragma unroll
+    for (int i = 0; i < MP; ++i) pc[i] = psrc[min((int)tid + 64 * NW * i, pieces - 1)];
+  } else {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) in[i] = load_x(wave + NW * i);
+  }
+  const size_t wbytes = (size_t)(nrb - (int64_t)blockIdx.x * NW) * ntiles * kUnitBytes;
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(W) + (size_t)blockIdx.x * NW * ntiles * kUnitBytes, 0, (int)(wbytes < 0x7FFFFFFFu ? wbytes : 0x7FFFFFFFu), 0x00027000);
+  const int woff = (int)(16u * r + 4u * (q ^ (r >> 2))), soff = kUnitSignBytes + 8 * (int)r;
+  const unsigned psel = 0x03020100u ^ (0x01010101u * (r & 3u));
+  const int unit0 = (wave * ntiles + t0) * kUnitBytes;
+  FewUnit u;
+  if (rb < nrb) few_load(wr, woff, soff, unit0, u);
+  auto pack = [&](int k, const In& v) {
+    if (k >= tasks) return;  // wave-uniform
+    const int tok = k % n_tok, t = k / n_tok;
+    const int64_t c0 = (int64_t)(t0 + t) * kTileCols + 4 * lane;
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 x0 = c0 < x.K ? v.x0 : z, x1 = c0 + 256 < x.K ? v.x1 : z;
+    if (x.nw) {
+      const float s = wave_sum(((x0.x * x0.x + x0.y * x0.y) + (x0.z * x0.z + x0.w * x0.w)) +
+                               ((x1.x * x1.x + x1.y * x1.y) + (x1.z * x1.z + x1.w * x1.w)));
+      if (lane == 0) ssqs[t][tok] = s;
+      x0 = make_float4(x0.x * v.w0.x, x0.y * v.w0.y, x0.z * v.w0.z, x0.w * v.w0.w);
+      x1 = make_float4(x1.x * v.w1.x, x1.y * v.w1.y, x1.z * v.w1.z, x1.w * v.w1.w);
+    }
+    few_pack<T>(smem + (size_t)t * FF::kTile, st, lane, tok, x0, x1);
+  };
+  if constexpr (PRE) {
+    u32x4* dst = reinterpret_cast<u32x4*>(smem);
+#pragma unroll
+    for (int i = 0; i < MP; ++i)
+      if ((int)tid + 64 * NW * i < pieces) dst[tid + 64 * NW * i] = pc[i];
+    for (int i = (int)tid + 64 * NW * MP; i < pieces; i += 64 * NW) dst[i] = psrc[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) pack(wave + NW * i, in[i]);
+    for (int k = wave + NW * MT; k < tasks; k += NW) pack(k, load_x(k));
+  }
+  lds_barrier();  // the weights stay in flight
+  if (!PRE && x.nw && gridDim.y > 1 && blockIdx.x == 0 && tid < (unsigned)n_tok) {
+    float s = ssqs[0][tid];
+    for (int t = 1; t < nt; ++t) s += ssqs[t][tid];
+    x.ssq[(size_t)blockIdx.y * x.ssq_ld + tid] = s;
+  }
+  if (rb >= nrb) return;
+  f32x4 acc[4];
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) acc[sb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < nt; ++t) {
+    FewUnit nx = u;
+    if (t + 1 < nt) few_load(wr, woff, soff, unit0 + (t + 1) * kUnitBytes, nx);
+    few_unit<T>(smem + (size_t)t * FF::kTile, lane, psel, u, acc);
+    u = nx;
+  }
+  y += (size_t)blockIdx.y * zstride;
+  if (gridDim.y > 1) accumulate = 0;
+#pragma unroll
+  for (int sb = 0; sb < 4; ++sb) few_slots<T>(acc[sb]);
+#pragma unroll
+  for (int v = 0; v < (T == 2 ? 2 : 4); ++v) {
+    const int tok = T == 2 ? v : (4 * (int)q + v) % T;
+    if (tok >= n_tok || (T == 2 && q) || (T == 4 && q) || (T == 8 && q > 1)) continue;
+    float inv = 1.0f;
+    if (!PRE && x.nw && gridDim.y == 1) {
+      float s = ssqs[0][tok];
+      for (int t = 1; t < nt; ++t) s += ssqs[t][tok];
+      inv = 1.0f / sqrtf(s / (float)x.K + x.eps);
+    }
+    float* yr = y + (size_t)tok * ldy + rb * kRowBlock + r;
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb)
+      if (rb * kRowBlock + 16 * sb + r < rows) {
+        const float val = acc[sb][v] * inv;
+        yr[16 * sb] = accumulate ? yr[16 * sb] + val : val;
+      }
+  }
 }
 
 }  // namespace dz

@@ -2,8 +2,7 @@
 // C ABI (Q1_0Matrix::{from_gguf, row_into_slice, matvec_into_slice, matvec_add_into_slice,
 // matvec_multi_into_slice}, Daiza-engine/src/model/weights.rs:83-972).
 #include "runtime.h"
-#include "q1_digits.h"
-#include "q1_gemm.h"
+#include "q1_wide.h"
 
 #include <cstdarg>
 #include <cstdio>
@@ -315,19 +314,6 @@ static int wide_splits(const Q1Dev& W, int n, int* tps) {
   return best;
 }
 
-// Workgroups wanted in flight (two per CU): a product with fewer splits its K tiles over
-// blockIdx.z and sums the partials in a second pass.
-constexpr int kGemmMinWgs = 512;
-
-static int gemm_splits(const Q1Dev& W, int* tps) {
-  const int64_t wgs = (W.nrb + 3) / 4;
-  const int nt = (int)W.ntiles;
-  int S = 1;
-  if (wgs < kGemmMinWgs && nt > 1) S = (int)std::min<int64_t>(nt, (kGemmMinWgs + wgs - 1) / wgs);
-  *tps = (nt + S - 1) / S;
-  return (nt + *tps - 1) / *tps;
-}
-
 hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int64_t ldy, int accumulate,
                           hipStream_t s, Scratch* split, GemmDefer* defer) {
   static bool attr = false;
@@ -354,10 +340,97 @@ hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int
   hipLaunchKernelGGL(q1_wide_kernel, dim3((unsigned)(g.nrg * g.ntg * S)), dim3(256), kWideShmem, s, W.data, W.rows, W.nrb,
                      (int)W.ntiles, g, dx, n, out, ld, zs, S > 1 ? 0 : accumulate);
   hipError_t e = hipGetLastError();
-  if (defer) *defer = GemmDefer{out, S, zs, nullptr, 0, W.cols, 0.f};
+  if (defer) *defer = GemmDefer{out, S, zs, nullptr, 0, 0, W.cols, 0.f};
   if (e != hipSuccess || S == 1 || defer) return e;
   hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((W.rows + 255) / 256), (unsigned)n), dim3(256), 0, s,
-                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, (const float*)nullptr, 0, W.cols, 0.f);
+                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, (const float*)nullptr, 0, 0, W.cols, 0.f);
+  return hipGetLastError();
+}
+
+// Launch shape of the few-column product: K tiles per workgroup (so splits) and waves per workgroup.
+struct FewPlan {
+  int nw, tps, splits;
+  unsigned chunks;
+};
+
+// A wave takes one row-block of the workgroup's K tiles, one unit after another, so a product wants its units
+// spread over enough waves (about kFewWaves) and no more splits than that takes: each split adds a pass over
+// partials.  Workgroups that pack their tiles themselves share that over eight waves, unless half of the CUs would
+// be left without one (at eight tokens 16480 x 5120 16.9 against 13.1 us, 5120 x 6144 7.6 against 8.0); with packed
+// tiles four waves spread better (16480 x 5120 9.5 against 10.5, 5120 x 17408 8.9 against 10.0).
+constexpr int kFewWaves = 2048;
+static FewPlan few_plan(const Q1Dev& W, int T, bool pre) {
+  FewPlan p;
+  const int nt = (int)W.ntiles;
+  const int64_t want = std::max<int64_t>(1, (kFewWaves + W.nrb - 1) / W.nrb);  // splits
+  p.tps = (int)std::max<int64_t>(1, (nt + want - 1) / want);
+  p.tps = std::min(p.tps, few_max_tiles(T));
+  p.splits = (nt + p.tps - 1) / p.tps;
+  p.nw = !pre && 2 * ((W.nrb + 7) / 8 * p.splits) >= device_cus() ? 8 : 4;
+  p.chunks = (unsigned)((W.nrb + p.nw - 1) / p.nw);
+  return p;
+}
+static int few_form(int n) { return n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16; }
+
+template <int T, int NW, bool PRE>
+static hipError_t launch_few(const FewPlan& p, const Q1Dev& W, const FewX& x, int n, float* y, int64_t ldy, int64_t zs,
+                             int accumulate, hipStream_t s) {
+  static bool attr = false;
+  if (!attr) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_few_kernel<T, NW, PRE>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)few_shmem<T>(NW, few_max_tiles(T)));
+    if (e != hipSuccess) return e;
+    attr = true;
+  }
+  hipLaunchKernelGGL((q1_few_kernel<T, NW, PRE>), dim3(p.chunks, (unsigned)p.splits), dim3(64 * NW), few_shmem<T>(NW, p.tps), s,
+                     W.data, W.rows, W.nrb, (int)W.ntiles, p.tps, x, n, y, ldy, zs, accumulate);
+  return hipGetLastError();
+}
+
+template <bool PRE>
+static hipError_t launch_few_t(int T, const FewPlan& p, const Q1Dev& W, const FewX& x, int n, float* y, int64_t ldy, int64_t zs,
+                               int accumulate, hipStream_t s) {
+#define DZ_FEW(T_) \
+  return p.nw == 8 ? launch_few<T_, 8, PRE>(p, W, x, n, y, ldy, zs, accumulate, s) : launch_few<T_, 4, PRE>(p, W, x, n, y, ldy, zs, accumulate, s)
+  switch (T) {
+    case 2: DZ_FEW(2);
+    case 4: DZ_FEW(4);
+    case 8: DZ_FEW(8);
+    default: DZ_FEW(16);
+  }
+#undef DZ_FEW
+}
+
+size_t few_tile_bytes(int n) {
+  switch (few_form(n)) {
+    case 2: return FewForm<2>::kTile;
+    case 4: return FewForm<4>::kTile;
+    case 8: return FewForm<8>::kTile;
+    default: return FewForm<16>::kTile;
+  }
+}
+
+hipError_t launch_q1_few_packed(const Q1Dev& W, const uint8_t* dig, const float* ssq, float eps, int n, float* y, int64_t ldy,
+                                int accumulate, hipStream_t s, Scratch* split, GemmDefer* defer) {
+  if (n < 1 || n > 16 || !split) return hipErrorInvalidValue;
+  FewX fx{};
+  fx.dig = dig;
+  fx.K = W.cols;
+  const int T = few_form(n);
+  const FewPlan p = few_plan(W, T, true);
+  const int S = p.splits;
+  const bool direct = S == 1 && !ssq;  // otherwise the sum of the partials (or of the one) applies 1/rms
+  const int64_t zs = (int64_t)n * W.rows;
+  float* out = y;
+  if (!direct) {
+    if (split->reserve((size_t)S * zs * sizeof(float))) return hipErrorOutOfMemory;
+    out = static_cast<float*>(split->ptr);
+  }
+  hipError_t e = launch_few_t<true>(T, p, W, fx, n, out, direct ? ldy : W.rows, zs, direct ? accumulate : 0, s);
+  if (defer) *defer = GemmDefer{out, direct ? 1 : std::max(S, 1), zs, ssq, ssq ? (int)W.ntiles : 0, n, W.cols, eps};
+  if (e != hipSuccess || direct || defer) return e;
+  hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((W.rows + 255) / 256), (unsigned)n), dim3(256), 0, s,
+                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, ssq, (int)W.ntiles, n, W.cols, eps);
   return hipGetLastError();
 }
 
@@ -365,26 +438,16 @@ hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n
                               int accumulate, hipStream_t s, Scratch* split, const float* norm_w, float eps,
                               GemmDefer* defer) {
   if ((W.cols & 3) || (ldx & 3)) return hipErrorInvalidValue;  // 16-byte loads of x rows
-  if (n > 16) return hipErrorInvalidValue;  // one 16-token block per workgroup
-  static bool attr = false;
-  if (!attr) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_gemm_kernel<false>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_shmem(false));
-    if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_gemm_kernel<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_shmem(true));
-    if (e != hipSuccess) return e;
-    attr = true;
-  }
-  GemmX gx{};
-  gx.xf = x;
-  gx.ldx = ldx;
-  gx.K = W.cols;
-  gx.nw = norm_w;
-  gx.eps = eps;
-  int tps;
-  int S = gemm_splits(W, &tps);
-  if (S > 1 && !split) S = 1, tps = (int)W.ntiles;
+  if (n > 16) return hipErrorInvalidValue;
+  FewX fx{};
+  fx.xf = x;
+  fx.ldx = ldx;
+  fx.K = W.cols;
+  fx.nw = norm_w;
+  fx.eps = eps;
+  const int T = few_form(n);
+  const FewPlan p = few_plan(W, T, false);
+  const int S = p.splits;
   float* out = y;
   int64_t ld = ldy, zs = 0;
   if (S > 1) {
@@ -394,23 +457,16 @@ hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n
     out = static_cast<float*>(split->ptr);
     ld = W.rows;
     if (norm_w) {
-      gx.ssq = out + (size_t)S * zs;
-      gx.ssq_ld = n;
+      fx.ssq = out + (size_t)S * zs;
+      fx.ssq_ld = n;
     }
   }
-  const dim3 g((unsigned)((W.nrb + 3) / 4), 1, (unsigned)S);
-  if (n <= 8)  // hi and mid of every token in one operand, lo in a second: two matrix instructions per step
-    hipLaunchKernelGGL(q1_gemm_kernel<true>, g, dim3(64 * kGemmWaves), gemm_shmem(true), s, W.data, W.rows, W.nrb,
-                       (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-  else
-    hipLaunchKernelGGL(q1_gemm_kernel<false>, g, dim3(64 * kGemmWaves), gemm_shmem(false), s, W.data, W.rows, W.nrb,
-                       (int)W.ntiles, tps, gx, n, out, ld, zs, accumulate);
-  hipError_t e = hipGetLastError();
-  const float* ssq = S > 1 && norm_w ? gx.ssq : nullptr;
-  if (defer) *defer = GemmDefer{out, S, zs, ssq, n, W.cols, eps};
+  const hipError_t e = launch_few_t<false>(T, p, W, fx, n, out, ld, zs, accumulate, s);
+  const float* ssq = S > 1 && norm_w ? fx.ssq : nullptr;
+  if (defer) *defer = GemmDefer{out, S, zs, ssq, S, n, W.cols, eps};
   if (e != hipSuccess || S == 1 || defer) return e;
   hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((W.rows + 255) / 256), (unsigned)n), dim3(256), 0, s,
-                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, ssq, n, W.cols, eps);
+                     (const float*)out, S, zs, W.rows, n, y, ldy, accumulate, ssq, S, n, W.cols, eps);
   return hipGetLastError();
 }
 

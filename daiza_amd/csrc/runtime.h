@@ -86,8 +86,9 @@ struct GemmDefer {
   const float* part = nullptr;
   int splits = 1;
   int64_t zstride = 0;
-  // a normed raw product: per-split sums of squares [splits][ssq_ld] (the caller applies 1/rms)
+  // a normed product: sums of squares [ssq_n][ssq_ld] (the caller applies 1/rms)
   const float* ssq = nullptr;
+  int ssq_n = 0;  // rows of ssq (the splits, or the tiles of a packed product)
   int ssq_ld = 0;
   int64_t K = 0;
   float eps = 0.f;
@@ -103,6 +104,13 @@ hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int
 hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n, float* y, int64_t ldy,
                               int accumulate, hipStream_t s, Scratch* split, const float* norm_w = nullptr,
                               float eps = 0.f, GemmDefer* defer = nullptr);
+
+// The few-token product (n <= 16) on digits that the kernel forming its activations has packed: `dig` holds
+// W.ntiles tiles of few_tile_bytes(n).  With ssq (sums of squares [W.ntiles][n] of the unweighted x) the product is
+// that of the RMS-normalised x, 1/rms applied by the sum of the split partials (which it always is then).
+size_t few_tile_bytes(int n);
+hipError_t launch_q1_few_packed(const Q1Dev& W, const uint8_t* dig, const float* ssq, float eps, int n, float* y, int64_t ldy,
+                                int accumulate, hipStream_t s, Scratch* split, GemmDefer* defer = nullptr);
 
 }  // namespace dz
 
