@@ -21,12 +21,22 @@ __device__ __forceinline__ float lane8_sum(float v) {
 // f16_to_f32 (tensor/tensor.rs:62-76), or a Q1_0 table through dequantize_q1_0_row_into
 // (quant.rs:161-194).  Grid (n, ceil(H / 1024)), 256 threads of four columns each: with one workgroup per token
 // the row's twenty dependent rounds took 13 us for eight tokens.
-__global__ __launch_bounds__(256) void bt_embed_kernel(const int* __restrict__ ids, int64_t H,
+struct FewIds {  // up to 16 tokens as a kernel argument (ids keeps them for what follows the forward)
+  int id[16];
+  int n;  // 0: the ids are in memory
+};
+__global__ __launch_bounds__(256) void bt_embed_kernel(int* __restrict__ ids, const FewIds fi, int64_t H,
                                                        const uint16_t* __restrict__ emb_f16,
                                                        const uint8_t* __restrict__ emb_q1, int emb_ntiles,
                                                        float* __restrict__ h) {
   const int t = blockIdx.x;
-  const int tok = ids[t];
+  int tok;
+  if (fi.n) {
+    tok = fi.id[t];
+    if (blockIdx.y == 0 && threadIdx.x == 0) ids[t] = tok;
+  } else {
+    tok = ids[t];
+  }
   const int64_t k0 = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 4;  // H is a multiple of 128
   if (k0 >= H) return;
   float o[4];
@@ -574,16 +584,42 @@ __global__ __launch_bounds__(64) void bt_chunk_scan_kernel(const float* __restri
   for (int J = 0; J < 8; ++J) *reinterpret_cast<f32x4*>(Sp + 16 * J) = S[J];
 }
 
-// Applies the first a recorded tokens of a verify chunk to the state: s = decay·s, s = fma(d, k, s)
-// per token, the same operations in the same order as the scan, so the result equals a scan over
-// those a tokens.  Grid 4·nvh, 256 threads (the scan's row mapping).
-__global__ __launch_bounds__(256) void bt_commit_state_kernel(float* __restrict__ state, DnRecord rec, int a, int nkh,
-                                                              int nvh) {
+// Rollback records and conv inputs of a verify chunk, every DeltaNet layer's one after another.
+struct DnRecords {
+  float* decay;  // [layer][cap][nvh]
+  float* d;      // [layer][cap][nvh * 128]
+  float* k;      // [layer][cap][nkh * 128]
+  float* x;      // [layer][cap][qkvd]
+  int cap;       // tokens per layer
+  __host__ __device__ DnRecord layer(int si, int nkh, int nvh) const {
+    const size_t c = (size_t)si * cap;
+    return DnRecord{decay + c * nvh, d + c * nvh * 128, k + c * nkh * 128};
+  }
+  __host__ __device__ float* conv(int si, int64_t qkvd) const { return x + (size_t)si * cap * qkvd; }
+};
+
+// Keeps the first a recorded tokens of a verify chunk in every DeltaNet layer (blockIdx.y).  Workgroups
+// [0, 4·nvh) apply them to the state: s = decay·s, s = fma(d, k, s) per token, the same operations in the same
+// order as the scan (and its row mapping), so the result equals a scan over those a tokens; the others
+// write the last four tokens' conv inputs to the ring (bt_ring_kernel; head0 = slot of the chunk's first token).
+__global__ __launch_bounds__(256) void bt_commit_kernel(float* __restrict__ state, float* __restrict__ conv,
+                                                        const int* __restrict__ ring_base, int p0, DnRecords recs, int a,
+                                                        int nkh, int nvh, int64_t qkvd) {
   constexpr int HD = 128;
   const unsigned tid = threadIdx.x;
+  const int si = blockIdx.y;
+  if ((int)blockIdx.x >= 4 * nvh) {
+    const int64_t ch = (int64_t)((int)blockIdx.x - 4 * nvh) * 256 + tid;
+    if (ch >= qkvd) return;
+    const int head0 = (ring_base[si] + p0) & 3;
+    const float* xin = recs.conv(si, qkvd);
+    for (int t = max(0, a - 4); t < a; ++t) conv[((size_t)si * 4 + ((head0 + t) & 3)) * qkvd + ch] = xin[(size_t)t * qkvd + ch];
+    return;
+  }
+  const DnRecord rec = recs.layer(si, nkh, nvh);
   const int vh = blockIdx.x >> 2, quarter = blockIdx.x & 3, kh = vh % nkh;
   const int i = quarter * 32 + (int)(tid >> 3), js = (int)(tid & 7u);
-  float* S = state + (size_t)vh * HD * HD + (size_t)i * HD + 16 * js;
+  float* S = state + ((size_t)si * nvh + vh) * HD * HD + (size_t)i * HD + 16 * js;
   float s[16];
   state_row_load(S, s);
   for (int t = 0; t < a; ++t) {
@@ -596,6 +632,27 @@ __global__ __launch_bounds__(256) void bt_commit_state_kernel(float* __restrict_
     for (int jj = 0; jj < 16; ++jj) s[jj] = __builtin_fmaf(d, kr[jj], s[jj]);
   }
   state_row_store(S, s);
+}
+
+// After a forward of tokens [0, n) at position p0 that is kept: the token log, TokState and the context's logits
+// (the last kept token's row), as forward_single_token leaves them.  Grid ceil(vocab / 1024), 256 threads.
+__global__ __launch_bounds__(256) void bt_finish_kernel(const int* __restrict__ ids, int n, int p0, int* __restrict__ toklog,
+                                                        TokState* __restrict__ st, const float* __restrict__ src,
+                                                        float* __restrict__ logits, int vocab) {
+  if (blockIdx.x == 0) {
+    for (int t = (int)threadIdx.x; t < n; t += 256) toklog[p0 + t] = ids[t];
+    if (threadIdx.x == 0) *st = TokState{p0 + n - 1, ids[n - 1], 0, 0, p0 + n, {0, 0, 0}};
+  }
+  const int c = (int)blockIdx.x * 1024 + (int)threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (c + 256 * k < vocab) logits[c + 256 * k] = src[c + 256 * k];
+}
+
+// TokState's next position, and the ring bases shifted with it (ring heads are kept relative to the position).
+__global__ __launch_bounds__(64) void set_pos_kernel(TokState* st, int pos, int* ring_base, int n, int shift) {
+  if (threadIdx.x == 0) st->pos_next = pos;
+  for (int i = (int)threadIdx.x; i < n; i += 64) ring_base[i] = (ring_base[i] + shift) & 3;
 }
 
 // Output gate per v-head (ssm_output_gate_avx2, ssm.rs:246-286):

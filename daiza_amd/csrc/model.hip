@@ -104,10 +104,8 @@ struct dz_ctx {
     dz::Scratch pack, split, arec, spec, chunk, dig;
     // verify records per DeltaNet layer: conv inputs [kv][qkvd] and the scan's rollback record
     int kv_cap = 0;
-    std::vector<float*> rx;
-    std::vector<dz::DnRecord> rec;
-    int pending = 0;          // tokens of the last verify forward (0: none)
-    std::vector<uint32_t> pending_ids;
+    dz::DnRecords recs{};
+    int pending = 0;          // tokens of the last verify forward (0: none); their ids are in `ids`
   } bt;
   std::vector<void*> allocs;
 };
@@ -795,18 +793,17 @@ static int ctx_peek_argmax(dz_ctx* x) {
   return DZ_OK;
 }
 
-static int ctx_set_pos_dev(dz_ctx* x, int pos);
-
 // Moves the position to pos while every DeltaNet layer's conv-ring head stays where it is: heads are
 // stored relative to the position ((ring_base + pos) & 3), so each base is rebased by the move.
 // SsmState::conv_head (cache/ssm_state.rs:10-39) is independent of the KV length, and neither
 // KvCache::truncate (kv_cache.rs:119-130) nor a position change touches it.
 static int ctx_move_pos(dz_ctx* x, int pos) {
-  const int old = x->pos_host;
-  for (size_t i = 0; i < x->ring_base.size(); ++i) x->ring_base[i] = ((x->ring_base[i] + old - pos) % 4 + 4) % 4;
-  if (!x->ring_base.empty())
-    DZ_HIP_CHECK(hipMemcpy(x->ring_base_dev, x->ring_base.data(), x->ring_base.size() * 4, hipMemcpyHostToDevice));
-  return ctx_set_pos_dev(x, pos);
+  const int shift = ((x->pos_host - pos) % 4 + 4) % 4;
+  for (int& b : x->ring_base) b = (b + shift) & 3;
+  hipLaunchKernelGGL(set_pos_kernel, dim3(1), dim3(64), 0, x->s, x->st, pos, x->ring_base_dev, x->m->n_ssm, shift);
+  DZ_HIP_CHECK(hipGetLastError());
+  x->pos_host = pos;
+  return DZ_OK;
 }
 
 // Refuses work on a context whose last token-kernel launch gave up part-way.
@@ -1250,8 +1247,6 @@ static void bt_release(dz_ctx* x) {
   x->bt.cap = 0;
   x->bt.kv_cap = 0;
   x->bt.logits_rows = 0;
-  x->bt.rx.clear();
-  x->bt.rec.clear();
   if (x->bt.pack.ptr) (void)hipFree(x->bt.pack.ptr);
   if (x->bt.split.ptr) (void)hipFree(x->bt.split.ptr);
   if (x->bt.arec.ptr) (void)hipFree(x->bt.arec.ptr);
@@ -1277,8 +1272,6 @@ static int bt_reserve(dz_ctx* x, int cap) {
   x->bt.cap = 0;
   x->bt.kv_cap = 0;
   x->bt.logits_rows = 0;
-  x->bt.rx.clear();
-  x->bt.rec.clear();
   const int64_t hd = c.ssm_state, kdim = (int64_t)c.ssm_k_heads * hd, inner = (int64_t)c.ssm_v_heads * hd;
   const int64_t qkvd = 2 * kdim + inner, qd = (int64_t)c.n_head * c.head_dim;
   int64_t rows_in = 1;
@@ -1312,16 +1305,14 @@ static int bt_reserve_verify(dz_ctx* x, int k) {
   const dz_config& c = x->m->cfg;
   const int64_t hd = c.ssm_state, kdim = (int64_t)c.ssm_k_heads * hd, inner = (int64_t)c.ssm_v_heads * hd;
   const int64_t qkvd = 2 * kdim + inner;
-  x->bt.rx.assign((size_t)x->m->n_ssm, nullptr);
-  x->bt.rec.assign((size_t)x->m->n_ssm, DnRecord{nullptr, nullptr, nullptr});
+  DnRecords& r = x->bt.recs;
+  const size_t lk = (size_t)x->m->n_ssm * k;
   auto& A = x->bt.allocs;
   int rc;
-  for (int i = 0; i < x->m->n_ssm; ++i) {
-    DnRecord& r = x->bt.rec[(size_t)i];
-    if ((rc = alloc_t(A, &x->bt.rx[(size_t)i], (size_t)k * qkvd)) || (rc = alloc_t(A, &r.decay, (size_t)k * c.ssm_v_heads)) ||
-        (rc = alloc_t(A, &r.d, (size_t)k * inner)) || (rc = alloc_t(A, &r.k, (size_t)k * kdim)))
-      return rc;
-  }
+  if ((rc = alloc_t(A, &r.x, lk * qkvd)) || (rc = alloc_t(A, &r.decay, lk * c.ssm_v_heads)) || (rc = alloc_t(A, &r.d, lk * inner)) ||
+      (rc = alloc_t(A, &r.k, lk * kdim)))
+    return rc;
+  r.cap = k;
   x->bt.kv_cap = k;
   return DZ_OK;
 }
@@ -1433,14 +1424,20 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
   if (verify && (rc = bt_reserve_verify(x, n))) return rc;
   for (int i = 0; i < n; ++i)
     if (ids[i] >= (uint32_t)c.vocab) return set_error(DZ_ERR_TENSOR, "token id %u >= vocab %d", ids[i], c.vocab);
-  DZ_HIP_CHECK(hipMemcpyAsync(x->bt.ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
+  FewIds fi{};
+  if (n <= 16) {
+    fi.n = n;
+    for (int i = 0; i < n; ++i) fi.id[i] = (int)ids[i];
+  } else {
+    DZ_HIP_CHECK(hipMemcpyAsync(x->bt.ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, s));
+  }
   const int p0 = x->pos_host;
   const int64_t H = c.hidden, hd = c.ssm_state, F = c.ffn;
   const int64_t kdim = (int64_t)c.ssm_k_heads * hd, inner = (int64_t)c.ssm_v_heads * hd, qkvd = 2 * kdim + inner;
   const int64_t qd = (int64_t)c.n_head * c.head_dim;
   const size_t kvsz = (size_t)c.n_head_kv * c.max_ctx * c.head_dim;
   const unsigned nb = (unsigned)n;
-  DZ_HIP_CHECK(launch(bt_embed_kernel, dim3(nb, (unsigned)((H + 1023) / 1024)), dim3(256), s, (const int*)x->bt.ids, H, (const uint16_t*)m->emb_f16,
+  DZ_HIP_CHECK(launch(bt_embed_kernel, dim3(nb, (unsigned)((H + 1023) / 1024)), dim3(256), s, x->bt.ids, fi, H, (const uint16_t*)m->emb_f16,
                       (const uint8_t*)m->emb_q1.data, (int)m->emb_q1.ntiles, x->bt.h));
   // few tokens (verify, short batches): every kernel that forms a product's activations packs them
   const bool few = n <= 16;
@@ -1469,10 +1466,10 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
       // (conv, SiLU and the q/k L2 norms in one launch)
       DZ_HIP_CHECK(launch(bt_conv_kernel, dim3(gch, nb), dim3(256), s, (const float*)x->bt.yin, ld_in, n,
                           (const float*)ring, head0, (const float*)l.conv_w, qkvd, x->bt.cout,
-                          verify ? x->bt.rx[(size_t)si] : nullptr, (int)c.ssm_k_heads, x->bt.qk));
+                          verify ? x->bt.recs.conv(si, qkvd) : (float*)nullptr, (int)c.ssm_k_heads, x->bt.qk));
       DnRecord rec{nullptr, nullptr, nullptr};
       if (verify) {
-        rec = x->bt.rec[(size_t)si];
+        rec = x->bt.recs.layer(si, (int)c.ssm_k_heads, (int)c.ssm_v_heads);
       } else {
         DZ_HIP_CHECK(launch(bt_ring_kernel, dim3(gch), dim3(256), s, (const float*)x->bt.yin, ld_in, std::max(0, n - 4),
                             n, ring, head0, qkvd));
@@ -1563,20 +1560,12 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
   return DZ_OK;
 }
 
-// After a forward of n tokens ids at p0 that is kept: the token log, TokState and the context's
-// logits (the last token's row of bt.logits, row `last_row`) as forward_single_token leaves them.
-static int bt_finish(dz_ctx* x, const uint32_t* ids, int n, int p0, int last_row) {
+// After a forward of n tokens (their ids in bt.ids) at p0 that is kept: the token log, TokState and the context's
+// logits (row `last_row` of bt.logits) as forward_single_token leaves them.  Enqueued; the caller waits.
+static int bt_finish(dz_ctx* x, int n, int p0, int last_row) {
   const dz_config& c = x->m->cfg;
-  DZ_HIP_CHECK(hipMemcpyAsync(x->toklog + p0, ids, (size_t)n * 4, hipMemcpyHostToDevice, x->s));
-  TokState st;
-  memset(&st, 0, sizeof st);
-  st.pos = p0 + n - 1;
-  st.token = (int)ids[n - 1];
-  st.pos_next = p0 + n;
-  DZ_HIP_CHECK(hipMemcpyAsync(x->st, &st, sizeof st, hipMemcpyHostToDevice, x->s));
-  DZ_HIP_CHECK(hipMemcpyAsync(x->logits, x->bt.logits + (size_t)last_row * c.vocab, (size_t)c.vocab * 4,
-                              hipMemcpyDeviceToDevice, x->s));
-  DZ_HIP_CHECK(hipStreamSynchronize(x->s));  // the host copies above read caller memory
+  DZ_HIP_CHECK(launch(bt_finish_kernel, dim3((unsigned)((c.vocab + 1023) / 1024)), dim3(256), x->s, (const int*)x->bt.ids, n,
+                      p0, x->toklog, x->st, (const float*)(x->bt.logits + (size_t)last_row * c.vocab), x->logits, (int)c.vocab));
   x->pos_host = p0 + n;
   return DZ_OK;
 }
@@ -1589,7 +1578,6 @@ static int bt_verify_forward(dz_ctx* x, const uint32_t* draft, int k) {
   x->bt.pending = 0;
   int rc = bt_forward(x, draft, k, k, true);
   if (rc) return rc;
-  x->bt.pending_ids.assign(draft, draft + k);
   x->bt.pending = k;
   return DZ_OK;
 }
@@ -1608,17 +1596,14 @@ static int bt_verify_commit(dz_ctx* x, int a) {
   const int64_t hd = c.ssm_state, kdim = (int64_t)c.ssm_k_heads * hd, inner = (int64_t)c.ssm_v_heads * hd;
   const int64_t qkvd = 2 * kdim + inner;
   const int p0 = x->pos_host;
-  for (const LayerDev& l : m->L) {
-    if (l.attn) continue;
-    const int si = l.kind_idx;
-    DZ_HIP_CHECK(launch(bt_commit_state_kernel, dim3((unsigned)(4 * c.ssm_v_heads)), dim3(256), x->s,
-                        x->ssm_state + (size_t)si * c.ssm_v_heads * hd * hd, x->bt.rec[(size_t)si], a,
-                        (int)c.ssm_k_heads, (int)c.ssm_v_heads));
-    DZ_HIP_CHECK(launch(bt_ring_kernel, dim3((unsigned)((qkvd + 255) / 256)), dim3(256), x->s,
-                        (const float*)x->bt.rx[(size_t)si], qkvd, std::max(0, a - 4), a,
-                        x->conv + (size_t)si * 4 * qkvd, (x->ring_base[(size_t)si] + p0) & 3, qkvd));
-  }
-  return bt_finish(x, x->bt.pending_ids.data(), a, p0, a - 1);
+  if (m->n_ssm)
+    DZ_HIP_CHECK(launch(bt_commit_kernel, dim3((unsigned)(4 * c.ssm_v_heads + (qkvd + 255) / 256), (unsigned)m->n_ssm), dim3(256),
+                        x->s, x->ssm_state, x->conv, (const int*)x->ring_base_dev, p0, x->bt.recs, a, (int)c.ssm_k_heads,
+                        (int)c.ssm_v_heads, qkvd));
+  const int rc = bt_finish(x, a, p0, a - 1);
+  if (rc) return rc;
+  DZ_HIP_CHECK(hipStreamSynchronize(x->s));
+  return DZ_OK;
 }
 
 // Device logits of a pending verify for the sampler (spec.hip): row 0 = the context's logits (they
@@ -1658,7 +1643,7 @@ static int bt_prefill(dz_ctx* x, const uint32_t* ids, int n, float* last_logits,
     const int k = std::min(chunk, n - i0);
     const int rows = per_pos ? k : 1;
     int rc = bt_forward(x, ids + i0, k, rows, false);
-    if (rc || (rc = bt_finish(x, ids + i0, k, x->pos_host, rows - 1))) return rc;
+    if (rc || (rc = bt_finish(x, k, x->pos_host, rows - 1))) return rc;
     if (per_pos)
       DZ_HIP_CHECK(hipMemcpyAsync(per_pos + (size_t)i0 * V, x->bt.logits, (size_t)k * V * 4, hipMemcpyDeviceToHost, x->s));
   }
@@ -1908,6 +1893,7 @@ int dz_ctx_set_ssm_state(dz_ctx* x, int layer, const float* state, const float* 
   const dz_config& c = x->m->cfg;
   const int64_t hd = c.ssm_state, nvh = c.ssm_v_heads, qkvd = (2 * (int64_t)c.ssm_k_heads + nvh) * hd;
   if (conv_head < 0 || conv_head > 3) return set_error(DZ_ERR_TENSOR, "conv_head %d", conv_head);
+  DZ_HIP_CHECK(hipStreamSynchronize(x->s));  // a position change may still be on its way to the ring bases
   DZ_HIP_CHECK(hipMemcpy(x->ssm_state + (size_t)l->kind_idx * nvh * hd * hd, state, (size_t)(nvh * hd * hd) * 4,
                          hipMemcpyHostToDevice));
   DZ_HIP_CHECK(hipMemcpy(x->conv + (size_t)l->kind_idx * 4 * qkvd, conv_hist, (size_t)(4 * qkvd) * 4, hipMemcpyHostToDevice));
