@@ -34,6 +34,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 6;
 
+// The signs' block scale, 2^-7: a group's 128 terms then sum without overflow whatever they are, as they do when
+// the f16 scale comes first; kSignUp takes it back where the row's sum is stored (both exact).
+constexpr int kSignScale = 0x78;
+constexpr float kSignUp = 128.0f;
+
 // 32 signs (bit 4j + k of w = element 8k + j) as f4 values: bit set -> +1 (0x2), clear -> -1 (0xA).
 __device__ __forceinline__ void expand_f4(unsigned w, i32x8& a) {
 #pragma unroll
@@ -41,13 +46,13 @@ __device__ __forceinline__ void expand_f4(unsigned w, i32x8& a) {
 }
 
 // Digit 0's block scale of a block whose largest |value| has the bits mb, and the exponent e its values are
-// taken by (v = x · 2^(4-e)).  Scales go down to 35 below digit 0's (an operand's zero slots included) and
-// have to stay block scales: a block whose largest value is below 2^-90 is held to 2^-115 absolute.
+// taken by (v = x · 2^(4-e)).  The scales go down to digit 5's, 25 below digit 0's, and have to stay block
+// scales (>= 0): a block whose largest value is below 2^-102 is held to 2^-131 absolute.
 __device__ __forceinline__ unsigned digit_scale(unsigned mb, int& e) {
   e = 0;
   if (mb >= 0x7F800000u) return 0xFFu;  // an infinity or a NaN in the block
   (void)frexpf(__builtin_bit_cast(float, mb), &e);
-  e = mb == 0 ? 0 : (e < -90 ? -90 : e);
+  e = mb == 0 ? 0 : (e < -101 ? -101 : e);
   return (unsigned)(126 + e);
 }
 
@@ -104,6 +109,9 @@ struct FewForm {
   static constexpr int kEx = 4 * kGrp;                            // the block scales: [lane] a byte per group
   static constexpr int kTile = kEx + 256;
 };
+// How far the block scale of slot p of an operand lies below digit 0's (slots past the six digits hold zeros and
+// take the last digit's).
+__host__ __device__ constexpr int slot_drop(int p) { return 5 * (p < kDigits ? p : kDigits - 1); }
 constexpr int kFewStage = 16 * 36 * 4;  // a wave's 512 staged columns, blocks of 32 padded to 36
 
 template <int CTRL>
@@ -175,7 +183,7 @@ __device__ __forceinline__ void few_pack(unsigned char* tile, float* st, unsigne
   });
   if (kq == 0) {
 #pragma unroll
-    for (int p = 0; p < FF::P; ++p) tile[FF::kEx + 4 * (16 * q + p * T + tok) + g] = (unsigned char)(b0 - 5 * p);
+    for (int p = 0; p < FF::P; ++p) tile[FF::kEx + 4 * (16 * q + p * T + tok) + g] = (unsigned char)(b0 - slot_drop(p));
   }
 }
 
@@ -207,7 +215,7 @@ __device__ __forceinline__ void few_pack_out(uint8_t* __restrict__ tile, unsigne
   if ((lane & 3u) == 0) {
 #pragma unroll
     for (int p = 0; p < FF::P; ++p)
-      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - 5 * p);
+      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - slot_drop(p));
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -233,6 +241,9 @@ template <int T>
 __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lane, unsigned psel, const FewUnit& u, f32x4 (&acc)[4]) {
   using FF = FewForm<T>;
   const unsigned ex = *reinterpret_cast<const unsigned*>(tile + FF::kEx + 4 * lane);
+  // operand f's slots: P digits further down than operand f - 1's, where there are that many (T = 4: the second
+  // operand's slots 2 and 3, rows 8 and up, hold zeros, and a scale that ran below 0 would borrow from its neighbour)
+  const unsigned drop = T == 4 && (lane & 8u) ? 0u : 0x05050505u * (unsigned)FF::P;
   const unsigned char* fl = tile + (lane >> 4) * FF::kBlk + 24 * (lane & 15u);
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
@@ -245,14 +256,14 @@ __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lan
       const u32x2* p = reinterpret_cast<const u32x2*>(fl + g * FF::kGrp + f * FF::kOp);
       const u32x2 p0 = p[0], p1 = p[1], p2 = p[2];
       const i32x8 a = {(int)p0.x, (int)p0.y, (int)p1.x, (int)p1.y, (int)p2.x, (int)p2.y, 0, 0};
-      const int sx = (int)(ex - 0x05050505u * (unsigned)(f * FF::P));
+      const int sx = (int)(ex - drop * (unsigned)f);
 #pragma unroll
       for (int sb = 0; sb < 4; ++sb) {
         const f32x4 c = f == FF::F - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
-        if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, 0x7F);
-        else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, 0x7F);
-        else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, 0x7F);
-        else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, 0x7F);
+        if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, kSignScale);
+        else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, kSignScale);
+        else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, kSignScale);
+        else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, kSignScale);
       }
     }
 #pragma unroll
@@ -427,11 +438,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
   for (int v = 0; v < (T == 2 ? 2 : 4); ++v) {
     const int tok = T == 2 ? v : (4 * (int)q + v) % T;
     if (tok >= n_tok || (T == 2 && q) || (T == 4 && q) || (T == 8 && q > 1)) continue;
-    float inv = 1.0f;
+    float inv = kSignUp;
     if (!PRE && x.nw && gridDim.y == 1) {
       float s = ssqs[0][tok];
       for (int t = 1; t < nt; ++t) s += ssqs[t][tok];
-      inv = 1.0f / sqrtf(s / (float)x.K + x.eps);
+      inv = kSignUp / sqrtf(s / (float)x.K + x.eps);
     }
     float* yr = y + (size_t)tok * ldy + rb * kRowBlock + r;
 #pragma unroll

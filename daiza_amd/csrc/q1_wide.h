@@ -115,12 +115,12 @@ __device__ __forceinline__ i32x8 read_frag(const unsigned char* f, unsigned lane
 //     matrix instructions (one per 16-row block).
 //   B operand (lane & 15 = weight row): 32 signs of one group as f4.
 //   D: lane holds tokens 4q .. 4q+3 of weight row lane & 15, so a group's scale is one value per lane.
-// The digits of the next half tile travel to the other LDS buffer (lds_dma16) while this one is
+// The digits of the next half tile travel to the other LDS buffer (lds_dma) while this one is
 // multiplied; its signs go into the registers that the expansion has just read.  Two workgroups share a CU
 // (2 x 72 KiB of LDS), so one's barrier and scale fmas hide behind the other's matrix instructions.
 // Bound by the matrix instructions: per group and wave 96 of them (about 20 cycles each) against
 // 18 KiB of LDS reads (48 B per cycle and CU) and ~130 VALU operations.
-// Grid: 1-D, row groups x token groups x splits (wide_tile); y and splits as q1_gemm_kernel's.
+// Grid: 1-D, row groups x token groups x splits (wide_tile); a split writes its partial to y + z·zstride.
 struct WideGrid {
   int nrg;  // row groups: ceil(nrb / kWideRb)
   int ntg;  // token groups: Np / kWideTok
@@ -204,8 +204,8 @@ __global__ __launch_bounds__(256, 2) void q1_wide_kernel(const uint8_t* __restri
   load_signs(t0, 0, 1);
   load_ex(t0, exv);
   if (tid < kWideTok) {  // 1/rms of the tokens, from the tiles' sums of squares
-    float inv = 1.0f;
-    if (x.ssq) inv = 1.0f / sqrtf(ordered_sum(x.ssq + tg * kWideTok + tid, x.Np, ntiles) / (float)x.K + x.eps);
+    float inv = kSignUp;
+    if (x.ssq) inv = kSignUp / sqrtf(ordered_sum(x.ssq + tg * kWideTok + tid, x.Np, ntiles) / (float)x.K + x.eps);
     tok_inv[tid] = inv;
   }
   lds_dma_wait();
@@ -244,10 +244,10 @@ __global__ __launch_bounds__(256, 2) void q1_wide_kernel(const uint8_t* __restri
 #pragma unroll
             for (int sb = 0; sb < SB; ++sb) {
               const f32x4 c = k == kDigits - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
-              if (h == 0 && g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, (int)sx, 0, 0x7F);
-              else if (h == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, (int)sx, 0, 0x7F);
-              else if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, (int)sx, 0, 0x7F);
-              else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, (int)sx, 0, 0x7F);
+              if (h == 0 && g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, (int)sx, 0, kSignScale);
+              else if (h == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, (int)sx, 0, kSignScale);
+              else if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, (int)sx, 0, kSignScale);
+              else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, (int)sx, 0, kSignScale);
             }
             a = an;
             asm("v_add_u32 %0, 0x5050505, %0" : "+v"(sx));  // (opaque: the six values would each take a register)

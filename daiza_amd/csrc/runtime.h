@@ -59,7 +59,7 @@ int ctx_usable(const dz_ctx* x);
 hipError_t launch_partial_reduce(const float* part, int64_t ld, int n_tg, const ReduceSeg* segs, int nseg,
                                  int accumulate, hipStream_t s);
 
-// N-column products on the matrix cores (q1_gemm.h): activations packed once per input, then
+// N-column products on the matrix cores (q1_digits.h, q1_wide.h): activations packed once per input, then
 // one launch per matrix.
 struct PackedX {
   uint8_t* dig = nullptr;   // digit operands (q1_digits.h)

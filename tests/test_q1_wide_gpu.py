@@ -74,3 +74,23 @@ def test_block_ranges_and_non_finite(dz):
     assert np.all(np.isnan(yb[7])) and np.all(np.isnan(yb[9]))
     keep = [i for i in range(n) if i not in (7, 9)]
     assert np.array_equal(yb[keep], y[keep])
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 7, 16, 20])
+def test_ends_of_the_range(dz, n):
+    """Activations near the ends of f32's exponent range, in every form of the product: tiny ones keep their
+    precision, and a group's terms do not overflow where the f16 scale brings the result back."""
+    rows, cols = 96, 640
+    rng = np.random.default_rng(n)
+    aos, w = _matrix(rng, rows, cols)
+    m = dz.Q1_0Matrix(aos, rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    for e in (-100, -93, -86, 110, 120):
+        xe = np.ldexp(x, e)
+        _check(m.matvec_batch(xe), w, xe)
+    # one group whose 128 terms of 2^122 have one sign in row 0: 2^129 before the scale, and every row's
+    # result at most 2^129 max(scale), which is finite
+    big = np.zeros_like(x)
+    big[:, :128] = np.ldexp(np.sign(w[0, :128]), 122)
+    assert 2.0 ** 129 * np.abs(w[:, :128]).max() < 2.0 ** 127
+    _check(m.matvec_batch(big), w, big)
