@@ -1,5 +1,5 @@
 // batch_kernels.h — the n-token forward (forward_batch, Daiza-engine/src/model/forward.rs:394-1407)
-// outside the projections, which run on the matrix cores (q1_gemm.h).  Activations are token-major
+// outside the projections, which run on the matrix cores (q1_digits.h, q1_wide.h).  Activations are token-major
 // [n][width] f32.  Used for prefill (dz_forward_batch) and for speculative verify, where the
 // DeltaNet scan records what a rollback needs instead of writing the state back.
 #pragma once
@@ -308,7 +308,10 @@ __global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __re
     const int t = t0 + (int)tid, tc = min(t, n - 1);
     const float x = yin[(size_t)tc * ldin + off_a + vh] + dt_bias[vh], b = yin[(size_t)tc * ldin + off_b + vh];
     const float spl = x > 20.0f ? x : logf(1.0f + expf(x));
-    la[tid] = t < n ? ssm_a[vh] * spl : 0.f;
+    // e^-10000 is 0 already: held there, differences of L stay exact enough behind a token that clears the state
+    // (an ln a of -inf would make them NaN)
+    const float ga = ssm_a[vh] * spl, gc = ga < -1e4f ? -1e4f : ga;
+    la[tid] = t < n ? gc : 0.f;
     bet[tid] = t < n ? sigmoidf_(b) : 0.f;
   }
   __syncthreads();
