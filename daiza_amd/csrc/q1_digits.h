@@ -320,7 +320,7 @@ __host__ __device__ constexpr size_t few_shmem(int nw, int tps) {
 // K tiles of a workgroup (its LDS)
 constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
 
-// Grid (ceil(nrb / NW), splits), 64·NW threads: workgroup (chunk, z) takes K tiles [z·tps, min(ntiles, (z+1)·tps))
+// Grid (ceil(nrb / NW), splits, blocks of 16 tokens), 64·NW threads: workgroup (chunk, z) takes K tiles [z·tps, min(ntiles, (z+1)·tps))
 // of NW row-blocks, one per wave.  The inputs are requested first, the first unit's weights behind them, and the
 // packing runs while the weights arrive; one barrier, then every wave goes its own way.  With more than one
 // split, workgroup z writes its partial to y + z·zstride.
@@ -342,6 +342,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
   __shared__ float ssqs[few_max_tiles(T)][T];
   const unsigned tid = threadIdx.x, lane = tid & 63u, r = lane & 15u, q = lane >> 4;
   const int wave = (int)__builtin_amdgcn_readfirstlane(tid >> 6);
+  // token block blockIdx.z: 16 columns of a product with more
+  const int tb = 16 * (int)blockIdx.z;
+  n_tok = min(n_tok - tb, 16);
   const int t0 = (int)blockIdx.y * tps, nt = min(ntiles - t0, tps);
   const int64_t rb = (int64_t)blockIdx.x * NW + wave;
   float* st = reinterpret_cast<float*>(smem + (size_t)tps * FF::kTile) + wave * (kFewStage / 4);
@@ -357,7 +360,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
     const int64_t c0 = (int64_t)(t0 + kc / n_tok) * kTileCols + 4 * lane, c1 = c0 + 256;
     // K is a multiple of 128, so a float4 is wholly in or out; past it, column 0 is read and dropped
     const bool i0 = c0 < x.K, i1 = c1 < x.K;
-    const float* p = x.xf + (size_t)tok * x.ldx;
+    const float* p = x.xf + (size_t)(tb + tok) * x.ldx;
     In v;
     v.x0 = *reinterpret_cast<const float4*>(p + (i0 ? c0 : 0));
     v.x1 = *reinterpret_cast<const float4*>(p + (i1 ? c1 : 0));
@@ -389,7 +392,6 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
   FewUnit u;
   if (rb < nrb) few_load(wr, woff, soff, unit0, u);
   auto pack = [&](int k, const In& v) {
-    if (k >= tasks) return;  // wave-uniform
     const int tok = k % n_tok, t = k / n_tok;
     const int64_t c0 = (int64_t)(t0 + t) * kTileCols + 4 * lane;
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -410,15 +412,19 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
       if ((int)tid + 64 * NW * i < pieces) dst[tid + 64 * NW * i] = pc[i];
     for (int i = (int)tid + 64 * NW * MP; i < pieces; i += 64 * NW) dst[i] = psrc[i];
   } else {
-#pragma unroll
-    for (int i = 0; i < MT; ++i) pack(wave + NW * i, in[i]);
-    for (int k = wave + NW * MT; k < tasks; k += NW) pack(k, load_x(k));
+    // (one copy of the packing code, which a call that is alone on the device fetches cold)
+#pragma unroll 1
+    for (int k = wave; k < tasks; k += NW) {
+      pack(k, in[0]);
+      in[0] = in[1];
+      if (k + 2 * NW < tasks) in[1] = load_x(k + 2 * NW);
+    }
   }
   lds_barrier();  // the weights stay in flight
   if (!PRE && x.nw && gridDim.y > 1 && blockIdx.x == 0 && tid < (unsigned)n_tok) {
     float s = ssqs[0][tid];
     for (int t = 1; t < nt; ++t) s += ssqs[t][tid];
-    x.ssq[(size_t)blockIdx.y * x.ssq_ld + tid] = s;
+    x.ssq[(size_t)blockIdx.y * x.ssq_ld + tb + tid] = s;
   }
   if (rb >= nrb) return;
   f32x4 acc[4];
@@ -444,7 +450,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
       for (int t = 1; t < nt; ++t) s += ssqs[t][tok];
       inv = kSignUp / sqrtf(s / (float)x.K + x.eps);
     }
-    float* yr = y + (size_t)tok * ldy + rb * kRowBlock + r;
+    float* yr = y + (size_t)(tb + tok) * ldy + rb * kRowBlock + r;
 #pragma unroll
     for (int sb = 0; sb < 4; ++sb)
       if (rb * kRowBlock + 16 * sb + r < rows) {

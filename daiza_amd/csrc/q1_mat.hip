@@ -357,19 +357,29 @@ struct FewPlan {
 // spread over enough waves (about kFewWaves) and no more splits than that takes: each split adds a pass over
 // partials.  Workgroups that pack their tiles themselves share that over eight waves, unless half of the CUs would
 // be left without one (at eight tokens 16480 x 5120 16.9 against 13.1 us, 5120 x 6144 7.6 against 8.0); with packed
-// tiles four waves spread better (16480 x 5120 9.5 against 10.5, 5120 x 17408 8.9 against 10.0).
+// tiles four waves spread better (16480 x 5120 9.5 against 10.5, 5120 x 17408 8.9 against 10.0), except in the form of
+// sixteen tokens, where a tile's 40 KiB of digits would be copied for every four row-blocks (a four-layer block's
+// forward of 9 tokens 560 us with four waves, 480 with eight; 16 tokens 591 and 513).
 constexpr int kFewWaves = 2048;
-static FewPlan few_plan(const Q1Dev& W, int T, bool pre) {
+static FewPlan few_plan(const Q1Dev& W, int n, int T, bool pre) {
   FewPlan p;
   const int nt = (int)W.ntiles;
-  const int64_t want = std::max<int64_t>(1, (kFewWaves + W.nrb - 1) / W.nrb);  // splits
+  const int64_t zb = (n + 15) / 16, waves = W.nrb * zb;
+  const int64_t want = std::max<int64_t>(1, (kFewWaves + waves - 1) / waves);  // splits
   p.tps = (int)std::max<int64_t>(1, (nt + want - 1) / want);
   p.tps = std::min(p.tps, few_max_tiles(T));
   p.splits = (nt + p.tps - 1) / p.tps;
-  p.nw = !pre && 2 * ((W.nrb + 7) / 8 * p.splits) >= device_cus() ? 8 : 4;
+  if (pre) p.nw = T == 16 ? 8 : 4;
+  else p.nw = 2 * ((W.nrb + 7) / 8 * zb * p.splits) >= device_cus() ? 8 : 4;
   p.chunks = (unsigned)((W.nrb + p.nw - 1) / p.nw);
   return p;
 }
+// More than 16 columns of a small product go in blocks of 16 through the few-column form: up to one unit per wave of
+// a round (kFewWaves), its workgroups are many and short where the wide form's 512 x 32 tiles leave CUs idle behind a
+// packing launch.  matvec_batch, us per call, wide form against this one: 1024 x 640 by 40 58.9 and 51.1, 5120 x 5120
+// by 24 87.2 and 80.5, 4096 x 1024 by 256 331 and 327; past the line 6000 x 2560 by 100 222.8 and 224.3,
+// 17408 x 5120 by 17 133.8 and 138.4.
+static bool few_blocks(const Q1Dev& W, int n) { return W.nrb * W.ntiles * ((n + 15) / 16) <= kFewWaves; }
 static int few_form(int n) { return n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16; }
 
 template <int T, int NW, bool PRE>
@@ -382,7 +392,7 @@ static hipError_t launch_few(const FewPlan& p, const Q1Dev& W, const FewX& x, in
     if (e != hipSuccess) return e;
     attr = true;
   }
-  hipLaunchKernelGGL((q1_few_kernel<T, NW, PRE>), dim3(p.chunks, (unsigned)p.splits), dim3(64 * NW), few_shmem<T>(NW, p.tps), s,
+  hipLaunchKernelGGL((q1_few_kernel<T, NW, PRE>), dim3(p.chunks, (unsigned)p.splits, (unsigned)((n + 15) / 16)), dim3(64 * NW), few_shmem<T>(NW, p.tps), s,
                      W.data, W.rows, W.nrb, (int)W.ntiles, p.tps, x, n, y, ldy, zs, accumulate);
   return hipGetLastError();
 }
@@ -417,7 +427,7 @@ hipError_t launch_q1_few_packed(const Q1Dev& W, const uint8_t* dig, const float*
   fx.dig = dig;
   fx.K = W.cols;
   const int T = few_form(n);
-  const FewPlan p = few_plan(W, T, true);
+  const FewPlan p = few_plan(W, n, T, true);
   const int S = p.splits;
   const bool direct = S == 1 && !ssq;  // otherwise the sum of the partials (or of the one) applies 1/rms
   const int64_t zs = (int64_t)n * W.rows;
@@ -438,7 +448,6 @@ hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n
                               int accumulate, hipStream_t s, Scratch* split, const float* norm_w, float eps,
                               GemmDefer* defer) {
   if ((W.cols & 3) || (ldx & 3)) return hipErrorInvalidValue;  // 16-byte loads of x rows
-  if (n > 16) return hipErrorInvalidValue;
   FewX fx{};
   fx.xf = x;
   fx.ldx = ldx;
@@ -446,7 +455,7 @@ hipError_t launch_q1_gemm_raw(const Q1Dev& W, const float* x, int64_t ldx, int n
   fx.nw = norm_w;
   fx.eps = eps;
   const int T = few_form(n);
-  const FewPlan p = few_plan(W, T, false);
+  const FewPlan p = few_plan(W, n, T, false);
   const int S = p.splits;
   float* out = y;
   int64_t ld = ldy, zs = 0;
@@ -785,7 +794,7 @@ int dz_q1_0_matvec_batch(dz_mat* m, const float* x, int n, float* y, int accumul
   float* yd = static_cast<float*>(g_y.ptr);
   DZ_HIP_CHECK(hipMemcpyAsync(xd, x, (size_t)n * K * 4, hipMemcpyHostToDevice, s));
   if (accumulate) DZ_HIP_CHECK(hipMemcpyAsync(yd, y, (size_t)n * R * 4, hipMemcpyHostToDevice, s));
-  if (n <= 16) {  // few tokens: the product packs its tiles itself (as the batched forward does)
+  if (n <= 16 || few_blocks(m->d, n)) {  // few tokens: the product packs its tiles itself (as the batched forward does)
     DZ_HIP_CHECK(launch_q1_gemm_raw(m->d, xd, (int64_t)K, n, yd, (int64_t)R, accumulate, s, &g_split));
   } else {
     DZ_HIP_CHECK(launch_x_pack(xd, (int64_t)K, (int64_t)K, n, nullptr, 0.f, p, s));

@@ -94,3 +94,22 @@ def test_ends_of_the_range(dz, n):
     big[:, :128] = np.ldexp(np.sign(w[0, :128]), 122)
     assert 2.0 ** 129 * np.abs(w[:, :128]).max() < 2.0 ** 127
     _check(m.matvec_batch(big), w, big)
+
+
+@pytest.mark.parametrize("rows,cols,n", [
+    (4613, 1152, 161),   # above the line between the 16-column blocks and the 512 x 32 tiles: ragged rows, half a
+    (5121, 640, 207),    # K tile, a token past a tile; one row into the last row group
+    (8192, 512, 256),    # the line itself (2048 units): blocks
+    (8192, 512, 257),    # and one column past it: tiles
+    (130, 1664, 250),    # blocks: three row-blocks, a ragged last block of columns, split K
+])
+def test_both_sides_of_the_block_line(dz, rows, cols, n):
+    rng = np.random.default_rng(rows + n)
+    aos, w = _matrix(rng, rows, cols)
+    m = dz.Q1_0Matrix(aos, rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    _check(m.matvec_batch(x), w, x)
+    y0 = rng.standard_normal((n, rows)).astype(np.float32)
+    y = y0.copy()
+    m.matvec_add_batch_into_slice(x, n, y)
+    _check(y - y0.astype(np.float64), w, x, extra=2.0 ** -23 * (np.abs(y0) + np.abs(y)))
