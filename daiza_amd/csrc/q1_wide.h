@@ -127,6 +127,13 @@ struct WideGrid {
   int tps;  // K tiles per split
 };
 
+// The row-block, counted from its row group's first, whose weights stand for row-block i of row group rg: i itself, or
+// the matrix's last where i lies past it.
+__host__ __device__ constexpr int wide_row_block(int rg, int i, int64_t nrb) {
+  const int64_t left = nrb - (int64_t)rg * kWideRb;
+  return i < left ? i : (int)left - 1;
+}
+
 // Workgroup index -> (row group, token group, split).  The hardware deals workgroups to the eight XCDs in turn, so
 // XCD x takes a contiguous run of the tile order, and that order walks bands of eight row groups token group by token
 // group: the workgroups an XCD runs together share eight row groups' weights and a few token groups' digits in its L2.
@@ -166,12 +173,14 @@ __global__ __launch_bounds__(256, 2) void q1_wide_kernel(const uint8_t* __restri
     lds_dma<4>(src, 16 * lane + 4096, dst + 4096);
     lds_dma<1>(src, 16 * lane + 8192, dst + 8192);
   };
-  // the weights of the workgroup's row-blocks; reads past the matrix return 0 (those rows are not stored)
+  // the weights of the workgroup's row-blocks; a row-block past the matrix reads the last one's (its rows are not
+  // stored): the buffer's bounds check does not cover the scalar offset
   const int64_t rb0 = (int64_t)rg * kWideRb + 2 * wave;
   const size_t wbytes = (size_t)(nrb - (int64_t)rg * kWideRb) * ntiles * kUnitBytes;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(W) + (size_t)rg * kWideRb * ntiles * kUnitBytes, 0, (int)(wbytes < 0x7FFFFFFFu ? wbytes : 0x7FFFFFFFu), 0x00027000);
-  const int u0 = (int)(2 * wave) * ntiles * kUnitBytes, u1 = u0 + ntiles * kUnitBytes;
+  const int u0 = wide_row_block(rg, 2 * (int)wave, nrb) * ntiles * kUnitBytes;
+  const int u1 = wide_row_block(rg, 2 * (int)wave + 1, nrb) * ntiles * kUnitBytes;
   const int woff = (int)(16u * r + 4u * (q ^ (r >> 2)));   // the lane's dword of a 16-row block's chunk
   const int soff = kUnitSignBytes + 8 * (int)r;
   const unsigned psel = 0x03020100u ^ (0x01010101u * (r & 3u));  // its bytes back to column order
