@@ -1893,7 +1893,7 @@ int dz_ctx_set_ssm_state(dz_ctx* x, int layer, const float* state, const float* 
   const dz_config& c = x->m->cfg;
   const int64_t hd = c.ssm_state, nvh = c.ssm_v_heads, qkvd = (2 * (int64_t)c.ssm_k_heads + nvh) * hd;
   if (conv_head < 0 || conv_head > 3) return set_error(DZ_ERR_TENSOR, "conv_head %d", conv_head);
-  DZ_HIP_CHECK(hipStreamSynchronize(x->s));  // a position change may still be on its way to the ring bases
+  DZ_HIP_CHECK(hipStreamSynchronize(x->s));  // the copies below are not ordered with the context's stream
   DZ_HIP_CHECK(hipMemcpy(x->ssm_state + (size_t)l->kind_idx * nvh * hd * hd, state, (size_t)(nvh * hd * hd) * 4,
                          hipMemcpyHostToDevice));
   DZ_HIP_CHECK(hipMemcpy(x->conv + (size_t)l->kind_idx * 4 * qkvd, conv_hist, (size_t)(4 * qkvd) * 4, hipMemcpyHostToDevice));
@@ -1925,6 +1925,8 @@ int dz_ctx_set_kv(dz_ctx* x, int layer, const float* k, const float* v, int len)
   if (rc) return rc;
   const dz_config& c = x->m->cfg;
   if (len < 0 || len > c.max_ctx) return set_error(DZ_ERR_TENSOR, "kv len %d", len);
+  // the copies below are not ordered with the context's stream: enqueued steps still read and append rows
+  DZ_HIP_CHECK(hipStreamSynchronize(x->s));
   const size_t kvsz = (size_t)c.n_head_kv * c.max_ctx * c.head_dim, hd = (size_t)c.head_dim;
   float* kb = x->kv + (size_t)l->kind_idx * 2 * kvsz;
   for (int h = 0; h < c.n_head_kv; ++h) {

@@ -303,6 +303,10 @@ int dz_ctx_get_ssm_state(dz_ctx* c, int layer, float* state, float* conv_hist, i
 int dz_ctx_set_kv(dz_ctx* c, int layer, const float* k, const float* v, int len);
 int dz_ctx_get_kv(dz_ctx* c, int layer, float* k, float* v, int len);
 int dz_ctx_kv_len(dz_ctx* c, int layer);
+/* The four set/get calls above wait for the work enqueued on the context's stream before they touch the state.
+ * The two below move the position in stream order and do not wait: steps enqueued before them
+ * (dz_ctx_mixer_step_dev) may still be running when they return, so a caller that reads or frees such a step's
+ * buffers synchronises dz_ctx_stream itself. */
 int dz_kv_truncate(dz_ctx* c, int len);                    /* KvCache::truncate (kv_cache.rs:119-130) */
 int dz_ctx_set_pos(dz_ctx* c, int pos);
 

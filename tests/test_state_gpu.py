@@ -314,3 +314,58 @@ def test_copy_state_across_shapes_and_paths(dz, oracle, monkeypatch):
         small.copy_state_from(long_ctx)
     assert e.value.code == dz.DZ_ERR_TENSOR
     assert small.pos == 1
+
+
+def _steps_dev(dz, ctx, h, out, n):
+    for t in range(n):
+        rc = dz.lib().dz_ctx_mixer_step_dev(ctx._h, 0, h[t].data_ptr(), out[t].data_ptr())
+        assert rc == dz.DZ_OK
+
+
+@pytest.mark.parametrize("attn", [True, False])
+def test_state_replaced_behind_enqueued_steps(dz, attn):
+    """dz_ctx_set_kv and dz_ctx_set_ssm_state wait for the steps enqueued before them, whose position change
+    (set_pos) does not: the enqueued steps and the one after the replacement give the same bits as with an explicit
+    wait after every call."""
+    torch = pytest.importorskip("torch")
+    L, n = 2000, 16
+    cfg = dz.Config.bonsai27b(max_ctx=L + n)
+    cfg.n_layers, cfg.vocab, cfg.full_attn_interval = 1, 512, 1 if attn else 4
+    m = dz.Model.synthetic(cfg, SEED + 9)
+    rng = np.random.default_rng(21)
+    if attn:
+        states = [[rng.standard_normal((cfg.n_head_kv, L, cfg.head_dim), dtype=np.float32) for _ in range(2)] for _ in range(2)]
+    else:
+        states = [[(rng.standard_normal(s) * 0.1).astype(np.float32)
+                   for s in ((cfg.ssm_v_heads, 128, 128), (4, cfg.qkv_dim))] for _ in range(2)]
+
+    def put(ctx, s):
+        if attn:
+            ctx.set_kv(0, *s)
+        else:
+            ctx.set_ssm_state(0, *s, 1)
+
+    def get(ctx):
+        return ctx.get_kv(0, L + 1) if attn else ctx.get_ssm_state(0)[:2]
+
+    h = torch.from_numpy(rng.standard_normal((n, cfg.hidden), dtype=np.float32)).cuda()
+    torch.cuda.synchronize()
+    res = []
+    for wait in (torch.cuda.synchronize, lambda: None):
+        ctx = dz.Context(m)
+        put(ctx, states[0])
+        ctx.set_pos(L)
+        out, last = torch.zeros_like(h), torch.zeros_like(h[:1])
+        torch.cuda.synchronize()
+        _steps_dev(dz, ctx, h, out, n)
+        wait()
+        ctx.set_pos(L)
+        wait()
+        put(ctx, states[1])
+        wait()
+        _steps_dev(dz, ctx, h, last, 1)
+        torch.cuda.synchronize()
+        res.append((out.cpu().numpy(), last.cpu().numpy(), *get(ctx)))
+        ctx.close()
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
