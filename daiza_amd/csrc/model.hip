@@ -1639,16 +1639,23 @@ static int bt_prefill(dz_ctx* x, const uint32_t* ids, int n, float* last_logits,
   const size_t V = (size_t)x->m->cfg.vocab;
   const int chunk = per_pos ? 128 : kBatchChunk;
   x->bt.pending = 0;
-  for (int i0 = 0; i0 < n; i0 += chunk) {
-    const int k = std::min(chunk, n - i0);
-    const int rows = per_pos ? k : 1;
-    int rc = bt_forward(x, ids + i0, k, rows, false);
-    if (rc || (rc = bt_finish(x, k, x->pos_host, rows - 1))) return rc;
-    if (per_pos)
-      DZ_HIP_CHECK(hipMemcpyAsync(per_pos + (size_t)i0 * V, x->bt.logits, (size_t)k * V * 4, hipMemcpyDeviceToHost, x->s));
-  }
-  if (last_logits) DZ_HIP_CHECK(hipMemcpyAsync(last_logits, x->logits, V * 4, hipMemcpyDeviceToHost, x->s));
-  DZ_HIP_CHECK(hipStreamSynchronize(x->s));
+  auto enqueue = [&]() -> int {
+    for (int i0 = 0; i0 < n; i0 += chunk) {
+      const int k = std::min(chunk, n - i0);
+      const int rows = per_pos ? k : 1;
+      int rc = bt_forward(x, ids + i0, k, rows, false);
+      if (rc || (rc = bt_finish(x, k, x->pos_host, rows - 1))) return rc;
+      if (per_pos)
+        DZ_HIP_CHECK(hipMemcpyAsync(per_pos + (size_t)i0 * V, x->bt.logits, (size_t)k * V * 4, hipMemcpyDeviceToHost, x->s));
+    }
+    if (last_logits) DZ_HIP_CHECK(hipMemcpyAsync(last_logits, x->logits, V * 4, hipMemcpyDeviceToHost, x->s));
+    return DZ_OK;
+  };
+  const int rc = enqueue();
+  // also when a later chunk is refused: the chunks before it still read ids and write per_pos
+  const hipError_t e = hipStreamSynchronize(x->s);
+  if (rc) return rc;
+  DZ_HIP_CHECK(e);
   return DZ_OK;
 }
 

@@ -2,6 +2,8 @@
 bad ids, empty batches, a full context and verify misuse are refused on the host with DZ_ERR_TENSOR
 before any launch, and the context stays usable with its state unchanged (checked against the
 oracle after each refusal)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,20 @@ def test_verify_misuse(dz, oracle):
     params = dz.SamplingParams(0.7, 20, 0.95)
     _refused(dz, ctx.spec_verify, [], None, params, dz.LcgRng(1), empty=True)
     _still_matches(ctx, om)
+
+
+def test_refusal_in_a_later_chunk_leaves_nothing_running(dz):
+    """A prompt of more than one chunk (1024 tokens) with a bad id in the second: the first chunk is kept, and when
+    the refusal returns, no work of it is left on the stream (it reads the caller's ids)."""
+    cfg = dz.Config.small(n_layers=4, max_ctx=1100)
+    ctx = dz.Context(dz.Model.synthetic(cfg, SEED))
+    ids = np.random.default_rng(1).integers(0, cfg.vocab, 1030).astype(np.uint32)
+    ids[1027] = cfg.vocab
+    ctx.forward_batch(ids[:1024])  # buffers grown, kernels loaded
+    ctx.reset()
+    with pytest.raises(dz.DaizaError) as e:
+        ctx.forward_batch(ids)
+    h = ctypes.CDLL("libamdhip64.so")
+    h.hipStreamQuery.argtypes = [ctypes.c_void_p]
+    assert h.hipStreamQuery(ctx.stream) == 0
+    assert e.value.code == dz.DZ_ERR_TENSOR and ctx.pos == 1024
