@@ -96,5 +96,5 @@ def test_refusal_in_a_later_chunk_leaves_nothing_running(dz):
         ctx.forward_batch(ids)
     h = ctypes.CDLL("libamdhip64.so")
     h.hipStreamQuery.argtypes = [ctypes.c_void_p]
-    assert h.hipStreamQuery(ctx.stream) == 0
+    assert h.hipStreamQuery(ctx.stream()) == 0
     assert e.value.code == dz.DZ_ERR_TENSOR and ctx.pos == 1024
