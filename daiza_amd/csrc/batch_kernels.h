@@ -801,6 +801,38 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
       for (int th = 0; th < 4; ++th) vv[4 * s + th] = *reinterpret_cast<const float4*>(vr + 64 * th);
     }
   };
+  // A block that some row of the wave does not see whole: the matrix instructions multiply the values of a masked
+  // position by that row's probability 0, which must not make NaN of an infinity or a NaN.  A position with such a
+  // value counts as zeros, and the rows that do see it get NaN.  (One fma per value; the rest is rare.)
+  const int rho_0 = 64 * tile + 16 * (int)w;
+  const int ctx_0 = rho_0 < rows ? min(pos0 + rho_0 / GRP + 1, pend) : pbeg;  // of the wave's first row: the smallest
+  auto hide_non_finite = [&](int pb) {
+    unsigned long long bad[4];  // positions pb + 4lk + s, as lanes
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      float nf = 0.f;
+#pragma unroll
+      for (int th = 0; th < 4; ++th) {
+        const float4 v4 = vv[4 * s + th];
+        nf = __builtin_fmaf(v4.x, 0.f, __builtin_fmaf(v4.y, 0.f, __builtin_fmaf(v4.z, 0.f, __builtin_fmaf(v4.w, 0.f, nf))));
+      }
+      bad[s] = __builtin_amdgcn_ballot_w64(nf != 0.f);
+    }
+    if ((bad[0] | bad[1] | bad[2] | bad[3]) == 0) return;
+    int first = 0x7FFFFFFF;
+#pragma unroll
+    for (int s = 3; s >= 0; --s) {
+      if (bad[s]) first = min(first, pb + 4 * (__builtin_ctzll(bad[s]) >> 4) + s);
+      if ((bad[s] >> (16 * lk)) & 0xFFFFu)
+#pragma unroll
+        for (int th = 0; th < 4; ++th) vv[4 * s + th] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (first < __shfl(ctx_r, 4 * lk + i))
+#pragma unroll
+        for (int t = 0; t < 16; ++t) o[t][i] = __builtin_nanf("");
+  };
   // scores of the block whose keys are in kk
   f32x4 s0, s1;
   auto scores = [&]() {
@@ -875,6 +907,7 @@ __global__ __launch_bounds__(256) void bt_attn_mfma_kernel(const float* __restri
         for (int t = 0; t < 16; ++t) o[t][i] *= a;
       }
     }
+    if (p0 + 16 > ctx_0) hide_non_finite(p0);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
