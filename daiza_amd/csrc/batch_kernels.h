@@ -287,6 +287,33 @@ __host__ __device__ inline ChunkPrep chunk_prep_carve(float* p, int n, int nkh, 
   return r;
 }
 
+// Causality for infinities and NaN.  T, N10 and A are 0 for a token's later ones, and 0 times a non-finite value is
+// NaN.  x: NT tiles of B operands (tile t, register r: token 16t + 4·(lane >> 4) + r of the lane's column).  Non-finite
+// values are set to 0; returns the first token that held one in the lane's column (16·NT: none), from which on the
+// column's results are NaN: a value that entered the recurrence stays in it.
+template <int NT>
+__device__ __forceinline__ int take_non_finite(f32x4 (&x)[NT], int lk) {
+  float nf = 0.f;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) nf = __builtin_fmaf(x[t][r], 0.f, nf);
+  int first = 16 * NT;
+  if (__builtin_amdgcn_ballot_w64(nf != 0.f)) {
+#pragma unroll
+    for (int t = NT - 1; t >= 0; --t)
+#pragma unroll
+      for (int r = 3; r >= 0; --r)
+        if (x[t][r] - x[t][r] != 0.f) {
+          x[t][r] = 0.f;
+          first = 16 * t + 4 * lk + r;
+        }
+    first = min(first, __shfl_xor(first, 16));
+    first = min(first, __shfl_xor(first, 32));
+  }
+  return first;
+}
+
 // Grid (nvh, chunks), 256 threads.  Tokens past n count as k = q = v = 0, β = 0, a = 1.
 // 16x16x4 f32 products: A lane (row = lane & 15, slot = lane >> 4), B lane (column, slot), D lane column
 // lane & 15, rows 4(lane >> 4) + i; step r of a 16-wide K block takes K index 4·slot + r, so that a lane's
@@ -356,9 +383,10 @@ __global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __re
     for (int i = 0; i < 4; ++i) {
       const int t = 16 * tt + 4 * lk + i;
       const bool in = t0 + t < n;  // (a token past n has read the last one's rows)
-      const float e = s <= t && in ? expf((float)(Ls[t] - Ls[s])) : 0.f;
+      const bool sees = s <= t && in;
+      const float e = sees ? expf((float)(Ls[t] - Ls[s])) : 0.f;
       N[t][s] = s < t ? bet[t] * e * dk[i] : 0.f;
-      o.a[(hv * C + t) * C + s] = e * dq[i];
+      o.a[(hv * C + t) * C + s] = sees ? e * dq[i] : 0.f;
     }
   } else {  // the tile above the diagonal, and (once per k-head) K^T
 #pragma unroll
@@ -399,23 +427,24 @@ __global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __re
       }
     }
     __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
-    f32x4 m = {0.f, 0.f, 0.f, 0.f}, tl = m;
+    f32x4 m[1] = {{0.f, 0.f, 0.f, 0.f}}, tl = m[0];
     const float4 na = *reinterpret_cast<const float4*>(&N[16 + ln][4 * lk]);
     const float4 t1 = *reinterpret_cast<const float4*>(&T[16 + ln][16 + 4 * lk]);
     const float nr[4] = {na.x, na.y, na.z, na.w}, tr[4] = {t1.x, t1.y, t1.z, t1.w};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) m = __builtin_amdgcn_mfma_f32_16x16x4f32(nr[r], T[4 * lk + r][ln], m, 0, 0, 0);
+    for (int r = 0; r < 4; ++r) m[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(nr[r], T[4 * lk + r][ln], m[0], 0, 0, 0);
+    const int nan0 = take_non_finite(m, lk);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) tl = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[r], m[r], tl, 0, 0, 0);
+    for (int r = 0; r < 4; ++r) tl = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[r], m[0][r], tl, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) T[16 + 4 * lk + i][ln] = -tl[i];
+    for (int i = 0; i < 4; ++i) T[16 + 4 * lk + i][ln] = 4 * lk + i < nan0 ? -tl[i] : __builtin_nanf("");
   }
   __syncthreads();
   // -W and U: wave w takes columns 32w .. 32w + 31 of both
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt) {
     const int col = 32 * (int)w + 16 * jt + ln;
-    float kx[2][4], vx[2][4];
+    f32x4 kx[2], vx[2];
 #pragma unroll
     for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -433,6 +462,7 @@ __global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __re
         kx[st][r] *= -be[s];
         vx[st][r] *= bet[s];
       }
+    const int nan_w = take_non_finite(kx, lk), nan_u = take_non_finite(vx, lk);
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
       f32x4 dw = {0.f, 0.f, 0.f, 0.f}, du = dw;
@@ -448,9 +478,10 @@ __global__ __launch_bounds__(256, 4) void bt_chunk_prep_kernel(const float* __re
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const size_t off = (hv * C + 16 * tt + 4 * lk + i) * HD + col;
-        o.w[off] = dw[i];
-        o.u[off] = du[i];
+        const int t = 16 * tt + 4 * lk + i;
+        const size_t off = (hv * C + t) * HD + col;
+        o.w[off] = t < nan_w ? dw[i] : __builtin_nanf("");
+        o.u[off] = t < nan_u ? du[i] : __builtin_nanf("");
       }
     }
   }
@@ -547,6 +578,17 @@ __global__ __launch_bounds__(64) void bt_chunk_scan_kernel(const float* __restri
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
       for (int r = 0; r < 4; ++r) yy[tt][r] *= ge[tt][r];
+    const int nan0 = take_non_finite(d, lk);
+    if (__builtin_amdgcn_ballot_w64(nan0 < C)) {  // the column's tokens from nan0 on, and its state
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * tt + 4 * lk + r >= nan0) yy[tt][r] = __builtin_nanf("");
+      if (nan0 < C)
+#pragma unroll
+        for (int J = 0; J < 8; ++J) S[J] = f32x4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       yy[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[0][r], d[0][r], yy[0], 0, 0, 0);
