@@ -84,18 +84,20 @@ __global__ __launch_bounds__(256) void digit_pack_kernel(const float* __restrict
 // N KiB (N <= 4) from g + voff (g wave-uniform, voff = 16·lane and whole KiB) to LDS lds_base + 16·lane:
 // 16 bytes per lane and KiB, without passing through registers.  The compiler does not count these
 // loads: the reader waits with lds_dma_wait before the barrier that publishes them.  m0 holds the LDS
-// base: set and used within one statement that names it as changed, so that nothing comes between.
+// base: one statement sets it, issues the loads and puts its old value back, so that the compiler's use of
+// m0 (it cannot be named as changed) and this one do not meet.
 template <int N>
 __device__ __forceinline__ void lds_dma(const void* g, unsigned voff, unsigned lds_base) {
   static_assert(N == 1 || N == 4, "the instruction offset holds three KiB");
+  unsigned old;
   if constexpr (N == 1)
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(g), "s"(lds_base)
-                 : "memory", "m0");
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(old) : "v"(voff), "s"(g), "s"(lds_base) : "memory");
   else
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\t"
-                 "global_load_lds_dwordx4 %0, %1 offset:1024\n\tglobal_load_lds_dwordx4 %0, %1 offset:2048\n\t"
-                 "global_load_lds_dwordx4 %0, %1 offset:3072" ::"v"(voff), "s"(g), "s"(lds_base)
-                 : "memory", "m0");
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:1024\n\tglobal_load_lds_dwordx4 %1, %2 offset:2048\n\t"
+                 "global_load_lds_dwordx4 %1, %2 offset:3072\n\ts_mov_b32 m0, %0"
+                 : "=&s"(old) : "v"(voff), "s"(g), "s"(lds_base) : "memory");
 }
 __device__ __forceinline__ void lds_dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
