@@ -6,16 +6,20 @@
 // is scale · Σ ±x.  The signs are f4 (e2m1) operands, ±1 exactly.  An activation is a fixed-point
 // number of six balanced base-32 digits relative to its block of 32 columns: with 2^e > max|x| >=
 // 2^(e-1) over the block, v = x · 2^(4-e) lies in [-16, 16] and
-//   v = d0 + d1/32 + ... + d5/32^5 + rest,   |d_i| <= 16 whole, |rest| <= 2^-26
+//   v = d0 + d1/32 + ... + d5/32^5 + rest,   |d_i| <= 16 whole, |rest| <= 2^-26 (at most 2^-29 of the largest v)
 // An integer d of that range is an f6 (e2m3) value in units of 1/8 exactly (codes 0..16 of the
 // magnitude are the integers 0..16), and the power of two of a digit is the block scale (e8m0) of
 // the matrix instruction.  v_mfma_scale_f32_16x16x128_f8f6f4 therefore sums 128 exact products per
 // digit into an f32 accumulator; digits go in from the smallest to the largest, then the group's sum
 // is multiplied by the f16 scale as it is added (one fma per group, where a three-part f16 split of
-// the activations takes twelve f32 additions per group).  The six digits carry every bit of an f32
-// whose exponent is within 6 of its block's largest and 2^-30 of the block's largest beside that,
-// beneath the rounding of an f32 dot product.  A block that holds an infinity or a NaN gets the NaN
-// scale (0xFF), so its token's results are NaN.
+// the activations takes twelve f32 additions per group).  Six digits carry every bit of an f32 whose
+// exponent is within 5 of its block's largest; smaller values are rounded to a grid of 2^-29 of the
+// block's largest, beneath the rounding of an f32 dot product.  Errors of a 2048 x 5120 product against 64
+// bits (2-norm; n = 2, 8 and 128 columns) with three f16 parts and with digits:
+//   standard normal columns                            1.6e-7  1.6e-7  2.2e-7    0.8e-7  0.9e-7  0.8e-7
+//   normal · e^(3 normal)                              1.7e-7  2.0e-7  2.1e-7    0.8e-7  0.8e-7  0.9e-7
+//   two of about 2^14 that cancel in every group       2.2e-4  2.2e-4  2.6e-4    0.8e-7  2.5e-4  2.5e-4
+// A block that holds an infinity or a NaN gets the NaN scale (0xFF), so its token's results are NaN.
 //
 // Rate.  The instruction runs at four times the f16 rate (measured 9.1 ns per 16x16x128 per SIMD,
 // 7.4 PFLOP/s over the device); six of them replace the twelve f16 ones (4 steps of 32 columns x 3
@@ -46,13 +50,15 @@ __device__ __forceinline__ void expand_f4(unsigned w, i32x8& a) {
 }
 
 // Digit 0's block scale of a block whose largest |value| has the bits mb, and the exponent e its values are
-// taken by (v = x · 2^(4-e)).  The scales go down to digit 5's, 25 below digit 0's, and have to stay block
-// scales (>= 0): a block whose largest value is below 2^-102 is held to 2^-131 absolute.
+// taken by (v = x · 2^(4-e)).  The scales go down to the last of the D digits', 5 (D - 1) below digit 0's,
+// and have to stay block scales (>= 0): a block whose largest value is below 2^(5D - 132) is held to 2^-131 absolute.
+template <int D>
 __device__ __forceinline__ unsigned digit_scale(unsigned mb, int& e) {
+  constexpr int lo = 5 * (D - 1) - 126;
   e = 0;
   if (mb >= 0x7F800000u) return 0xFFu;  // an infinity or a NaN in the block
   (void)frexpf(__builtin_bit_cast(float, mb), &e);
-  e = mb == 0 ? 0 : (e < -101 ? -101 : e);
+  e = mb == 0 ? 0 : (e < lo ? lo : e);
   return (unsigned)(126 + e);
 }
 
@@ -65,7 +71,7 @@ __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)
     mb = b > mb ? b : mb;
   }
   int e;
-  const unsigned b0 = digit_scale(mb, e);
+  const unsigned b0 = digit_scale<kDigits>(mb, e);
   const bool finite = b0 != 0xFFu;
   f32x16 a, b;
 #pragma unroll
@@ -95,12 +101,13 @@ __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)
 // The 16 rows of the token operand hold T tokens x P = 16/T digits (row ρ = p·T + token, digit f·P + p of
 // operand f), so a group of 128 columns takes F operands and F matrix instructions per 16 weight rows:
 //   n <= 2: T = 2, P = 8, F = 1;  n <= 4: T = 4, P = 4, F = 2;  n <= 8: T = 8, P = 2, F = 3;  else T = 16, F = 6
-// (slots past the six digits hold zeros).  A weight row's sums of the slots are kept apart until the end and
-// then added.
+// The first two have room for eight digits and hold eight (activations to 2^-39 of their block's largest), the others
+// six.  A weight row's sums of the slots are kept apart until the end and then added.
 template <int T>
 struct FewForm {
   static constexpr int P = 16 / T;
   static constexpr int F = (kDigits + P - 1) / P;
+  static constexpr int D = F * P;  // digits
   // LDS of a tile: [group][operand][block q: 416 B][row ρ: 24 B], the block and group strides chosen so that the
   // 2-byte writes of the packing (16 blocks x 4 quarters at once) meet few banks twice
   static constexpr int kBlk = 16 * 24 + 32;
@@ -109,9 +116,6 @@ struct FewForm {
   static constexpr int kEx = 4 * kGrp;                            // the block scales: [lane] a byte per group
   static constexpr int kTile = kEx + 256;
 };
-// How far the block scale of slot p of an operand lies below digit 0's (slots past the six digits hold zeros and
-// take the last digit's).
-__host__ __device__ constexpr int slot_drop(int p) { return 5 * (p < kDigits ? p : kDigits - 1); }
 constexpr int kFewStage = 16 * 36 * 4;  // a wave's 512 staged columns, blocks of 32 padded to 36
 
 template <int CTRL>
@@ -122,8 +126,8 @@ __device__ __forceinline__ unsigned dpp_umax(unsigned v) {
 
 // One wave's 512 columns of a token (lane: columns 4·lane and 256 + 4·lane as x0, x1; st the wave's staging
 // area) split into digits: lane (block blk = lane >> 2, quarter kq) takes columns 4j + kq of its block, elements
-// 8kq .. 8kq + 7 of a digit operand: 48 bits, handed to put(digit, lo, hi) for every slot of form T (zero past
-// the six digits).  Returns digit 0's block scale.
+// 8kq .. 8kq + 7 of a digit operand: 48 bits, handed to put(digit, lo, hi).  Returns digit 0's block scale (slot p
+// of an operand lies 5p below its slot 0).
 template <int T, class Put>
 __device__ __forceinline__ unsigned few_digits(float* st, unsigned lane, float4 x0, float4 x1, Put&& put) {
   using FF = FewForm<T>;
@@ -144,27 +148,22 @@ __device__ __forceinline__ unsigned few_digits(float* st, unsigned lane, float4 
   mb = dpp_umax<0xB1>(mb);  // the block's four quarters: quad xor 1, xor 2
   mb = dpp_umax<0x4E>(mb);
   int e;
-  const unsigned b0 = digit_scale(mb, e);
+  const unsigned b0 = digit_scale<FF::D>(mb, e);
   const int sh = 4 - e;
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[j] = b0 != 0xFFu ? ldexpf(v[j], sh) : 0.f;
   f32x16 ra = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, rb = ra;
 #pragma unroll
-  for (int k = 0; k < FF::F * FF::P; ++k) {
-    unsigned lo = 0, hi = 0;
-    if (k < kDigits) {
+  for (int k = 0; k < FF::D; ++k) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float r = __builtin_rintf(v[j]);
-        v[j] = (v[j] - r) * 32.0f;
-        if (j & 1) rb[j >> 1] = r;
-        else ra[j >> 1] = r;
-      }
-      const u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
-      lo = d[0];
-      hi = d[1];
+    for (int j = 0; j < 8; ++j) {
+      const float r = __builtin_rintf(v[j]);
+      v[j] = (v[j] - r) * 32.0f;
+      if (j & 1) rb[j >> 1] = r;
+      else ra[j >> 1] = r;
     }
-    put(k, lo, hi);
+    const u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
+    put(k, d[0], d[1]);
   }
   return b0;
 }
@@ -183,19 +182,19 @@ __device__ __forceinline__ void few_pack(unsigned char* tile, float* st, unsigne
   });
   if (kq == 0) {
 #pragma unroll
-    for (int p = 0; p < FF::P; ++p) tile[FF::kEx + 4 * (16 * q + p * T + tok) + g] = (unsigned char)(b0 - slot_drop(p));
+    for (int p = 0; p < FF::P; ++p) tile[FF::kEx + 4 * (16 * q + p * T + tok) + g] = (unsigned char)(b0 - 5 * p);
   }
 }
 
 // The same into a tile in global memory (layout FewForm<T>), for kernels that hand their results to a product:
-// rec is FF::F·FF::P·384 bytes of the wave's LDS, from which the 24-byte pieces go out as 8-byte words.
+// rec is FF::D·384 bytes of the wave's LDS, from which the 24-byte pieces go out as 8-byte words.
 template <int T>
-__host__ __device__ constexpr int few_rec() { return FewForm<T>::F * FewForm<T>::P * 384; }
+__host__ __device__ constexpr int few_rec() { return FewForm<T>::D * 384; }
 template <int T>
 __device__ __forceinline__ void few_pack_out(uint8_t* __restrict__ tile, unsigned char* rec, float* st, unsigned lane, int tok,
                                              float4 x0, float4 x1) {
   using FF = FewForm<T>;
-  constexpr int W = FF::F * FF::P * 48;  // 8-byte words
+  constexpr int W = FF::D * 48;  // 8-byte words
   const unsigned b0 = few_digits<T>(st, lane, x0, x1, [&](int k, unsigned lo, unsigned hi) {
     unsigned short* w = reinterpret_cast<unsigned short*>(rec + 384 * k + 6 * lane);  // [digit][block][24 B]
     w[0] = (unsigned short)lo;
@@ -215,7 +214,7 @@ __device__ __forceinline__ void few_pack_out(uint8_t* __restrict__ tile, unsigne
   if ((lane & 3u) == 0) {
 #pragma unroll
     for (int p = 0; p < FF::P; ++p)
-      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - slot_drop(p));
+      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - 5 * p);
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -241,9 +240,8 @@ template <int T>
 __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lane, unsigned psel, const FewUnit& u, f32x4 (&acc)[4]) {
   using FF = FewForm<T>;
   const unsigned ex = *reinterpret_cast<const unsigned*>(tile + FF::kEx + 4 * lane);
-  // operand f's slots: P digits further down than operand f - 1's, where there are that many (T = 4: the second
-  // operand's slots 2 and 3, rows 8 and up, hold zeros, and a scale that ran below 0 would borrow from its neighbour)
-  const unsigned drop = T == 4 && (lane & 8u) ? 0u : 0x05050505u * (unsigned)FF::P;
+  // operand f's slots: P digits further down than operand f - 1's (no borrow: digit 0's scales are >= 5 (D - 1))
+  constexpr unsigned drop = 0x05050505u * (unsigned)FF::P;
   const unsigned char* fl = tile + (lane >> 4) * FF::kBlk + 24 * (lane & 15u);
 #pragma unroll
   for (int g = 0; g < 4; ++g) {

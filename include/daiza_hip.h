@@ -88,10 +88,12 @@ int dz_q1_0_matvec(dz_mat* m, const float* x, float* y, int accumulate);
 int dz_q1_0_matvec_multi(dz_mat* const* mats, int n, const float* x, float* const* ys);
 
 /* n columns at once: y[i] = W x[i] (accumulate = 0) or y[i] += W x[i] for i < n; host x[n][cols],
- * y[n][rows].  Runs on the matrix cores with the activations split into three f16 parts (33
- * significant bits: f32 width) and exact ±scale weights, so it agrees with an f32 dot product to
- * within f32 accumulation order.  Replaces matvec_batch_into_slice / matvec_add_batch_into_slice
- * (weights.rs:475-682, 976-980). */
+ * y[n][rows].  Runs on the matrix cores with exact ±scale weights and the activations as digits of a
+ * fixed-point number per 32 columns: values within 5 powers of two of the largest of their 32 keep every bit, smaller
+ * ones are held to 2^-29 of it (2^-39 for n <= 4), beneath the rounding of an f32 dot product, with which it
+ * agrees to within f32 accumulation order.  A column with an infinity or a NaN gives NaN, and no other is
+ * touched.  Replaces matvec_batch_into_slice / matvec_add_batch_into_slice (weights.rs:475-682,
+ * 976-980).  dz_forward_batch and dz_verify_forward take their products the same way. */
 int dz_q1_0_matvec_batch(dz_mat* m, const float* x, int n, float* y, int accumulate);
 
 /* Same as dz_q1_0_matvec on device pointers, enqueued on `stream` (a hipStream_t, NULL = default),

@@ -3,7 +3,7 @@ its tiles, against float64; and the forward that hands its activations over as d
 the oracle.
 
 Bound of the product: the sums of a group's digits and of the groups are f32 additions of partial sums, at most
-(8 + ngroups) per slot and 8 between the slots and splits, and the digits keep 2^-29 of their 32-column block's
+(8 + ngroups) per slot and 8 between the slots and splits, and the digits keep 2^-29 (n <= 4: 2^-39) of their 32-column block's
 largest value: |err| <= (ngroups + 24) 2^-24 Σ|w x| + 2^-29 Σ|w| max|x|.
 """
 import numpy as np
@@ -43,6 +43,25 @@ def test_forms(dz, n, rows, cols):
     ya = y0.copy()
     m.matvec_add_batch_into_slice(x, n, ya)
     assert np.all(np.abs(ya - (y0 + ref)) <= bound + 2.0 ** -23 * (np.abs(y0) + np.abs(ya)))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_small_values_beside_large_ones(dz, n):
+    """Up to four columns, an f32 ten powers of two below the largest of its block comes through with every bit:
+    two values 2^10 that cancel in the row, and one with its lowest significand bits set beside them."""
+    rows, cols = 64, 256
+    rng = np.random.default_rng(n)
+    blk = np.empty((rows, cols // 128, 18), np.uint8)
+    blk[:, :, 2:] = rng.integers(0, 256, (rows, cols // 128, 16), dtype=np.uint8)
+    blk[:, :, 0], blk[:, :, 1] = 0x00, 0x3C  # f16 1.0
+    blk[:, :, 2] = blk[:, :, 2] & 0xFC | 1   # column 0 of a group is +, column 1 is -
+    m = dz.Q1_0Matrix(blk.reshape(-1), rows, cols)
+    v = (1 + (rng.integers(0, 1 << 23, n) | 3) / 2.0 ** 23).astype(np.float32)
+    x = np.zeros((n, cols), np.float32)
+    x[:, 128] = x[:, 129] = 2.0 ** 10
+    x[:, 128 + 21] = v
+    sign = ((blk[:, 1, 2 + 21 // 8] >> (21 % 8)) & 1).astype(np.float32) * 2 - 1
+    assert np.array_equal(m.matvec_batch(x), sign[None] * v[:, None])
 
 
 def test_non_finite_token(dz):
