@@ -1071,7 +1071,6 @@ struct FewOut {
 };
 template <int T>
 __device__ __forceinline__ void few_out(const FewOut<T>& o, float4 x0, float4 x1) {
-  __shared__ __align__(16) unsigned char rec[few_rec<T>()];
   __shared__ __align__(16) float st[kFewStage / 4];
   const unsigned lane = threadIdx.x;
   const int t = blockIdx.x, tok = blockIdx.y;
@@ -1085,7 +1084,8 @@ __device__ __forceinline__ void few_out(const FewOut<T>& o, float4 x0, float4 x1
     x0 = make_float4(x0.x * w0.x, x0.y * w0.y, x0.z * w0.z, x0.w * w0.w);
     x1 = make_float4(x1.x * w1.x, x1.y * w1.y, x1.z * w1.z, x1.w * w1.w);
   }
-  few_pack_out<T>(o.dig + (size_t)t * FewForm<T>::kTile, rec, st, lane, tok, x0, x1);
+  few_stage(st, lane, x0, x1);
+  few_pack<T>(o.dig + (size_t)t * FewForm<T>::kTile, st, lane, tok);
 }
 
 // out[m] = Σ_z p[m][z·stride] for z < n in split order (four consecutive columns each), N splits of all M sums in

@@ -109,7 +109,7 @@ struct FewForm {
   static constexpr int F = (kDigits + P - 1) / P;
   static constexpr int D = F * P;  // digits
   // LDS of a tile: [group][operand][block q: 416 B][row ρ: 24 B], the block and group strides chosen so that the
-  // 2-byte writes of the packing (16 blocks x 4 quarters at once) meet few banks twice
+  // writes of the packing (16 blocks at once) meet few banks twice
   static constexpr int kBlk = 16 * 24 + 32;
   static constexpr int kOp = 4 * kBlk;
   static constexpr int kGrp = F * kOp + 32;
@@ -124,16 +124,27 @@ __device__ __forceinline__ unsigned dpp_umax(unsigned v) {
   return o > v ? o : v;
 }
 
-// One wave's 512 columns of a token (lane: columns 4·lane and 256 + 4·lane as x0, x1; st the wave's staging
-// area) split into digits: lane (block blk = lane >> 2, quarter kq) takes columns 4j + kq of its block, elements
-// 8kq .. 8kq + 7 of a digit operand: 48 bits, handed to put(digit, lo, hi).  Returns digit 0's block scale (slot p
-// of an operand lies 5p below its slot 0).
-template <int T, class Put>
-__device__ __forceinline__ unsigned few_digits(float* st, unsigned lane, float4 x0, float4 x1, Put&& put) {
-  using FF = FewForm<T>;
+// A wave's 512 columns of a token (lane: columns 4·lane and 256 + 4·lane as x0, x1) to the staging area st.
+__device__ __forceinline__ void few_stage(float* st, unsigned lane, float4 x0, float4 x1) {
   *reinterpret_cast<float4*>(st + 36 * (lane >> 3) + 4 * (lane & 7u)) = x0;
   *reinterpret_cast<float4*>(st + 36 * (8 + (lane >> 3)) + 4 * (lane & 7u)) = x1;
   __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
+}
+
+// The value of the next lane of the quad (the last one's own).
+__device__ __forceinline__ unsigned dpp_next(unsigned v) {
+  return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xF9, 0xF, 0xF, false);  // quad_perm [1,2,3,3]
+}
+
+// 512 staged columns split into digits: lane (block blk = lane >> 2, quarter kq) takes columns 4j + kq of its block, elements
+// 8kq .. 8kq + 7 of a digit operand: 48 bits.  A block's 24 bytes of a digit leave as three aligned 8-byte pieces,
+// each formed with the next lane's bits: put(digit, piece), of which piece kq of the block is lane kq's (kq < 3).
+// Returns digit 0's block scale (slot p of an operand lies 5p below its slot 0).
+// The packing is a chain of a wave (about 1700 cycles).  Written in parts of 16 and 32 bits at byte 6·kq, misaligned for
+// half the lanes, the digits bound the CU's LDS: 2450 cycles per task and wave with four waves packing, 1960 with pieces.
+template <int T, class Put>
+__device__ __forceinline__ unsigned few_digits(const float* st, unsigned lane, Put&& put) {
+  using FF = FewForm<T>;
   const unsigned blk = lane >> 2, kq = lane & 3u;
   float v[8];
 #pragma unroll
@@ -149,36 +160,46 @@ __device__ __forceinline__ unsigned few_digits(float* st, unsigned lane, float4 
   mb = dpp_umax<0x4E>(mb);
   int e;
   const unsigned b0 = digit_scale<FF::D>(mb, e);
-  const int sh = 4 - e;
+  // 2^(4-e); 0 for a block that is not finite (its digits do not matter beside the NaN scale, but are formed)
+  const float up = __builtin_bit_cast(float, (unsigned)(131 - e) << 23);
+  const bool finite = b0 != 0xFFu;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = b0 != 0xFFu ? ldexpf(v[j], sh) : 0.f;
-  f32x16 ra = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, rb = ra;
+  for (int j = 0; j < 8; ++j) v[j] = finite ? v[j] * up : 0.f;
 #pragma unroll
-  for (int k = 0; k < FF::D; ++k) {
+  for (int k0 = 0; k0 < FF::D; k0 += 4) {
+    // digit k0 + i takes elements 8i .. 8i + 7 of the conversion: element 2m is ra[m], 2m + 1 is rb[m]
+    f32x16 ra = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, rb = ra;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float r = __builtin_rintf(v[j]);
-      v[j] = (v[j] - r) * 32.0f;
-      if (j & 1) rb[j >> 1] = r;
-      else ra[j >> 1] = r;
-    }
+    for (int i = 0; i < 4 && k0 + i < FF::D; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        // the nearest whole number of v·32^k (|.| <= 16): what adding 3·2^22 leaves
+        const float r = __builtin_fmaf(v[j], (float)(1ull << (5 * (k0 + i))), 12582912.f) - 12582912.f;
+        v[j] = __builtin_fmaf(r, -1.0f / (float)(1ull << (5 * (k0 + i))), v[j]);
+        if (j & 1) rb[4 * i + (j >> 1)] = r;
+        else ra[4 * i + (j >> 1)] = r;
+      }
     const u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
-    put(k, d[0], d[1]);
+#pragma unroll
+    for (int i = 0; i < 4 && k0 + i < FF::D; ++i) {
+      const int h = 3 * (i >> 1);
+      const unsigned lo = i & 1 ? d[h + 1] >> 16 | d[h + 2] << 16 : d[h], hi = i & 1 ? d[h + 2] >> 16 : d[h + 1] & 0xFFFFu;
+      const unsigned nlo = dpp_next(lo), nhi = dpp_next(hi);
+      const unsigned w1 = hi | nlo << 16, w2 = nlo >> 16 | nhi << 16;  // lo, w1, w2: this lane's and the next one's
+      put(k0 + i, u32x2{kq == 0 ? lo : kq == 1 ? lo >> 16 | w1 << 16 : w1, kq == 0 ? w1 : kq == 1 ? w1 >> 16 | w2 << 16 : w2});
+    }
   }
   return b0;
 }
 
-// Packs the wave's 512 columns of token tok into the LDS tile.
+// Packs the 512 staged columns of token tok into the LDS tile.
 template <int T>
-__device__ __forceinline__ void few_pack(unsigned char* tile, float* st, unsigned lane, int tok, float4 x0, float4 x1) {
+__device__ __forceinline__ void few_pack(unsigned char* tile, const float* st, unsigned lane, int tok) {
   using FF = FewForm<T>;
   const unsigned g = lane >> 4, q = (lane >> 2) & 3u, kq = lane & 3u;
-  unsigned char* o = tile + g * FF::kGrp + q * FF::kBlk + 6 * kq;
-  const unsigned b0 = few_digits<T>(st, lane, x0, x1, [&](int k, unsigned lo, unsigned hi) {
-    unsigned short* w = reinterpret_cast<unsigned short*>(o + (k / FF::P) * FF::kOp + 24 * ((k % FF::P) * T + tok));
-    w[0] = (unsigned short)lo;
-    w[1] = (unsigned short)(lo >> 16);
-    w[2] = (unsigned short)hi;
+  unsigned char* o = tile + g * FF::kGrp + q * FF::kBlk + 24 * tok + 8 * kq;
+  const unsigned b0 = few_digits<T>(st, lane, [&](int k, u32x2 piece) {
+    if (kq < 3) *reinterpret_cast<u32x2*>(o + (k / FF::P) * FF::kOp + 24 * (k % FF::P) * T) = piece;
   });
   if (kq == 0) {
 #pragma unroll
@@ -186,90 +207,73 @@ __device__ __forceinline__ void few_pack(unsigned char* tile, float* st, unsigne
   }
 }
 
-// The same into a tile in global memory (layout FewForm<T>), for kernels that hand their results to a product:
-// rec is FF::D·384 bytes of the wave's LDS, from which the 24-byte pieces go out as 8-byte words.
-template <int T>
-__host__ __device__ constexpr int few_rec() { return FewForm<T>::D * 384; }
-template <int T>
-__device__ __forceinline__ void few_pack_out(uint8_t* __restrict__ tile, unsigned char* rec, float* st, unsigned lane, int tok,
-                                             float4 x0, float4 x1) {
-  using FF = FewForm<T>;
-  constexpr int W = FF::D * 48;  // 8-byte words
-  const unsigned b0 = few_digits<T>(st, lane, x0, x1, [&](int k, unsigned lo, unsigned hi) {
-    unsigned short* w = reinterpret_cast<unsigned short*>(rec + 384 * k + 6 * lane);  // [digit][block][24 B]
-    w[0] = (unsigned short)lo;
-    w[1] = (unsigned short)(lo >> 16);
-    w[2] = (unsigned short)hi;
-  });
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int i = 0; i < (W + 63) / 64; ++i) {
-    const int w = 64 * i + (int)lane;
-    if (W % 64 == 0 || w < W) {
-      const int k = w / 48, blk = (w % 48) / 3, part = w % 3;
-      *reinterpret_cast<u32x2*>(tile + (blk >> 2) * FF::kGrp + (k / FF::P) * FF::kOp + (blk & 3) * FF::kBlk +
-                                24 * ((k % FF::P) * T + tok) + 8 * part) = *reinterpret_cast<const u32x2*>(rec + 8 * w);
-    }
-  }
-  if ((lane & 3u) == 0) {
-#pragma unroll
-    for (int p = 0; p < FF::P; ++p)
-      tile[FF::kEx + 4 * (16 * ((lane >> 2) & 3u) + p * T + tok) + (lane >> 4)] = (uint8_t)(b0 - 5 * p);
-  }
-  __builtin_amdgcn_wave_barrier();
-}
-
-// A unit's weights in a wave: the signs of (16-row block sb, group g) and the rows' four scales.
+// A unit's weights in a wave: the signs of (16-row block sb0 + sb, group g) and the rows' four scales.  A wave takes the
+// four 16-row blocks of a row-block (SB = 4, sb0 = 0) or two of them (SB = 2, sb0 = 0 or 2).
+template <int SB>
 struct FewUnit {
-  unsigned s[4][4];  // [g][sb]
-  u32x2 sc[4];
+  unsigned s[4][SB];  // [g][sb]
+  u32x2 sc[SB];
 };
-__device__ __forceinline__ void few_load(const __amdgpu_buffer_rsrc_t& wr, int woff, int soff, int unit, FewUnit& u) {
+template <int SB>
+__device__ __forceinline__ void few_load(const __amdgpu_buffer_rsrc_t& wr, int woff, int soff, int unit, int sb0, FewUnit<SB>& u) {
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-      u.s[g][sb] = __builtin_amdgcn_raw_buffer_load_b32(wr, woff, unit + 1024 * (g ^ sb) + 256 * sb, 0);
+    for (int sb = 0; sb < SB; ++sb)
+      u.s[g][sb] = __builtin_amdgcn_raw_buffer_load_b32(wr, woff, unit + 1024 * (g ^ (sb0 + sb)) + 256 * (sb0 + sb), 0);
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb)
-    u.sc[sb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, soff, unit + 128 * sb, 0));
+  for (int sb = 0; sb < SB; ++sb)
+    u.sc[sb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, soff, unit + 128 * (sb0 + sb), 0));
 }
 
-// acc[sb] += the unit's products with the tile's digits: slot rows 4q + i of weight row 16·sb + r.
-template <int T>
-__device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lane, unsigned psel, const FewUnit& u, f32x4 (&acc)[4]) {
+// acc[sb] += the unit's products with the tile's digits: slot rows 4q + i of weight row 16·(sb0 + sb) + r.
+template <int T, int SB>
+__device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lane, unsigned psel, int sb0, const FewUnit<SB>& u,
+                                         f32x4 (&acc)[SB]) {
   using FF = FewForm<T>;
   const unsigned ex = *reinterpret_cast<const unsigned*>(tile + FF::kEx + 4 * lane);
   // operand f's slots: P digits further down than operand f - 1's (no borrow: digit 0's scales are >= 5 (D - 1))
   constexpr unsigned drop = 0x05050505u * (unsigned)FF::P;
   const unsigned char* fl = tile + (lane >> 4) * FF::kBlk + 24 * (lane & 15u);
+  // step i: operand F - 1 - i % F of group i / F.  Its digits are read a step before the matrix instructions that use
+  // them: read where they are used, every step waited out the LDS (one wave per SIMD; T = 16, four instructions per
+  // step: 4900 cycles a unit, with the reads ahead 3600)
+  constexpr int STEPS = 4 * FF::F;
+  auto read = [&](int i) {
+    const u32x2* p = reinterpret_cast<const u32x2*>(fl + (i / FF::F) * FF::kGrp + (FF::F - 1 - i % FF::F) * FF::kOp);
+    const u32x2 p0 = p[0], p1 = p[1], p2 = p[2];
+    return i32x8{(int)p0.x, (int)p0.y, (int)p1.x, (int)p1.y, (int)p2.x, (int)p2.y, 0, 0};
+  };
+  i32x8 a = read(0), b[SB];
+  f32x4 d[SB];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    i32x8 b[4];
+  for (int i = 0; i < STEPS; ++i) {
+    const int g = i / FF::F, f = FF::F - 1 - i % FF::F;
+    const i32x8 an = i + 1 < STEPS ? read(i + 1) : a;
+    __builtin_amdgcn_sched_barrier(0);
+    if (f == FF::F - 1) {
 #pragma unroll
-    for (int sb = 0; sb < 4; ++sb) expand_f4(__builtin_amdgcn_perm(u.s[g][sb], u.s[g][sb], psel), b[sb]);
-    f32x4 d[4];
-#pragma unroll
-    for (int f = FF::F - 1; f >= 0; --f) {
-      const u32x2* p = reinterpret_cast<const u32x2*>(fl + g * FF::kGrp + f * FF::kOp);
-      const u32x2 p0 = p[0], p1 = p[1], p2 = p[2];
-      const i32x8 a = {(int)p0.x, (int)p0.y, (int)p1.x, (int)p1.y, (int)p2.x, (int)p2.y, 0, 0};
-      const int sx = (int)(ex - drop * (unsigned)f);
-#pragma unroll
-      for (int sb = 0; sb < 4; ++sb) {
-        const f32x4 c = f == FF::F - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
-        if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, kSignScale);
-        else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, kSignScale);
-        else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, kSignScale);
-        else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, kSignScale);
-      }
+      for (int sb = 0; sb < SB; ++sb) expand_f4(__builtin_amdgcn_perm(u.s[g][sb], u.s[g][sb], psel), b[sb]);
     }
+    const int sx = (int)(ex - drop * (unsigned)f);
 #pragma unroll
-    for (int sb = 0; sb < 4; ++sb) {
-      const unsigned slot = (unsigned)(g ^ sb), two = u.sc[sb][slot >> 1];
-      const float sf = (float)__builtin_bit_cast(_Float16, (unsigned short)(slot & 1 ? two >> 16 : two & 0xFFFFu));
+    for (int sb = 0; sb < SB; ++sb) {
+      const f32x4 c = f == FF::F - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
+      if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, kSignScale);
+      else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, kSignScale);
+      else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, kSignScale);
+      else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, kSignScale);
+    }
+    a = an;
+    if (f == 0) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) acc[sb][v] = __builtin_fmaf(sf, d[sb][v], acc[sb][v]);
+      for (int sb = 0; sb < SB; ++sb) {
+        const unsigned slot = (unsigned)(g ^ (sb0 + sb));
+        const unsigned h = (unsigned)(__builtin_bit_cast(unsigned long long, u.sc[sb]) >> (16 * slot));
+        const float sf = (float)__builtin_bit_cast(_Float16, (unsigned short)h);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[sb][v] = __builtin_fmaf(sf, d[sb][v], acc[sb][v]);
+      }
     }
   }
 }
@@ -311,17 +315,22 @@ struct FewX {
   int ssq_ld;
   float eps;
 };
+// Packing tasks of a wave whose inputs are requested and staged at once.  Requested one by one behind the weights, each
+// task waited a memory round trip: 3300 cycles per task (64 x 128 by 16: four tasks a wave, 8.8 us the launch).
 template <int T>
+constexpr int kFewAhead = T <= 4 ? 1 : 2;
+// (a packed product's tiles come as they are and need no staging area)
+template <int T, bool PRE>
 __host__ __device__ constexpr size_t few_shmem(int nw, int tps) {
-  return (size_t)tps * FewForm<T>::kTile + (size_t)nw * kFewStage;
+  return (size_t)tps * FewForm<T>::kTile + (PRE ? 0 : (size_t)nw * kFewAhead<T> * kFewStage);
 }
 // K tiles of a workgroup (its LDS)
 constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
 
-// Grid (ceil(nrb / NW), splits, blocks of 16 tokens), 64·NW threads: workgroup (chunk, z) takes K tiles [z·tps, min(ntiles, (z+1)·tps))
-// of NW row-blocks, one per wave.  The inputs are requested first, the first unit's weights behind them, and the
-// packing runs while the weights arrive; one barrier, then every wave goes its own way.  With more than one
-// split, workgroup z writes its partial to y + z·zstride.
+// Grid (ceil(nrb / RB), splits, blocks of 16 tokens), 64·NW threads: workgroup (chunk, z) takes K tiles [z·tps, min(ntiles, (z+1)·tps))
+// of RB row-blocks, one per wave, or two waves to a row-block (RB = NW / 2).  The inputs are requested first, the first unit's
+// weights behind them, and the packing runs while the weights arrive; one barrier, then every wave goes its own way.  With more
+// than one split, workgroup z writes its partial to y + z·zstride.
 // At eight tokens a product is bound by latencies: of 34816 x 5120's 15.2 us (packed tiles) about 7 are launch, digits
 // and the stores of the partials, 5 the weights (25 MB) and 3 the signs' expansion and the matrix instructions.  The
 // f16 form it replaced (three parts, K tiles packed one by one with a barrier each) against this one with packed
@@ -330,7 +339,7 @@ constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
 //
 // PRE: the digits come packed by the kernel that formed the activations: at eight tokens the packing costs 2 to
 // 4 us of each product.
-template <int T, int NW, bool PRE>
+template <int T, int NW, int RB, bool PRE>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
                                                                      int ntiles, int tps, const FewX x, int n_tok,
                                                                      float* __restrict__ y, int64_t ldy, int64_t zstride,
@@ -344,11 +353,13 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
   const int tb = 16 * (int)blockIdx.z;
   n_tok = min(n_tok - tb, 16);
   const int t0 = (int)blockIdx.y * tps, nt = min(ntiles - t0, tps);
-  const int64_t rb = (int64_t)blockIdx.x * NW + wave;
-  float* st = reinterpret_cast<float*>(smem + (size_t)tps * FF::kTile) + wave * (kFewStage / 4);
-  // packing task i of the wave: (token, tile) number wave + NW·i, tokens first.  The first MT tasks' inputs are
-  // requested before any weights: the CU returns loads in issue order
-  constexpr int MT = 2;
+  constexpr int SB = 4 * RB / NW;  // 16-row blocks of a wave
+  const int64_t rb = (int64_t)blockIdx.x * RB + wave * SB / 4;
+  const int sb0 = wave * SB % 4;
+  constexpr int MT = kFewAhead<T>;
+  float* st = reinterpret_cast<float*>(smem + (size_t)tps * FF::kTile) + wave * (MT * kFewStage / 4);
+  // packing task i of the wave: (token, tile) number wave + NW·i, tokens first.  MT at a time: the first ones' inputs
+  // are requested before any weights (the CU returns loads in issue order) and staged behind a wait for them alone
   const int tasks = n_tok * nt;
   struct In {
     float4 x0, x1, w0, w1;
@@ -381,15 +392,15 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
 #pragma unroll
     for (int i = 0; i < MT; ++i) in[i] = load_x(wave + NW * i);
   }
-  const size_t wbytes = (size_t)(nrb - (int64_t)blockIdx.x * NW) * ntiles * kUnitBytes;
+  const size_t wbytes = (size_t)(nrb - (int64_t)blockIdx.x * RB) * ntiles * kUnitBytes;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(W) + (size_t)blockIdx.x * NW * ntiles * kUnitBytes, 0, (int)(wbytes < 0x7FFFFFFFu ? wbytes : 0x7FFFFFFFu), 0x00027000);
+      const_cast<uint8_t*>(W) + (size_t)blockIdx.x * RB * ntiles * kUnitBytes, 0, (int)(wbytes < 0x7FFFFFFFu ? wbytes : 0x7FFFFFFFu), 0x00027000);
   const int woff = (int)(16u * r + 4u * (q ^ (r >> 2))), soff = kUnitSignBytes + 8 * (int)r;
   const unsigned psel = 0x03020100u ^ (0x01010101u * (r & 3u));
-  const int unit0 = (wave * ntiles + t0) * kUnitBytes;
-  FewUnit u;
-  if (rb < nrb) few_load(wr, woff, soff, unit0, u);
-  auto pack = [&](int k, const In& v) {
+  const int unit0 = (wave * SB / 4 * ntiles + t0) * kUnitBytes;
+  FewUnit<SB> u;
+  if (rb < nrb) few_load(wr, woff, soff, unit0, sb0, u);
+  auto stage = [&](int k, int i, const In& v) {
     const int tok = k % n_tok, t = k / n_tok;
     const int64_t c0 = (int64_t)(t0 + t) * kTileCols + 4 * lane;
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -397,11 +408,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
     if (x.nw) {
       const float s = wave_sum(((x0.x * x0.x + x0.y * x0.y) + (x0.z * x0.z + x0.w * x0.w)) +
                                ((x1.x * x1.x + x1.y * x1.y) + (x1.z * x1.z + x1.w * x1.w)));
-      if (lane == 0) ssqs[t][tok] = s;
+      if (lane == 0 && k < tasks) ssqs[t][tok] = s;
       x0 = make_float4(x0.x * v.w0.x, x0.y * v.w0.y, x0.z * v.w0.z, x0.w * v.w0.w);
       x1 = make_float4(x1.x * v.w1.x, x1.y * v.w1.y, x1.z * v.w1.z, x1.w * v.w1.w);
     }
-    few_pack<T>(smem + (size_t)t * FF::kTile, st, lane, tok, x0, x1);
+    few_stage(st + i * (kFewStage / 4), lane, x0, x1);
   };
   if constexpr (PRE) {
     u32x4* dst = reinterpret_cast<u32x4*>(smem);
@@ -410,12 +421,20 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
       if ((int)tid + 64 * NW * i < pieces) dst[tid + 64 * NW * i] = pc[i];
     for (int i = (int)tid + 64 * NW * MP; i < pieces; i += 64 * NW) dst[i] = psrc[i];
   } else {
-    // (one copy of the packing code, which a call that is alone on the device fetches cold)
+    for (int k0 = wave; k0 < tasks; k0 += MT * NW) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) stage(k0 + NW * i, i, in[i]);
+      if (k0 + MT * NW < tasks) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) in[i] = load_x(k0 + NW * (MT + i));
+      }
+      // (one copy of the packing code, which a call that is alone on the device fetches cold)
 #pragma unroll 1
-    for (int k = wave; k < tasks; k += NW) {
-      pack(k, in[0]);
-      in[0] = in[1];
-      if (k + 2 * NW < tasks) in[1] = load_x(k + 2 * NW);
+      for (int i = 0; i < MT; ++i) {
+        const int k = k0 + NW * i;
+        if (k < tasks) few_pack<T>(smem + (size_t)(k / n_tok) * FF::kTile, st + i * (kFewStage / 4), lane, k % n_tok);
+      }
+      __builtin_amdgcn_wave_barrier();
     }
   }
   lds_barrier();  // the weights stay in flight
@@ -425,19 +444,19 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
     x.ssq[(size_t)blockIdx.y * x.ssq_ld + tb + tid] = s;
   }
   if (rb >= nrb) return;
-  f32x4 acc[4];
+  f32x4 acc[SB];
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb) acc[sb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int sb = 0; sb < SB; ++sb) acc[sb] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int t = 0; t < nt; ++t) {
-    FewUnit nx = u;
-    if (t + 1 < nt) few_load(wr, woff, soff, unit0 + (t + 1) * kUnitBytes, nx);
-    few_unit<T>(smem + (size_t)t * FF::kTile, lane, psel, u, acc);
+    FewUnit<SB> nx = u;
+    if (t + 1 < nt) few_load(wr, woff, soff, unit0 + (t + 1) * kUnitBytes, sb0, nx);
+    few_unit<T>(smem + (size_t)t * FF::kTile, lane, psel, sb0, u, acc);
     u = nx;
   }
   y += (size_t)blockIdx.y * zstride;
   if (gridDim.y > 1) accumulate = 0;
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb) few_slots<T>(acc[sb]);
+  for (int sb = 0; sb < SB; ++sb) few_slots<T>(acc[sb]);
 #pragma unroll
   for (int v = 0; v < (T == 2 ? 2 : 4); ++v) {
     const int tok = T == 2 ? v : (4 * (int)q + v) % T;
@@ -448,10 +467,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const 
       for (int t = 1; t < nt; ++t) s += ssqs[t][tok];
       inv = kSignUp / sqrtf(s / (float)x.K + x.eps);
     }
-    float* yr = y + (size_t)(tb + tok) * ldy + rb * kRowBlock + r;
+    float* yr = y + (size_t)(tb + tok) * ldy + rb * kRowBlock + 16 * sb0 + r;
 #pragma unroll
-    for (int sb = 0; sb < 4; ++sb)
-      if (rb * kRowBlock + 16 * sb + r < rows) {
+    for (int sb = 0; sb < SB; ++sb)
+      if (rb * kRowBlock + 16 * (sb0 + sb) + r < rows) {
         const float val = acc[sb][v] * inv;
         yr[16 * sb] = accumulate ? yr[16 * sb] + val : val;
       }

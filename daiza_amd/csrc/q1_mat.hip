@@ -347,16 +347,18 @@ hipError_t launch_q1_gemm(const Q1Dev& W, const PackedX& p, int n, float* y, int
   return hipGetLastError();
 }
 
-// Launch shape of the few-column product: K tiles per workgroup (so splits) and waves per workgroup.
+// Launch shape of the few-column product: K tiles per workgroup (so splits) and row-blocks per workgroup.
 struct FewPlan {
-  int nw, tps, splits;
+  int rbs, tps, splits;
   unsigned chunks;
 };
 
 // A wave takes one row-block of the workgroup's K tiles, one unit after another, so a product wants its units
 // spread over enough waves (about kFewWaves) and no more splits than that takes: each split adds a pass over
-// partials.  Workgroups that pack their tiles themselves share that over eight waves, unless half of the CUs would
-// be left without one (at eight tokens 16480 x 5120 16.9 against 13.1 us, 5120 x 6144 7.6 against 8.0); with packed
+// partials.  Workgroups that pack their tiles themselves share that over eight waves: of a row-block each, or, where half
+// of the CUs would be left without a workgroup, two to a row-block, which halves a wave's unit and epilogue as well
+// (matvec_batch, us per call, against four waves of a row-block each: 1000 x 1024 by 5 39.0 and 37.7, 200 x 17408 by 12
+// 71.8 and 69.3, 5120 x 6144 by 16 69.4 and 66.8).  With packed
 // tiles four waves spread better (16480 x 5120 9.5 against 10.5, 5120 x 17408 8.9 against 10.0), except in the form of
 // sixteen tokens, where a tile's 40 KiB of digits would be copied for every four row-blocks (a four-layer block's
 // forward of 9 tokens 560 us with four waves, 480 with eight; 16 tokens 591 and 513).
@@ -369,9 +371,9 @@ static FewPlan few_plan(const Q1Dev& W, int n, int T, bool pre) {
   p.tps = (int)std::max<int64_t>(1, (nt + want - 1) / want);
   p.tps = std::min(p.tps, few_max_tiles(T));
   p.splits = (nt + p.tps - 1) / p.tps;
-  if (pre) p.nw = T == 16 ? 8 : 4;
-  else p.nw = 2 * ((W.nrb + 7) / 8 * zb * p.splits) >= device_cus() ? 8 : 4;
-  p.chunks = (unsigned)((W.nrb + p.nw - 1) / p.nw);
+  if (pre) p.rbs = T == 16 ? 8 : 4;
+  else p.rbs = 2 * ((W.nrb + 7) / 8 * zb * p.splits) >= device_cus() ? 8 : 4;
+  p.chunks = (unsigned)((W.nrb + p.rbs - 1) / p.rbs);
   return p;
 }
 // More than 16 columns of a small product go in blocks of 16 through the few-column form: up to one unit per wave of
@@ -382,33 +384,42 @@ static FewPlan few_plan(const Q1Dev& W, int n, int T, bool pre) {
 static bool few_blocks(const Q1Dev& W, int n) { return W.nrb * W.ntiles * ((n + 15) / 16) <= kFewWaves; }
 static int few_form(int n) { return n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16; }
 
-template <int T, int NW, bool PRE>
+template <int T, int NW, int RB, bool PRE>
 static hipError_t launch_few(const FewPlan& p, const Q1Dev& W, const FewX& x, int n, float* y, int64_t ldy, int64_t zs,
                              int accumulate, hipStream_t s) {
+  const auto kernel = q1_few_kernel<T, NW, RB, PRE>;
   static bool attr = false;
   if (!attr) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(q1_few_kernel<T, NW, PRE>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)few_shmem<T>(NW, few_max_tiles(T)));
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)few_shmem<T, PRE>(NW, few_max_tiles(T)));
     if (e != hipSuccess) return e;
     attr = true;
   }
-  hipLaunchKernelGGL((q1_few_kernel<T, NW, PRE>), dim3(p.chunks, (unsigned)p.splits, (unsigned)((n + 15) / 16)), dim3(64 * NW), few_shmem<T>(NW, p.tps), s,
-                     W.data, W.rows, W.nrb, (int)W.ntiles, p.tps, x, n, y, ldy, zs, accumulate);
+  const size_t sh = few_shmem<T, PRE>(NW, p.tps);
+  hipLaunchKernelGGL(kernel, dim3(p.chunks, (unsigned)p.splits, (unsigned)((n + 15) / 16)), dim3(64 * NW), sh, s, W.data, W.rows, W.nrb,
+                     (int)W.ntiles, p.tps, x, n, y, ldy, zs, accumulate);
   return hipGetLastError();
 }
 
 template <bool PRE>
 static hipError_t launch_few_t(int T, const FewPlan& p, const Q1Dev& W, const FewX& x, int n, float* y, int64_t ldy, int64_t zs,
                                int accumulate, hipStream_t s) {
-#define DZ_FEW(T_) \
-  return p.nw == 8 ? launch_few<T_, 8, PRE>(p, W, x, n, y, ldy, zs, accumulate, s) : launch_few<T_, 4, PRE>(p, W, x, n, y, ldy, zs, accumulate, s)
+  auto go = [&](auto B) {
+    constexpr int T_ = decltype(B)::value;
+    if constexpr (PRE) {
+      constexpr int NW = T_ == 16 ? 8 : 4;
+      return launch_few<T_, NW, NW, true>(p, W, x, n, y, ldy, zs, accumulate, s);
+    } else {
+      return p.rbs == 8 ? launch_few<T_, 8, 8, false>(p, W, x, n, y, ldy, zs, accumulate, s)
+                        : launch_few<T_, 8, 4, false>(p, W, x, n, y, ldy, zs, accumulate, s);
+    }
+  };
   switch (T) {
-    case 2: DZ_FEW(2);
-    case 4: DZ_FEW(4);
-    case 8: DZ_FEW(8);
-    default: DZ_FEW(16);
+    case 2: return go(std::integral_constant<int, 2>{});
+    case 4: return go(std::integral_constant<int, 4>{});
+    case 8: return go(std::integral_constant<int, 8>{});
+    default: return go(std::integral_constant<int, 16>{});
   }
-#undef DZ_FEW
 }
 
 size_t few_tile_bytes(int n) {

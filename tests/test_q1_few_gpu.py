@@ -26,7 +26,8 @@ def _matrix(rng, rows, cols):
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("rows,cols", [(1, 128), (65, 640), (511, 1152), (2100, 512), (70, 17408)])
+@pytest.mark.parametrize("rows,cols", [(1, 128), (65, 640), (511, 1152), (2100, 512), (70, 17408),  # two waves a row-block
+                                       (66100, 256)])  # a wave each (more than half of the CUs have a workgroup)
 def test_forms(dz, n, rows, cols):
     rng = np.random.default_rng(rows * 31 + cols + n)
     aos, w = _matrix(rng, rows, cols)
