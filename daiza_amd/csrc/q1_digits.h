@@ -62,6 +62,16 @@ __device__ __forceinline__ unsigned digit_scale(unsigned mb, int& e) {
   return (unsigned)(126 + e);
 }
 
+// 32 whole numbers of at most 16 as f6 codes: element 2i is ra[i], 2i + 1 is rb[i], each over 8 (code n for n).
+// The conversion writes its result while it still reads its sources, and the compiler does not keep them apart: where
+// the last digit's result took its sources' registers, that digit came out wrong for a wave now and then (2^-26 of
+// the block's largest value, from one run to the next).  The statement below needs all three at once.
+__device__ __forceinline__ u32x6 digit_codes(const f32x16& ra, const f32x16& rb) {
+  u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
+  asm("" : "+v"(d) : "v"(ra), "v"(rb));
+  return d;
+}
+
 // The six digit operands and digit 0's block scale of 32 values (column order).
 __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)[kDigits]) {
   unsigned mb = 0;
@@ -90,8 +100,7 @@ __device__ __forceinline__ unsigned pack_digits(const float (&x)[32], u32x6 (&d)
       a[i] = (a[i] - ra[i]) * 32.0f;
       b[i] = (b[i] - rb[i]) * 32.0f;
     }
-    // element 2i = ra[i], 2i + 1 = rb[i], each over 8: code n for a whole n
-    d[k] = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
+    d[k] = digit_codes(ra, rb);
   }
   return b0;
 }
@@ -179,7 +188,7 @@ __device__ __forceinline__ unsigned few_digits(const float* st, unsigned lane, P
         if (j & 1) rb[4 * i + (j >> 1)] = r;
         else ra[4 * i + (j >> 1)] = r;
       }
-    const u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);
+    const u32x6 d = digit_codes(ra, rb);
 #pragma unroll
     for (int i = 0; i < 4 && k0 + i < FF::D; ++i) {
       const int h = 3 * (i >> 1);
@@ -339,8 +348,10 @@ constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
 //
 // PRE: the digits come packed by the kernel that formed the activations: at eight tokens the packing costs 2 to
 // 4 us of each product.
+// (Registers: about kFewWaves waves run, so a CU rarely holds two of these workgroups; the form of sixteen tokens that
+// packs its own tiles takes a few more than two would leave it.)
 template <int T, int NW, int RB, bool PRE>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 4 : 3) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
+__global__ __launch_bounds__(64 * NW, NW < 8 ? 3 : T == 16 && RB == 8 && !PRE ? 2 : 4) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
                                                                      int ntiles, int tps, const FewX x, int n_tok,
                                                                      float* __restrict__ y, int64_t ldy, int64_t zstride,
                                                                      int accumulate) {
