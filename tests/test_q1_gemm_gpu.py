@@ -2,17 +2,19 @@
 prefill and speculative verify run on the matrix cores.
 
 Bar: every column within 1e-3 normwise relative error of the reference quad kernel
-(quant.rs:614-740) applied to that column, and in practice ~1e-7: the weights are exact f16
-operands and the activations are carried at f32 width (three f16 parts, 33 significant bits), so
-only the f32 accumulation order differs; a full-mantissa input through unit scales comes back bit
-for bit.  Closed forms pin the sign convention and the scale handling independently of the oracle.
-Cases with n <= 16 run the raw form (each K tile packed in LDS with its own scale per token), the
-others the packed form (one scale per token, packed by a separate pass).
+(quant.rs:614-740) applied to that column, and in practice ~1e-7: the signs are exact operands and the
+activations are digits of a fixed-point number per 32 columns (2^-29 of the block's largest value, up
+to four columns 2^-39), beneath the rounding of an f32 sum; a full-mantissa input through unit scales
+comes back bit for bit.  Closed forms pin the sign convention and the scale handling independently of the
+oracle.  Up to 16 columns, and more of a small product, run the few-column form (2, 4, 8 or 16 tokens per
+operand, packed in the LDS of the workgroups that use them), the others the wide form (packed by a pass of
+its own).
 """
 import numpy as np
 import pytest
 
 from conftest import normwise_rel
+from test_q1_wide_gpu import is_wide
 
 pytestmark = pytest.mark.gpu
 
@@ -113,13 +115,14 @@ def test_basis_columns_and_scales(dz, oracle):
         assert np.array_equal(y[i], want), k
 
 
-@pytest.mark.parametrize("n", [1, 5, 8, 9, 16, 17, 40])
+@pytest.mark.parametrize("n", [1, 5, 8, 9, 16, 17, 40, 8200])
 def test_activations_carried_at_f32_width(dz, n):
     """x = v_i e_k with v_i an f32 whose 24-bit significand has its low bits set, through a
     matrix of unit scales: every output is exactly +-v_i, which a product carrying fewer than 24
-    significant bits of the activation (a two-part f16 split keeps 22) would round.  All three
-    forms: paired (n <= 8), raw (9..16), packed (> 16)."""
+    significant bits of the activation (a two-part f16 split keeps 22) would round.  Every form: up to
+    2, 4, 8 and 16 columns, blocks of 16, and tiles."""
     rows, cols = 128, 1024
+    assert is_wide(rows, cols, n) == (n == 8200)
     rng = np.random.default_rng(n)
     blk = np.empty((rows, cols // 128, 18), np.uint8)
     blk[:, :, 2:] = rng.integers(0, 256, (rows, cols // 128, 16), dtype=np.uint8)
@@ -143,7 +146,7 @@ def test_activations_carried_at_f32_width(dz, n):
 
 
 def test_wide_dynamic_range(dz, oracle):
-    # per-token power-of-two scaling: rows of very different magnitude keep their own precision
+    # block scales per token: rows of very different magnitude keep their own precision
     rows, cols = 256, 2048
     aos = oracle.synth_q1_0(SEED, K_GATE, 5, rows, cols)
     m = dz.Q1_0Matrix(aos, rows, cols)
@@ -158,16 +161,17 @@ def test_wide_dynamic_range(dz, oracle):
 
 
 def test_tiles_of_different_magnitude(dz, oracle):
-    # within one token, K tiles 2^20 apart: the raw form scales each tile on its own (n <= 16), the
-    # packed form (n = 17) scales the row; both stay within the bar of the reference
+    # within one token, K tiles 2^20 apart: every block of 32 columns has its own scale, in the forms of two columns,
+    # blocks of 16 and tiles
     rows, cols = 128, 2048
     aos = oracle.synth_q1_0(SEED, K_GATE, 6, rows, cols)
     m = dz.Q1_0Matrix(aos, rows, cols)
-    for n in (2, 17):
+    for n in (2, 17, 4100):
+        assert is_wide(rows, cols, n) == (n == 4100)
         x = _xs(oracle, n, cols, layer=7)
         x[:, :512] *= 1024.0
         x[:, 1536:] *= 1.0 / 1024.0
         y = m.matvec_batch(x)
-        for i in range(n):
+        for i in list(range(min(n, 40))) + [n - 1]:
             ref = oracle.matvec(aos, rows, cols, x[i])
             assert normwise_rel(y[i], ref) < 1e-5, (n, i)
