@@ -1349,8 +1349,8 @@ static hipError_t launch_bt_attn_mfma(int grp, int nkv, int nch, hipStream_t s, 
 }
 
 // Position chunks of the chunk's attention: whole blocks of 16 positions, enough of them that the row
-// tiles of all kv-heads make about kAttnWgs workgroups (one round of the CUs for few tokens, where
-// every workgroup is as long; two where later row tiles see more than earlier ones), at most 256 (the
+// tiles of all kv-heads make about 256 workgroups for few tokens (one round of the CUs, as every workgroup
+// is as long) and 512 for more (later row tiles see more than earlier ones), at most 256 chunks (the
 // merge's bound).  A chunk's records cost a pass of their own, so a prefill whose row tiles fill the
 // device keeps one chunk, which needs none.
 static int bt_attn_mfma_chunks(int n, int grp, int nkv, int ctx_max, int* csz) {
@@ -1544,7 +1544,7 @@ static int bt_forward(dz_ctx* x, const uint32_t* ids, int n, int out_rows, bool 
     if ((rc = bt_gemm(x, l.gate_up, x->bt.h, H, n, l.post_norm, x->bt.ygu, 2 * F, 0, &gd))) return rc;
     if (gd.splits > 1)
       DZ_HIP_CHECK(launch(bt_split_swiglu_kernel, dim3((unsigned)((F + 255) / 256), nb), dim3(256), s, gd.part,
-                          gd.splits, gd.zstride, F, n, x->bt.sw, gd.ssq, gd.ssq_n, gd.ssq_ld, gd.K, gd.eps));
+                          gd.splits, gd.zstride, F, n, x->bt.sw));
     else
       DZ_HIP_CHECK(launch(bt_swiglu_kernel, dim3((unsigned)((F + 255) / 256), nb), dim3(256), s,
                           (const float*)x->bt.ygu, F, n, x->bt.sw));

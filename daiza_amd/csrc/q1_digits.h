@@ -64,7 +64,7 @@ __device__ __forceinline__ unsigned digit_scale(unsigned mb, int& e) {
 
 // 32 whole numbers of at most 16 as f6 codes: element 2i is ra[i], 2i + 1 is rb[i], each over 8 (code n for n).
 // The conversion writes its result while it still reads its sources, and the compiler does not keep them apart: where
-// the last digit's result took its sources' registers, that digit came out wrong for a wave now and then (2^-26 of
+// the last digit's result took its sources' registers, that digit came out wrong for a wave now and then (up to 2^-24 of
 // the block's largest value, from one run to the next).  The statement below needs all three at once.
 __device__ __forceinline__ u32x6 digit_codes(const f32x16& ra, const f32x16& rb) {
   u32x6 d = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(ra, rb, 8.0f);

@@ -797,15 +797,16 @@ int dz_q1_0_matvec_batch(dz_mat* m, const float* x, int n, float* y, int accumul
   int rc = ensure_device();
   if (rc) return rc;
   const size_t K = (size_t)m->d.cols, R = (size_t)m->d.rows;
+  const bool few = n <= 16 || few_blocks(m->d, n);  // the product packs its tiles itself
   PackedX p;
-  if ((rc = packed_x_reserve(g_pack, n, (int64_t)K, &p))) return rc;
+  if (!few && (rc = packed_x_reserve(g_pack, n, (int64_t)K, &p))) return rc;
   if ((rc = g_x.reserve((size_t)n * K * 4)) || (rc = g_y.reserve((size_t)n * R * 4))) return rc;
   hipStream_t s = lib_stream();
   float* xd = static_cast<float*>(g_x.ptr);
   float* yd = static_cast<float*>(g_y.ptr);
   DZ_HIP_CHECK(hipMemcpyAsync(xd, x, (size_t)n * K * 4, hipMemcpyHostToDevice, s));
   if (accumulate) DZ_HIP_CHECK(hipMemcpyAsync(yd, y, (size_t)n * R * 4, hipMemcpyHostToDevice, s));
-  if (n <= 16 || few_blocks(m->d, n)) {  // few tokens: the product packs its tiles itself (as the batched forward does)
+  if (few) {
     DZ_HIP_CHECK(launch_q1_gemm_raw(m->d, xd, (int64_t)K, n, yd, (int64_t)R, accumulate, s, &g_split));
   } else {
     DZ_HIP_CHECK(launch_x_pack(xd, (int64_t)K, (int64_t)K, n, nullptr, 0.f, p, s));
