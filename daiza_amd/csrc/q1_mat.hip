@@ -295,8 +295,9 @@ static int device_cus() {
 }
 
 // Splits of the wide product's K tiles: the workgroups go to the CUs in whole workgroups, and one tile of one
-// workgroup takes about kWideTileUs of a CU's matrix cores; a split adds a pass over its partials (written
-// and read back at about 4 TB/s) and a launch.
+// workgroup takes about kWideTileUs of a CU that holds two; a split adds a pass over its partials (written
+// and read back at about 4 TB/s) and a launch.  (A CU that holds one is slower than half of that: 5120 x 6144 at 1024
+// tokens takes 118 us where this counts 86.)
 constexpr double kWideTileUs = 3.6;
 static int wide_splits(const Q1Dev& W, int n, int* tps) {
   const int64_t wgs = ((W.nrb + kWideRb - 1) / kWideRb) * ((n + kWideTok - 1) / kWideTok);

@@ -124,8 +124,10 @@ __device__ __forceinline__ i32x8 read_frag(const unsigned char* f, unsigned lane
 // The digits of the next half tile travel to the other LDS buffer (lds_dma) while this one is
 // multiplied; its signs go into the registers that the expansion has just read.  Two workgroups share a CU
 // (2 x 72 KiB of LDS), so one's barrier and scale fmas hide behind the other's matrix instructions.
-// Bound by the matrix instructions: per group and wave 96 of them (about 20 cycles each) against
-// 18 KiB of LDS reads (48 B per cycle and CU) and ~130 VALU operations.
+// Per group and wave 96 matrix instructions (16 cycles each) against 18 KiB of LDS reads (48 B per cycle and
+// CU) and ~130 VALU operations.  Matrix cores busy at 1024 tokens (share of the launch, all SIMDs): 34816 x 5120 59%,
+// 5120 x 17408 53%, 16480 x 5120 49%, 5120 x 6144 35%: the first is mostly waiting within a CU, the others lose whole
+// rounds besides (1056 workgroups of 16480 rows over 512 places; 320 of 6144 columns, so most CUs hold one).
 // Grid: 1-D, row groups x token groups x splits (wide_tile); a split writes its partial to y + z·zstride.
 struct WideGrid {
   int nrg;  // row groups: ceil(nrb / kWideRb)
