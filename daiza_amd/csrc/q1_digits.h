@@ -16,9 +16,9 @@
 // exponent is within 5 of its block's largest; smaller values are rounded to a grid of 2^-29 of the
 // block's largest, beneath the rounding of an f32 dot product.  Errors of a 2048 x 5120 product against 64
 // bits (2-norm; n = 2, 8 and 128 columns) with three f16 parts and with digits:
-//   standard normal columns                            1.6e-7  1.6e-7  2.2e-7    0.8e-7  0.9e-7  0.8e-7
-//   normal · e^(3 normal)                              1.7e-7  2.0e-7  2.1e-7    0.8e-7  0.8e-7  0.9e-7
-//   two of about 2^14 that cancel in every group       2.2e-4  2.2e-4  2.6e-4    0.8e-7  2.5e-4  2.5e-4
+//   standard normal columns                            1.6e-7  1.6e-7  2.2e-7    0.8e-7  0.8e-7  0.8e-7
+//   normal · e^(3 normal)                              1.7e-7  2.0e-7  2.1e-7    0.8e-7  0.7e-7  0.8e-7
+//   two of about 2^14 that cancel in every group       2.2e-4  2.2e-4  2.6e-4    0.8e-7  1.2e-5  2.4e-4
 // A block that holds an infinity or a NaN gets the NaN scale (0xFF), so its token's results are NaN.
 //
 // Rate.  The instruction runs at four times the f16 rate (measured 9.1 ns per 16x16x128 per SIMD,
@@ -253,8 +253,12 @@ __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lan
     const u32x2 p0 = p[0], p1 = p[1], p2 = p[2];
     return i32x8{(int)p0.x, (int)p0.y, (int)p1.x, (int)p1.y, (int)p2.x, (int)p2.y, 0, 0};
   };
+  // T = 4 and 8: operand 0's sums (the largest digits) start from 0 too and join by an fma.  Added onto the others' in the
+  // accumulator, large values that cancel would round those away, to 2^-24 of the values before they cancel (the third
+  // line of the errors above: 2.5e-4 at eight columns).
+  constexpr bool kApart = T == 4 || T == 8;
   i32x8 a = read(0), b[SB];
-  f32x4 d[SB];
+  f32x4 d[SB], top[SB];
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
     const int g = i / FF::F, f = FF::F - 1 - i % FF::F;
@@ -267,11 +271,12 @@ __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lan
     const int sx = (int)(ex - drop * (unsigned)f);
 #pragma unroll
     for (int sb = 0; sb < SB; ++sb) {
-      const f32x4 c = f == FF::F - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
-      if (g == 0) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, kSignScale);
-      else if (g == 1) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, kSignScale);
-      else if (g == 2) d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, kSignScale);
-      else d[sb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, kSignScale);
+      const f32x4 c = f == FF::F - 1 || (kApart && f == 0) ? f32x4{0.f, 0.f, 0.f, 0.f} : d[sb];
+      f32x4& o = kApart && f == 0 ? top[sb] : d[sb];
+      if (g == 0) o = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 0, sx, 0, kSignScale);
+      else if (g == 1) o = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 1, sx, 0, kSignScale);
+      else if (g == 2) o = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 2, sx, 0, kSignScale);
+      else o = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[sb], c, 2, 4, 3, sx, 0, kSignScale);
     }
     a = an;
     if (f == 0) {
@@ -281,7 +286,10 @@ __device__ __forceinline__ void few_unit(const unsigned char* tile, unsigned lan
         const unsigned h = (unsigned)(__builtin_bit_cast(unsigned long long, u.sc[sb]) >> (16 * slot));
         const float sf = (float)__builtin_bit_cast(_Float16, (unsigned short)h);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[sb][v] = __builtin_fmaf(sf, d[sb][v], acc[sb][v]);
+        for (int v = 0; v < 4; ++v) {
+          acc[sb][v] = __builtin_fmaf(sf, d[sb][v], acc[sb][v]);
+          if constexpr (kApart) acc[sb][v] = __builtin_fmaf(sf, top[sb][v], acc[sb][v]);
+        }
       }
     }
   }
@@ -348,10 +356,10 @@ constexpr int few_max_tiles(int T) { return T == 16 ? 2 : 4; }
 //
 // PRE: the digits come packed by the kernel that formed the activations: at eight tokens the packing costs 2 to
 // 4 us of each product.
-// (Registers: about kFewWaves waves run, so a CU rarely holds two of these workgroups; the form of sixteen tokens that
-// packs its own tiles takes a few more than two would leave it.)
+// (Registers: about kFewWaves waves run, so a CU rarely holds two of these workgroups; the larger forms that pack their
+// own tiles take a few more than two would leave them.)
 template <int T, int NW, int RB, bool PRE>
-__global__ __launch_bounds__(64 * NW, NW < 8 ? 3 : T == 16 && RB == 8 && !PRE ? 2 : 4) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
+__global__ __launch_bounds__(64 * NW, NW < 8 ? 3 : T >= 4 && RB == 8 && !PRE ? 2 : 4) void q1_few_kernel(const uint8_t* __restrict__ W, int64_t rows, int64_t nrb,
                                                                      int ntiles, int tps, const FewX x, int n_tok,
                                                                      float* __restrict__ y, int64_t ldy, int64_t zstride,
                                                                      int accumulate) {

@@ -65,6 +65,26 @@ def test_small_values_beside_large_ones(dz, n):
     assert np.array_equal(m.matvec_batch(x), sign[None] * v[:, None])
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 8])
+def test_large_values_that_cancel(dz, n):
+    """Two values of 2^20 and more that cancel in every group of every row, among standard normal ones: up to eight
+    columns the sums of the largest digits round nothing else away, so the error is that of the digits' grid, at most
+    2^-29 (n <= 4: 2^-39) of the large value per column against results of columns of size 1, and f32 rounding."""
+    rows, cols = 512, 2048
+    rng = np.random.default_rng(n)
+    aos, _ = _matrix(rng, rows, cols)
+    blk = aos.reshape(rows, cols // 128, 18)
+    blk[:, :, 2 + 5] = (blk[:, :, 2 + 5] & 0xFE) | (1 - ((blk[:, :, 2] >> 3) & 1))  # column 40's sign: not column 3's
+    sign = np.unpackbits(blk[:, :, 2:], axis=-1, bitorder="little").astype(np.float64) * 2 - 1
+    w = (sign * np.ascontiguousarray(blk[:, :, :2]).view(np.float16).astype(np.float64)).reshape(rows, cols)
+    m = dz.Q1_0Matrix(np.ascontiguousarray(blk.reshape(-1)), rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[:, 3::128] = x[:, 40::128] = 2.0 ** 20 * (1 + rng.random((n, cols // 128)))
+    ref = x.astype(np.float64) @ w.T
+    err = np.linalg.norm(m.matvec_batch(x) - ref) / np.linalg.norm(ref)
+    assert err < 2.0 ** 21 * 2.0 ** (-39 if n <= 4 else -29) + 1e-6, err
+
+
 def test_non_finite_token(dz):
     rng = np.random.default_rng(9)
     aos, _ = _matrix(rng, 130, 1024)
