@@ -3,8 +3,9 @@ its tiles, against float64; and the forward that hands its activations over as d
 the oracle.
 
 Bound of the product: the sums of a group's digits and of the groups are f32 additions of partial sums, at most
-(8 + ngroups) per slot and 8 between the slots and splits, and the digits keep 2^-29 (n <= 4: 2^-39) of their 32-column block's
-largest value: |err| <= (ngroups + 24) 2^-24 Σ|w x| + 2^-29 Σ|w| max|x|.
+(8 + 2 ngroups) per slot (two fmas join a group's sums in the forms of four and eight tokens) and 8 between the
+slots and splits, and the digits keep 2^-29 (n <= 4: 2^-39) of their 32-column block's largest value:
+|err| <= (2 ngroups + 24) 2^-24 Σ|w x| + 2^-29 Σ|w| max|x|.
 """
 import numpy as np
 import pytest
@@ -37,7 +38,7 @@ def test_forms(dz, n, rows, cols):
     x[0, :32] = 0
     y0 = rng.standard_normal((n, rows)).astype(np.float32)
     ref = x.astype(np.float64) @ w.T
-    bound = ((cols // 128 + 24) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w).T)
+    bound = ((2 * (cols // 128) + 24) * 2.0 ** -24 * (np.abs(x.astype(np.float64)) @ np.abs(w).T)
              + 2.0 ** -29 * np.abs(x).max(1)[:, None] * np.abs(w).sum(1)[None])
     y = m.matvec_batch(x)
     assert np.all(np.abs(y - ref) <= bound)
